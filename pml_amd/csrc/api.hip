@@ -322,11 +322,11 @@ pmlg_status run_product_on(pmlg_ctx ctx, const Tables *T, W *Ah, W *Bh, W *Ch, v
             "ntt_fwd(B)");
     if (prof)
         prof_end(ctx, s, &pr);
-    // The 8-limb MFMA product leaves V 2^-64 mod p (Montgomery REDC) in [0, 4p);
+    // Products of 64-bit words come as V 2^-64 mod p (Montgomery REDC) in [0, 4p);
     // the inverse transform then scales by N^-1 2^64 instead of N^-1.
     ModConst mc = ctx->mc;
     NttTab<W> itab = tab;
-    if (kind == PW_MFMA && sizeof(W) == 8) {
+    if (sizeof(W) == 8) {
         const unsigned __int128 vmax = (unsigned __int128)k * (ctx->p - 1) * (ctx->p - 1);
         mc.redc_small = vmax < (((unsigned __int128)(3 * ctx->p - 1)) << 64) ? 1 : 0;
         itab.ninv = tab.ninvr;
@@ -385,16 +385,18 @@ pmlg_status check_ctx(pmlg_ctx ctx)
 pmlg_status pick_kind(pmlg_ctx ctx, int method, int64_t m, int64_t k, int64_t n,
                       PointwiseKind *kind)
 {
-    const bool mfma_ok = ctx->mc.limbs > 0 && mfma_supported((int)m, (int)k, (int)n, ctx->mc.limbs, ctx->p);
     if (method == PMLG_METHOD_PLAIN) {
         *kind = PW_PLAIN;
     } else if (method == PMLG_METHOD_MFMA) {
-        if (!mfma_ok)
+        if (!mfma_supported((int)m, (int)k, (int)n, ctx->mc.limbs, ctx->p))
             return fail(PMLG_ERR_UNSUPPORTED,
                         "MFMA pointwise kernel: shape or modulus outside its limits");
         *kind = PW_MFMA;
     } else if (method == PMLG_METHOD_AUTO) {
-        *kind = mfma_ok ? PW_MFMA : PW_PLAIN;
+        *kind = mfma_exact((int)m, (int)k, (int)n, ctx->mc.limbs, ctx->p) &&
+                        mfma_pays((int)m, (int)k, (int)n, ctx->mc.limbs)
+                    ? PW_MFMA
+                    : PW_PLAIN;
     } else {
         return fail(PMLG_ERR_ARG, "unknown method");
     }

@@ -4,14 +4,14 @@
 // A plan groups the products by what a launch can share:
 //   * forward transforms by (modulus, transform length, radix): one
 //     segment-table launch per group covers every entry of every operand;
-//   * pointwise products by (modulus, kernel, points per workgroup): one
+//   * pointwise products by (modulus, kernel, points per task): one
 //     persistent launch per group walks the task list of all its products;
 //   * inverse transforms by (modulus, length, radix, output scaling);
 //   * short products by direct (schoolbook) convolution, one persistent
 //     launch per modulus.
 // The launch sequence is captured into a hipGraph on the first run and
 // replayed afterwards.  Each product's configuration (algorithm, pointwise
-// kernel, radix of the register transforms, points per MFMA workgroup) comes
+// kernel, radix of the register transforms, points per MFMA task) comes
 // from the caller, the learned cost model, the autotuner's cache or the
 // threshold rule, in that order; the result is the same exact product
 // whichever runs.
@@ -137,14 +137,14 @@ unsigned grid_for(int64_t items, int64_t cap = 4096)
 // configurations
 // ---------------------------------------------------------------------------
 const ProdConfig kConfigs[kNumConfigs] = {
-    // school, kind,     fwd_e, inv_e, pb_shift
+    // school, kind,     fwd_e, inv_e, single_pt
     {1, PW_PLAIN, 5, 4, 0},  // 0: direct convolution
     {0, PW_PLAIN, 5, 4, 0},  // 1: transforms + plain pointwise
     {0, PW_MFMA, 5, 4, 0},   // 2: transforms + int8-limb MFMA pointwise
     {0, PW_PLAIN, 4, 4, 0},  // 3: plain, radix-16 forward passes
     {0, PW_MFMA, 4, 4, 0},   // 4: MFMA, radix-16 forward passes
     {0, PW_MFMA, 5, 5, 0},   // 5: MFMA, radix-32 inverse passes
-    {0, PW_MFMA, 5, 4, 1},   // 6: MFMA, half the points per workgroup
+    {0, PW_MFMA, 5, 4, 1},   // 6: MFMA, one point per task
     {0, PW_PLAIN, 5, 5, 0},  // 7: plain, radix-32 inverse passes
 };
 
@@ -163,7 +163,7 @@ bool config_valid(pmlg_ctx ctx, int64_t m, int64_t k, int64_t n, int64_t lenA, i
         ceil_log2(lenA + lenB - 1) > std::min(ctx->max_log, seg_max))
         return false;
     if (cf.kind == PW_MFMA)
-        return ctx->mc.limbs > 0 && mfma_supported((int)m, (int)k, (int)n, ctx->mc.limbs, ctx->p);
+        return mfma_supported((int)m, (int)k, (int)n, ctx->mc.limbs, ctx->p);
     return true;
 }
 
@@ -303,11 +303,10 @@ struct InvGroup {
 struct PwGroup {
     pmlg_ctx ctx;
     PointwiseKind kind;
-    int pb;
+    int pt;  // points per MFMA task
     size_t seg_off;
     int nseg;
     int64_t blocks;
-    size_t lds;
 };
 struct SchoolGroup {
     pmlg_ctx ctx;
@@ -407,9 +406,9 @@ pmlg_status launch_pw(pmlg_batch_plan plan, hipStream_t s)
             continue;
         // persistent grid: a few workgroups per CU, never more than the tasks
         const int grid = (int)std::min<int64_t>(g.blocks, g.kind == PW_MFMA ? 512 : 2048);
-        HIP_TRY(launch_pointwise_segs<W>(g.kind, g.pb,
+        HIP_TRY(launch_pointwise_segs<W>(g.kind, g.pt,
                                          reinterpret_cast<const PwSeg<W> *>(tb + g.seg_off),
-                                         g.nseg, g.blocks, g.lds, grid, g.ctx->mc, s),
+                                         g.nseg, g.blocks, grid, g.ctx->mc, s),
                 "batched pointwise products");
     }
     return PMLG_OK;
@@ -495,8 +494,7 @@ template <typename W>
 void add_segments(const pmlg_mul_desc &d, const ProdInfo &pi, unsigned char *arena,
                   std::map<std::tuple<pmlg_ctx, int, int, int>, std::vector<FwdSeg<uint64_t, W>>> &fwd,
                   std::map<std::tuple<pmlg_ctx, int, int, int>, std::vector<InvSeg<W, uint64_t>>> &inv,
-                  std::map<std::tuple<pmlg_ctx, int, int>, std::vector<PwSeg<W>>> &pw,
-                  std::map<std::tuple<pmlg_ctx, int, int>, size_t> &pw_lds)
+                  std::map<std::tuple<pmlg_ctx, int, int>, std::vector<PwSeg<W>>> &pw)
 {
     pmlg_ctx ctx = d.ctx;
     const ProdConfig &cf = kConfigs[pi.config];
@@ -513,14 +511,10 @@ void add_segments(const pmlg_mul_desc &d, const ProdInfo &pi, unsigned char *are
     auto &fv = fwd[{ctx, logN, cf.fwd_e, trunc}];
     fv.push_back(FwdSeg<uint64_t, W>{d.A, Ah, d.lenA, d.lenA, d.m * d.k, 0, trunc, 0});
     fv.push_back(FwdSeg<uint64_t, W>{d.B, Bh, d.lenB, d.lenB, d.k * d.n, 0, trunc, 0});
-    const bool redc = cf.kind == PW_MFMA && sizeof(W) == 8;
+    const bool redc = sizeof(W) == 8;
     inv[{ctx, logN, cf.inv_e, (redc ? 1 : 0) | (trunc << 1)}].push_back(
         InvSeg<W, uint64_t>{Ch, d.C, tmp, lenC, 0, lenC, d.m * d.n, 0, 0, trunc, 0});
-    int pb = 0;
-    if (cf.kind == PW_MFMA) {
-        pb = pw_pick_pb((int)d.m, (int)d.k, (int)d.n, ctx->mc.limbs, logP) >> cf.pb_shift;
-        pb = std::max(pb, 1);
-    }
+    const int pt = cf.kind == PW_MFMA ? pw_points(sizeof(W), logP, cf.single_pt != 0) : 0;
     PwSeg<W> ps{};
     ps.Ah = Ah;
     ps.Bh = Bh;
@@ -536,20 +530,14 @@ void add_segments(const pmlg_mul_desc &d, const ProdInfo &pi, unsigned char *are
         const unsigned __int128 vmax = (unsigned __int128)d.k * (ctx->p - 1) * (ctx->p - 1);
         ps.redc_small = vmax < (((unsigned __int128)(3 * ctx->p - 1)) << 64) ? 1 : 0;
     }
-    const auto key = std::make_tuple(ctx, (int)cf.kind, pb);
-    pw[key].push_back(ps);
-    if (cf.kind == PW_MFMA) {
-        size_t &l = pw_lds[key];
-        l = std::max(l, pw_mfma_lds(pb, (int)d.m, (int)d.k, (int)d.n, ctx->mc.limbs));
-    }
+    pw[std::make_tuple(ctx, (int)cf.kind, pt)].push_back(ps);
 }
 
 template <typename W>
 void finish_groups(pmlg_batch_plan plan, Blob &blob,
                    std::map<std::tuple<pmlg_ctx, int, int, int>, std::vector<FwdSeg<uint64_t, W>>> &fwd,
                    std::map<std::tuple<pmlg_ctx, int, int, int>, std::vector<InvSeg<W, uint64_t>>> &inv,
-                   std::map<std::tuple<pmlg_ctx, int, int>, std::vector<PwSeg<W>>> &pw,
-                   std::map<std::tuple<pmlg_ctx, int, int>, size_t> &pw_lds)
+                   std::map<std::tuple<pmlg_ctx, int, int>, std::vector<PwSeg<W>>> &pw)
 {
     for (auto &kv : fwd) {
         const int logN = std::get<1>(kv.first);
@@ -580,14 +568,13 @@ void finish_groups(pmlg_batch_plan plan, Blob &blob,
     }
     for (auto &kv : pw) {
         const PointwiseKind kind = (PointwiseKind)std::get<1>(kv.first);
-        const int pb = std::get<2>(kv.first);
+        const int pt = std::get<2>(kv.first);
         int64_t b = 0;
         for (auto &sg : kv.second) {
             sg.block0 = b;
-            b += pw_seg_blocks(kind, pb, sg.m, sg.n, sg.N);
+            b += pw_seg_blocks(kind, pt, sg.m, sg.n, sg.N);
         }
-        PwGroup g{std::get<0>(kv.first), kind, pb, blob.add(kv.second), (int)kv.second.size(), b,
-                  kind == PW_MFMA ? pw_lds[kv.first] : 0};
+        PwGroup g{std::get<0>(kv.first), kind, pt, blob.add(kv.second), (int)kv.second.size(), b};
         plan->pw.push_back(g);
     }
 }
@@ -736,18 +723,17 @@ pmlg_status build_plan(pmlg_batch_plan *out, const pmlg_mul_desc *descs, int64_t
     std::map<std::tuple<pmlg_ctx, int, int, int>, std::vector<InvSeg<uint32_t, uint64_t>>> i32;
     std::map<std::tuple<pmlg_ctx, int, int>, std::vector<PwSeg<uint64_t>>> p64;
     std::map<std::tuple<pmlg_ctx, int, int>, std::vector<PwSeg<uint32_t>>> p32;
-    std::map<std::tuple<pmlg_ctx, int, int>, size_t> l64, l32;
     for (int64_t i = 0; i < count; ++i) {
         const ProdInfo &pi = plan->prods[i];
         if (pi.config < 0 || kConfigs[pi.config].school)
             continue;
         if (descs[i].ctx->small)
-            add_segments<uint32_t>(descs[i], pi, arena, f32, i32, p32, l32);
+            add_segments<uint32_t>(descs[i], pi, arena, f32, i32, p32);
         else
-            add_segments<uint64_t>(descs[i], pi, arena, f64, i64, p64, l64);
+            add_segments<uint64_t>(descs[i], pi, arena, f64, i64, p64);
     }
-    finish_groups<uint64_t>(plan.get(), blob, f64, i64, p64, l64);
-    finish_groups<uint32_t>(plan.get(), blob, f32, i32, p32, l32);
+    finish_groups<uint64_t>(plan.get(), blob, f64, i64, p64);
+    finish_groups<uint32_t>(plan.get(), blob, f32, i32, p32);
     for (auto &kv : school) {
         int64_t b = 0;
         for (auto &sg : kv.second) {

@@ -179,11 +179,15 @@ hipError_t launch_pointwise(PointwiseKind kind, const W *Ah, const W *Bh, W *Ch,
                             int n, int64_t N, int logP, int logPc, const ModConst &mc,
                             hipStream_t s);
 
-// Whether the int8-limb MFMA kernel supports this shape.
+// Whether the int8-digit MFMA kernel is exact for this shape and modulus,
+// whether it is the faster of the two where it is, and whether an explicit
+// request for it (method or configuration) is accepted.
+bool mfma_exact(int m, int k, int n, int limbs, uint64_t p);
+bool mfma_pays(int m, int k, int n, int limbs);
 bool mfma_supported(int m, int k, int n, int limbs, uint64_t p);
 
 // One product of a batched pointwise launch (evaluations in blocked layout,
-// N points); tasks [block0, block0 + pw_seg_blocks(...)) are its own.
+// N points); blocks [block0, block0 + pw_seg_blocks(...)) are its own.
 template <typename W>
 struct PwSeg {
     const W *Ah, *Bh;
@@ -192,17 +196,14 @@ struct PwSeg {
     int64_t N, block0;
     int32_t redc_small, logPc;  // logPc: runs of C_hat
 };
-int64_t pw_seg_blocks(PointwiseKind kind, int pb, int m, int n, int64_t N);
-// LDS bytes of an MFMA task with pb points per workgroup
-size_t pw_mfma_lds(int pb, int m, int k, int n, int limbs);
-// largest points-per-workgroup (<= 2^logP) whose limb planes fit 64 KiB
-int pw_pick_pb(int m, int k, int n, int limbs, int logP);
-// Persistent launch over all tasks of nseg products sharing one prime:
-// `grid` workgroups (0: one per task) walk the task list; MFMA tasks use pb
-// points per workgroup and `lds` bytes (the maximum over the products).
+// points per task of the MFMA kernel: 16 bytes of a run, or one
+int pw_points(int elem_bytes, int logP, bool single);
+int64_t pw_seg_blocks(PointwiseKind kind, int pt, int m, int n, int64_t N);
+// Persistent launch over all blocks of nseg products sharing one prime:
+// `grid` workgroups (0: one per block) walk the block list; MFMA tasks take
+// pt points each.
 template <typename W>
-hipError_t launch_pointwise_segs(PointwiseKind kind, int pb, const PwSeg<W> *segs, int nseg,
-                                 int64_t blocks, size_t lds, int grid, const ModConst &mc,
-                                 hipStream_t s);
+hipError_t launch_pointwise_segs(PointwiseKind kind, int pt, const PwSeg<W> *segs, int nseg,
+                                 int64_t blocks, int grid, const ModConst &mc, hipStream_t s);
 
 }  // namespace pmlg
