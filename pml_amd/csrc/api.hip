@@ -310,16 +310,9 @@ pmlg_status run_product_on(pmlg_ctx ctx, const Tables *T, W *Ah, W *Bh, W *Ch, v
     pr.stage = -1;
     if (prof)
         prof_begin(ctx, 0, s, &pr);
-    HIP_TRY((launch_ntt_fwd<uint64_t, W>(dA, strideA, la, Ah, m * k, logN, logP, tune, tab, p, s,
-                                         tmpf, ct, trunc)),
-            "ntt_fwd(A)");
-    if (prof) {
-        prof_end(ctx, s, &pr);
-        prof_begin(ctx, 0, s, &pr);
-    }
-    HIP_TRY((launch_ntt_fwd<uint64_t, W>(dB, strideB, lb, Bh, k * n, logN, logP, tune, tab, p, s,
-                                         tmpf, ct, trunc)),
-            "ntt_fwd(B)");
+    const FwdOp<uint64_t, W> ops[2] = {{dA, strideA, la, Ah, m * k}, {dB, strideB, lb, Bh, k * n}};
+    HIP_TRY((launch_ntt_fwd<uint64_t, W>(ops, 2, logN, logP, tune, tab, p, s, tmpf, ct, trunc)),
+            "ntt_fwd");
     if (prof)
         prof_end(ctx, s, &pr);
     // Products of 64-bit words come as V 2^-64 mod p (Montgomery REDC) in [0, 4p);
@@ -435,7 +428,7 @@ pmlg_status mulmid_dev_strided(pmlg_ctx ctx, uint64_t *dOut, int64_t out_stride,
     const int64_t lc = la + lb - 1;
     // cyclic length: no wrapped term may land in [nlo, hi_eff)
     int64_t need = hi_eff > lc - nlo ? hi_eff : lc - nlo;
-    const int logN = ceil_log2(need);
+    const int logN = transform_log(need);
     if (logN > ctx->max_log) {
         // no 2^logN-th root of unity mod p (or p composite): multi-prime path
         if (hi_eff < nhi)
@@ -712,7 +705,7 @@ pmlg_status pmlg_polmat_mul_dev_noalloc(pmlg_ctx ctx, uint64_t *dC, const uint64
         HIP_TRY(fill_zero(dC, m * n * lenC, s), "fill_zero");
         return PMLG_OK;
     }
-    const int logN = ceil_log2(lenC);
+    const int logN = transform_log(lenC);
     if (logN > ctx->max_log)
         return fail(PMLG_ERR_UNSUPPORTED,
                     "pmlg_polmat_mul_dev_noalloc: transform length 2^" + std::to_string(logN) +

@@ -8,6 +8,22 @@
 
 namespace pmlg {
 
+// Uniform values read from a segment table, as scalars, and a pointer among
+// them as one to global memory.  Pointers loaded from memory are generic to
+// the compiler: every access through them would be a flat one, and what a
+// flat load returns counts as divergent.
+__device__ __forceinline__ int64_t uniform(int64_t x)
+{
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)x);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)((uint64_t)x >> 32));
+    return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+template <typename T>
+__device__ __forceinline__ T *as_global(T *p)
+{
+    return (T *)(__attribute__((address_space(1))) T *)(uint64_t)uniform(reinterpret_cast<int64_t>(p));
+}
+
 // Root-of-unity tables for one (p, log2 N): tw[t] = w^t, itw[t] = w^-t for
 // t < N, with their Shoup companions; w a primitive N-th root of unity.
 template <typename W>
@@ -101,15 +117,22 @@ inline bool trunc_ok(int logN, int64_t lenC)
            lenC <= 3 * (((int64_t)1 << logN) >> 2);
 }
 
-// Forward transforms of `count` entries: entry e reads in[e*in_stride + i]
-// for i < in_len (zero beyond), writes its N evaluations in blocked layout
-// (the first 3N/4 when trunc).  Transforms longer than 4 times the LDS limit
-// run a column pass first into tmp (count*N words of Win) with the tables ct.
+// Forward transforms of one or two operands in one launch: `count` entries
+// each, entry e reads in[e*in_stride + i] for i < in_len (zero beyond), writes
+// its N evaluations in blocked layout (the first 3N/4 when trunc).  logN >= 1.
+// Transforms longer than 4 times the LDS limit run a column pass first into
+// tmp (the larger count times N words of Win) with the tables ct.
 template <typename Win, typename W>
-hipError_t launch_ntt_fwd(const Win *in, int64_t in_stride, int64_t in_len, W *out,
-                          int64_t count, int logN, int logP, const NttTune &tune,
-                          const NttTab<W> &tab, W p, hipStream_t s, Win *tmp = nullptr,
-                          const ColTab<W> *ct = nullptr, bool trunc = false);
+struct FwdOp {
+    const Win *in;
+    int64_t in_stride, in_len;
+    W *out;
+    int64_t count;
+};
+template <typename Win, typename W>
+hipError_t launch_ntt_fwd(const FwdOp<Win, W> *ops, int nops, int logN, int logP,
+                          const NttTune &tune, const NttTab<W> &tab, W p, hipStream_t s,
+                          Win *tmp = nullptr, const ColTab<W> *ct = nullptr, bool trunc = false);
 
 // Inverse transforms (blocked input): coefficients [lo, hi) of each entry
 // (clipped to N), scaled by 1/N, written to out[e*out_stride + (i - lo)] as
@@ -127,7 +150,8 @@ hipError_t launch_ntt_inv(const W *in, Wout *out, int64_t out_stride, int64_t lo
 // Segment tables of the batched launches.  One launch serves many operand
 // matrices (segments) that share a prime and a transform length; segment s
 // owns the workgroups [block0, block0 + blocks) of the launch, found by a
-// binary search on block0 (segments sorted by block0, no gaps).
+// binary search on block0 (segments sorted by block0, no gaps).  The direct
+// launches pass their one or two segments by value.
 // ---------------------------------------------------------------------------
 
 // Forward: `count` entries, entry e at in + e*in_stride (first in_len words

@@ -1,15 +1,17 @@
 // Batched number-theoretic transforms over Z/pZ at 2^k-th roots of unity.
 //
 // Forward: decimation in frequency (natural order in, bit-reversed order out
-// inside each LDS sub-transform).  Inverse: decimation in time, exact inverse
-// of the forward up to the factor N.  Pointwise products work position by
+// inside each sub-transform).  Inverse: decimation in time, exact inverse of
+// the forward up to the factor N.  Pointwise products work position by
 // position, so the evaluation order never has to be undone.
 //
-// One workgroup holds `nb` sub-transforms of size M = 2^logM in LDS and runs
-// every radix-2 stage there.  When N = R*M exceeds the LDS limit, the first
-// radix-R stage is applied while loading (y_g[i] = w^(i g) sum_t x[i+Mt] w_R^(tg),
+// A sub-transform of size M = 2^logM lives in the registers of M / 2^LOGE
+// threads (below).  When N = R*M exceeds the largest M, the first radix-R
+// stage is applied while loading (y_g[i] = w^(i g) sum_t x[i+Mt] w_R^(tg),
 // whose size-M transform is X[R k + g]); the inverse runs the R size-M inverse
 // transforms and a merge pass x[o] = N^-1 sum_g w^(-o g) z_g[o mod M].
+#include <type_traits>
+
 #include "internal.hpp"
 
 namespace pmlg {
@@ -17,15 +19,15 @@ namespace pmlg {
 namespace {
 
 constexpr int kThreads = 256;
-#ifndef PMLG_INV_WAVES
-#define PMLG_INV_WAVES 4
-#endif
-constexpr int kInvWaves = PMLG_INV_WAVES;  // minimum waves per SIMD of the inverse register kernels
-// minimum waves per SIMD of the radix-32 forward register kernels: their
-// 256-thread workgroups alone ask for one, which lets the register allocator
-// drift past 256 registers (one wave per SIMD, 1.6x slower) on small changes
-// of the surrounding code; two keep them at or below 256.
-constexpr int kFwdWaves32 = 2;
+// transforms split into sub-transforms (logR > 0) have sub-transforms of at
+// least this size, one per workgroup
+constexpr int kRegMinLog = 11;
+// Waves per SIMD of the register kernels, by log2 of the elements a thread
+// holds: eight 64-bit words leave room for four, sixteen for four within 128
+// registers, thirty-two for two.  Without the bound the register allocator
+// drifts past the next limit on small changes of the surrounding code.
+template <int LOGE>
+constexpr int kXformWaves = LOGE == 5 ? 2 : 4;
 
 // Point-blocked evaluation layout: position `pos` of entry `e` (of `count`
 // entries) lives at ((pos >> logP) * count + e) * P + (pos mod P), P = 2^logP,
@@ -101,189 +103,6 @@ __device__ __forceinline__ void trunc_correct(W &c0, W &c1, W &c2, W c3, const N
     c2 = c2 >= p ? c2 - p : c2;
 }
 
-// Units u0 .. u0+nb-1 (of `units` = count << logR) of one operand: the
-// workgroup body shared by the direct and the segment-table launches.
-template <typename Win, typename W>
-__device__ __forceinline__ void fwd_lds_body(const Win *__restrict__ in, int64_t in_stride,
-                                             int64_t in_len, W *__restrict__ out, int64_t units,
-                                             int64_t u0, int logN, int logR, int lognb, int logP,
-                                             const NttTab<W> &tab, W p, bool trunc = false)
-{
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-    W *s = reinterpret_cast<W *>(smem_raw);
-    const int logM = logN - logR;
-    const int M = 1 << logM;
-    const int R = 1 << logR;
-    const int nb = 1 << lognb;
-    const int64_t N = (int64_t)1 << logN;
-    const W p2 = p + p;
-
-    // load (with the radix-R split when R > 1)
-    for (int idx = threadIdx.x; idx < nb * M; idx += kThreads) {
-        const int t = idx >> logM;
-        const int i1 = idx & (M - 1);
-        const int64_t u = u0 + t;
-        W v = 0;
-        if (u < units) {
-            const int64_t e = u >> logR;
-            const int g = (int)(u & (R - 1));
-            const Win *x = in + e * in_stride;
-            if (R == 1) {
-                v = (i1 < in_len) ? (W)x[i1] : (W)0;
-            } else {
-                W acc = 0;
-                for (int t2 = 0; t2 < R; ++t2) {
-                    const int64_t src = (int64_t)i1 + (int64_t)M * t2;
-                    if (src < in_len) {
-                        const int64_t widx = ((int64_t)M * g * t2) & (N - 1);
-                        W xv = (W)x[src];
-                        acc = add_2p<W>(acc, tw_mul<W>(xv, tab.tw, tab.twq, widx, p), p2);
-                    }
-                }
-                v = tw_mul<W>(acc, tab.tw, tab.twq, (int64_t)i1 * g, p);
-            }
-        }
-        s[idx] = v;
-    }
-    __syncthreads();
-
-    // DIF radix-2 stages; sub-transform root is w^R, twiddle w_M^(j M/2h) = w^(j << (logN-lh-1))
-    const int halfM = M >> 1;
-    for (int lh = logM - 1; lh >= 0; --lh) {
-        const int h = 1 << lh;
-        const int sh = logN - lh - 1;
-        for (int b = threadIdx.x; b < nb * halfM; b += kThreads) {
-            const int t = b >> (logM - 1);
-            const int bb = b & (halfM - 1);
-            const int j = bb & (h - 1);
-            const int i = t * M + ((bb >> lh) << (lh + 1)) + j;
-            const W a = s[i], c = s[i + h];
-            s[i] = add_2p<W>(a, c, p2);
-            s[i + h] = tw_mul<W>(sub_2p<W>(a, c, p2), tab.tw, tab.twq, (int64_t)j << sh, p);
-        }
-        __syncthreads();
-    }
-
-    // store: unit u = (e, g) -> out[e*N + g*M + i]; a 3/4-truncated transform
-    // (R = 1) keeps the positions below 3M/4
-    for (int idx = threadIdx.x; idx < nb * M; idx += kThreads) {
-        const int t = idx >> logM;
-        const int i1 = idx & (M - 1);
-        const int64_t u = u0 + t;
-        if (u < units && !(trunc && R == 1 && i1 >= 3 * (M >> 2))) {
-            const int64_t e = u >> logR;
-            const int g = (int)(u & (R - 1));
-            out[blk_addr(e, (int64_t)g * M + i1, units >> logR, logP)] = reduce_2p<W>(s[idx], p);
-        }
-    }
-}
-
-template <typename Win, typename W>
-__global__ void __launch_bounds__(kThreads)
-ntt_fwd_kernel(const Win *__restrict__ in, int64_t in_stride, int64_t in_len,
-               W *__restrict__ out, int64_t units, int logN, int logR, int lognb, int logP,
-               NttTab<W> tab, W p, int trunc)
-{
-    fwd_lds_body<Win, W>(in, in_stride, in_len, out, units, (int64_t)blockIdx.x << lognb, logN,
-                         logR, lognb, logP, tab, p, trunc != 0);
-}
-
-template <typename W, typename Wout>
-__device__ __forceinline__ void inv_lds_body(const W *__restrict__ in, Wout *__restrict__ out,
-                                             int64_t out_stride, int64_t lo, int64_t hi,
-                                             W *__restrict__ tmp, int64_t units, int64_t u0,
-                                             int logN, int logR, int lognb, int logP,
-                                             const NttTab<W> &tab, W p, bool trunc = false)
-{
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-    W *s = reinterpret_cast<W *>(smem_raw);
-    const int logM = logN - logR;
-    const int M = 1 << logM;
-    const int R = 1 << logR;
-    const int nb = 1 << lognb;
-    const int64_t N = (int64_t)1 << logN;
-    const W p2 = p + p;
-
-    for (int idx = threadIdx.x; idx < nb * M; idx += kThreads) {
-        const int t = idx >> logM;
-        const int i1 = idx & (M - 1);
-        const int64_t u = u0 + t;
-        W v = 0;
-        if (u < units) {
-            const int64_t e = u >> logR;
-            const int g = (int)(u & (R - 1));
-            if (!(trunc && i1 >= 3 * (M >> 2))) {  // a truncated product's dropped quarter
-                v = in[blk_addr(e, (int64_t)g * M + i1, units >> logR, logP)];
-                v = v >= p2 ? v - p2 : v;  // products may arrive in [0, 4p)
-            }
-        }
-        s[idx] = v;
-    }
-    __syncthreads();
-
-    // DIT radix-2 stages with inverse twiddles, h = 1 .. M/2
-    const int halfM = M >> 1;
-    for (int lh = 0; lh < logM; ++lh) {
-        const int h = 1 << lh;
-        const int sh = logN - lh - 1;
-        for (int b = threadIdx.x; b < nb * halfM; b += kThreads) {
-            const int t = b >> (logM - 1);
-            const int bb = b & (halfM - 1);
-            const int j = bb & (h - 1);
-            const int i = t * M + ((bb >> lh) << (lh + 1)) + j;
-            const W a = s[i];
-            const W c = tw_mul<W>(s[i + h], tab.itw, tab.itwq, (int64_t)j << sh, p);
-            s[i] = add_2p<W>(a, c, p2);
-            W d = a + p2 - c;  // (0, 4p)
-            s[i + h] = d >= p2 ? d - p2 : d;
-        }
-        __syncthreads();
-    }
-
-    if (trunc && R == 1) {
-        // scaled outputs, corrected by the dropped quarter (trunc_correct)
-        const int M4 = M >> 2;
-        for (int b = threadIdx.x; b < nb * M4; b += kThreads) {
-            const int t = b >> (logM - 2);
-            const int i = b & (M4 - 1);
-            W *q = s + t * M + i;
-            W c0 = shoup<W>(q[0], tab.ninv, tab.ninvq, p), c1 = shoup<W>(q[M4], tab.ninv, tab.ninvq, p);
-            W c2 = shoup<W>(q[2 * M4], tab.ninv, tab.ninvq, p);
-            trunc_correct<W>(c0, c1, c2, shoup<W>(q[3 * M4], tab.ninv, tab.ninvq, p), tab, p);
-            q[0] = c0;
-            q[M4] = c1;
-            q[2 * M4] = c2;
-        }
-        __syncthreads();
-    }
-    for (int idx = threadIdx.x; idx < nb * M; idx += kThreads) {
-        const int t = idx >> logM;
-        const int i1 = idx & (M - 1);
-        const int64_t u = u0 + t;
-        if (u >= units)
-            continue;
-        const int64_t e = u >> logR;
-        if (R == 1) {
-            if (i1 >= lo && i1 < hi)
-                out[e * out_stride + (i1 - lo)] =
-                    (Wout)(trunc && R == 1 ? s[idx] : shoup<W>(s[idx], tab.ninv, tab.ninvq, p));
-        } else {
-            const int g = (int)(u & (R - 1));
-            tmp[e * N + (int64_t)g * M + i1] = s[idx];
-        }
-    }
-}
-
-template <typename W, typename Wout>
-__global__ void __launch_bounds__(kThreads)
-ntt_inv_kernel(const W *__restrict__ in, Wout *__restrict__ out, int64_t out_stride, int64_t lo,
-               int64_t hi, W *__restrict__ tmp, int64_t units, int logN, int logR, int lognb,
-               int logP, NttTab<W> tab, W p, int trunc)
-{
-    inv_lds_body<W, Wout>(in, out, out_stride, lo, hi, tmp, units, (int64_t)blockIdx.x << lognb,
-                          logN, logR, lognb, logP, tab, p, trunc != 0);
-}
-
 // x[o] = N^-1 * sum_g w^(-(o g) mod N) z_g[o mod M], o in [lo, hi)
 template <typename W, typename Wout>
 __device__ __forceinline__ void merge_one(const W *__restrict__ z, Wout *__restrict__ out,
@@ -356,24 +175,85 @@ ntt_merge_kernel(const W *__restrict__ z, Wout *__restrict__ out, int64_t out_st
         merge_one<W, Wout>(z, out, out_stride, lo, width, idx, logN, logR, tab, p);
 }
 
-inline int pick_lognb(int logM)
+// ===========================================================================
+// Register-resident transforms for 2 <= M <= 2^14.
+//
+// Each of the T = M / E threads of a transform keeps E = 2^LOGE elements in
+// registers.  The L = log2 M radix-2 stages are grouped into passes of LOGE
+// stages (the last one possibly shorter); a pass starting at stage S0 with R
+// stages acts on the index bits [BLO, BLO+R), BLO = L-S0-R, and every thread
+// owns whole groups of 2^R elements that differ only in those bits.  Between
+// passes the elements go through LDS, laid out with one padding word every 32
+// to spread the banks.  Stage s pairs bit b = L-1-s; the twiddle of a pair
+// whose lower index is i is w_M^((i mod 2^b) 2^s), read from the per-stage
+// table at x = i mod 2^b.
+//
+// Transforms below 2^11 points share a workgroup of 256 threads, 256 / T of
+// them; up to 64 threads a transform lies within one wave, and its exchanges
+// need no workgroup barrier.  (A radix-2 stage per LDS round trip and barrier,
+// as these sizes had before, took 446 us for both operands of 128 x 128
+// matrices of length 512 at 1024 points, 60-bit prime; these kernels take
+// 196, and 28.8 -> 8.9 us for 16 x 16 matrices of length 256.)
+// ===========================================================================
+// Buffer descriptor of `bytes` bytes at the uniform address p: loads past its
+// end give 0 and stores past it are dropped, so a row of elements cut by a
+// length needs no branch per element (branches around the loads keep the
+// register allocator from overlapping them; per-element selects cost three
+// instructions each).
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void *p, int64_t bytes)
 {
-    const int want = 11;  // at least 2048 elements per workgroup
-    return logM >= want ? 0 : want - logM;
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, (int)bytes, 0x00027000);
+}
+constexpr uint32_t kOutside = 0xfffffff8u;  // an offset past every buffer
+typedef uint32_t v2u __attribute__((ext_vector_type(2)));
+
+// word at byte offset `off` of a buffer of 64-bit words; a 32-bit word reads
+// the low half
+template <typename W>
+__device__ __forceinline__ W buffer_word(__amdgpu_buffer_rsrc_t r, uint32_t off)
+{
+    if constexpr (sizeof(W) == 8) {
+        const v2u v = __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, 0, 0);
+        return ((uint64_t)v.y << 32) | v.x;
+    } else {
+        return __builtin_amdgcn_raw_buffer_load_b32(r, (int)off, 0, 0);
+    }
+}
+__device__ __forceinline__ void buffer_store(__amdgpu_buffer_rsrc_t r, uint32_t off, uint64_t x)
+{
+    const v2u v = {(uint32_t)x, (uint32_t)(x >> 32)};
+    __builtin_amdgcn_raw_buffer_store_b64(v, r, (int)off, 0, 0);
 }
 
-// ===========================================================================
-// Register-resident transforms for 2^11 <= M <= 2^14.
-//
-// Each of the T = M / E threads keeps E = 2^LOGE elements in registers.  The
-// L = log2 M radix-2 stages are grouped into passes of LOGE stages (the last
-// one possibly shorter); a pass starting at stage S0 with R stages acts on the
-// index bits [BLO, BLO+R), BLO = L-S0-R, and every thread owns whole groups of
-// 2^R elements that differ only in those bits.  Between passes the elements go
-// through LDS, laid out with one padding word every 32 to spread the banks.
-// Stage s pairs bit b = L-1-s; the twiddle of a pair whose lower index is i is
-// w_M^((i mod 2^b) 2^s), read from the per-stage table at x = i mod 2^b.
-// ===========================================================================
+// log2 of the elements per thread below 2^11 points: more threads than the
+// longer transforms use, since these calls have few transforms or short ones
+constexpr int small_log_e(int L)
+{
+    return L <= 3 ? L : (L == 7 || L == 8 || L == 10) ? 4 : 3;
+}
+
+// transforms per workgroup and its threads
+template <int L, int LOGE>
+constexpr int kXforms = L >= 11 ? 1 : 256 >> (L - LOGE);
+template <int L, int LOGE>
+constexpr int kXformThreads = kXforms<L, LOGE> << (L - LOGE);
+// words of LDS of one transform
+template <int L>
+constexpr int kXformLds = (1 << L) + (1 << L) / 32;
+
+// order the LDS accesses of a transform's threads between two phases
+template <int L, int LOGE>
+__device__ __forceinline__ void xform_sync()
+{
+    if constexpr (L - LOGE > 6) {
+        __syncthreads();
+    } else {
+        // within one wave: its LDS operations take effect in program order
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+}
 
 __device__ __forceinline__ int swz(int a)
 {
@@ -793,9 +673,9 @@ __device__ __forceinline__ void fwd_passes(W (&x)[1 << LOGE], W (&tw)[2 * ((1 <<
     if constexpr (S0 + PS::R < L) {
         load_pass_tw<W, L, LOGE, S0 + PS::R>(tw, t, stw);  // in flight during the exchange
         lds_store<W, L, LOGE, S0>(x, lds, t);
-        __syncthreads();
+        xform_sync<L, LOGE>();
         lds_load<W, L, LOGE, S0 + PS::R>(x, lds, t);
-        __syncthreads();
+        xform_sync<L, LOGE>();
         constexpr int B1 = LOOSE ? fwd_pass_out(PS::R, B0, false) : 2;
         fwd_passes<W, LOOSE, L, LOGE, S0 + PS::R, B1>(x, tw, lds, t, stw, k, false, trunc);
     }
@@ -904,77 +784,137 @@ __device__ __forceinline__ void inv_passes(W (&x)[1 << LOGE], W (&tw)[2 * ((1 <<
         inv_stages<W, LOOSE, L, LOGE, S0, B0, 0>(x, tw, k);
     if constexpr (S0 > 0) {
         load_pass_tw<W, L, LOGE, S0 - LOGE>(tw, t, tab.sitw);
-        __syncthreads();  // every thread has finished reading the previous arrangement
+        xform_sync<L, LOGE>();  // every thread has finished reading the previous arrangement
         lds_store<W, L, LOGE, S0>(x, lds, t);
-        __syncthreads();
+        xform_sync<L, LOGE>();
         lds_load<W, L, LOGE, S0 - LOGE>(x, lds, t);
         constexpr int B1 = LOOSE ? inv_pass_out(PS::R, B0, PS::BLO == 0) : 2;
         inv_passes<W, LOOSE, L, LOGE, S0 - LOGE, B1>(x, tw, lds, t, tab, k, trunc);
     }
 }
 
-// pre: the input rows are the column pass's outputs (row g of entry e at
-// in + e*in_stride + g*M, every word valid): no radix-R step on the load.
-template <typename Win, typename W, bool LOOSE, int L, int LOGE>
+// Transform number u0 + sub of a segment (sub-transform gg = u mod R of entry
+// u / R) by the thread with index t of its transform; lds: the transform's own
+// words; u0 is uniform.  Threads of a transform past the last one (live false)
+// run along and store nothing.
+// MODE: one transform per entry (kWhole), the radix-R step on the load (kSplit:
+// R = 2 or 4 sub-transforms per entry) or the column pass's outputs (kRows: row
+// g of entry e at in + e*in_stride + g*M, every word valid).
+enum FwdMode { kWhole, kSplit, kRows };
+template <typename Win, typename W, bool LOOSE, int L, int LOGE, int MODE>
 __device__ __forceinline__ void fwd_reg_body(const Win *__restrict__ in, int64_t in_stride,
-                                             int64_t in_len, W *__restrict__ out, int64_t units,
-                                             int64_t u, int logR, int logP, const NttTab<W> &tab,
-                                             W p, bool pre = false, bool trunc = false)
+                                             int64_t in_len, W *__restrict__ out, int64_t count,
+                                             int64_t u0, int sub, bool live, W *lds, int t, int logR,
+                                             int logP, const NttTab<W> &tab, W p, bool trunc)
 {
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-    W *lds = reinterpret_cast<W *>(smem_raw);
+    static_assert(sizeof(Win) == 8, "inputs are 64-bit words");
     constexpr int E = 1 << LOGE, M = 1 << L;
-    const int t = threadIdx.x;
-    const int64_t e = u >> logR;
+    if constexpr (MODE == kWhole)
+        logR = 0;
     const int R = 1 << logR;
-    const int gg = (int)(u & (R - 1));
-    const int logN = L + logR;
-    const int64_t N = (int64_t)1 << logN;
-    const W p2 = p + p;
-    const Win *xin = in + e * in_stride;
+    const int64_t e0 = u0 >> logR;  // uniform
+    const int64_t e = live ? e0 + sub : e0;
+    const int gg = (int)(u0 & (R - 1));
+    const Win *xin = in + e0 * in_stride;
     // truncated: with a radix-4 split the fourth sub-transform (frequencies
     // 3 mod 4) is dropped (the whole workgroup returns), without a split the
     // last quarter of the positions
-    if (trunc && R == 4 && gg == 3)
+    if (MODE == kSplit && trunc && gg == 3)
         return;
-    const bool tq = trunc && R == 1;
+    const bool tq = MODE == kWhole && trunc;
 
     W tw[2 * (E - 1)];
-    load_pass_tw<W, L, LOGE, 0>(tw, t, tab.stw);
     W x[E];
     // pass-0 arrangement: element j of thread t is index (j << (L-LOGE)) | t
+    if constexpr (MODE == kRows) {
+        load_pass_tw<W, L, LOGE, 0>(tw, t, tab.stw);
 #pragma unroll
-    for (int j = 0; j < E; ++j) {
-        const int i1 = (j << (L - LOGE)) | t;
-        W v = 0;
-        if (pre) {
-            v = (W)xin[(int64_t)gg * M + i1];
-        } else if (R == 1) {
-            if (i1 < in_len)
-                v = (W)xin[i1];
+        for (int j = 0; j < E; ++j)
+            x[j] = (W)xin[(int64_t)gg * M + ((j << (L - LOGE)) | t)];
+    } else if constexpr (MODE == kWhole) {
+        const int len = in_len < M ? (int)in_len : M;
+        if constexpr (kXforms<L, LOGE> == 1) {
+            const __amdgpu_buffer_rsrc_t r = buffer_of(xin, (int64_t)len * 8);
+#pragma unroll
+            for (int j = 0; j < E; ++j)
+                x[j] = buffer_word<W>(r, (uint32_t)((j << (L - LOGE)) | t) * 8);
         } else {
-            W acc = 0;
-            for (int t2 = 0; t2 < R; ++t2) {
-                const int64_t src = (int64_t)i1 + (int64_t)M * t2;
-                if (src < in_len) {
-                    const int64_t widx = ((int64_t)M * gg * t2) & (N - 1);
-                    acc = add_2p<W>(acc, shoup_lazy((W)xin[src], tab.tw[widx], tab.twq[widx], p), p2);
+            // the workgroup's entries in one buffer (256 entries of stride
+            // below 2^20 words; longer strides take plain loads)
+            if (in_stride < ((int64_t)1 << 20)) {
+                const __amdgpu_buffer_rsrc_t r =
+                    buffer_of(xin, (int64_t)kXforms<L, LOGE> * in_stride * 8);
+                const uint32_t base = (uint32_t)(e - e0) * (uint32_t)in_stride * 8;
+#pragma unroll
+                for (int j = 0; j < E; ++j) {
+                    const int i1 = (j << (L - LOGE)) | t;
+                    x[j] = buffer_word<W>(r, i1 < len ? base + (uint32_t)i1 * 8 : kOutside);
+                }
+            } else {
+                const Win *xe = xin + (e - e0) * in_stride;
+#pragma unroll
+                for (int j = 0; j < E; ++j) {
+                    const int i1 = (j << (L - LOGE)) | t;
+                    const W v = (W)xe[i1 < len ? i1 : 0];
+                    x[j] = i1 < len ? v : (W)0;
                 }
             }
-            const int64_t widx = (int64_t)i1 * gg;
-            v = shoup_lazy(acc, tab.tw[widx], tab.twq[widx], p);
         }
-        x[j] = v;
+        // the inputs' offsets are dead before the twiddles' registers fill
+        __builtin_amdgcn_sched_barrier(0);
+        load_pass_tw<W, L, LOGE, 0>(tw, t, tab.stw);
+    } else {
+        const int64_t N = (int64_t)M << logR;
+        const W p2 = p + p;
+        const int64_t len = in_len < N ? in_len : N;
+        const __amdgpu_buffer_rsrc_t r = buffer_of(xin, len * 8);
+        const int nt = (int)((len + M - 1) >> L);  // rows of M words with an input
+#pragma unroll
+        for (int j = 0; j < E; ++j)
+            x[j] = buffer_word<W>(r, (uint32_t)((j << (L - LOGE)) | t) * 8);
+        for (int t2 = 1; t2 < nt; ++t2) {
+            const int64_t widx = ((int64_t)M * gg * t2) & (N - 1);  // uniform
+            const W w = tab.tw[widx], wq = tab.twq[widx];
+            constexpr int G = E < 8 ? E : 8;  // loads in flight together
+#pragma unroll
+            for (int j0 = 0; j0 < E; j0 += G) {
+                W v[G];
+#pragma unroll
+                for (int j = 0; j < G; ++j)
+                    v[j] = buffer_word<W>(r, (uint32_t)((((j0 + j) << (L - LOGE)) | t) + (t2 << L)) * 8);
+#pragma unroll
+                for (int j = 0; j < G; ++j)
+                    x[j0 + j] = add_2p<W>(x[j0 + j], shoup_lazy(v[j], w, wq, p), p2);
+            }
+        }
+        if (gg > 0) {
+            constexpr int G = E < 8 ? E : 8;
+#pragma unroll
+            for (int j0 = 0; j0 < E; j0 += G) {
+                W w[G], wq[G];
+#pragma unroll
+                for (int j = 0; j < G; ++j) {
+                    const uint32_t widx = (uint32_t)(((j0 + j) << (L - LOGE)) | t) * (uint32_t)gg;
+                    w[j] = tab.tw[widx];
+                    wq[j] = tab.twq[widx];
+                }
+#pragma unroll
+                for (int j = 0; j < G; ++j)
+                    x[j0 + j] = shoup_lazy(x[j0 + j], w[j], wq[j], p);
+            }
+        }
+        load_pass_tw<W, L, LOGE, 0>(tw, t, tab.stw);
     }
     const Bfly<W> k(p);
     // inputs below 2p (coefficients, the column-in-load sums, or the column
     // pass's reduced rows); a direct load of at most M/2 coefficients leaves
     // the upper half zero
     fwd_passes<W, LOOSE, L, LOGE, 0, 2>(x, tw, lds, t, tab.stw, k,
-                                        !pre && R == 1 && in_len <= (M >> 1), tq);
+                                        MODE == kWhole && in_len <= (M >> 1), tq);
     // the last pass leaves each thread runs of 2^R consecutive positions:
     // store them from registers (no LDS round trip)
-    const int64_t count = units >> logR;
+    if (!live)
+        return;
     using PSL = PassShape<L, LOGE, last_pass_start<L, LOGE>()>;
     constexpr int RUN = 1 << PSL::R;
     // words per vector store: within one layout block of 2^logP positions
@@ -984,7 +924,7 @@ __device__ __forceinline__ void fwd_reg_body(const Win *__restrict__ in, int64_t
     for (int g = 0; g < PSL::G; ++g) {
         // a truncated transform keeps the positions below 3M/4 (a run lies
         // within one quarter)
-        if (tq && PSL::index(t, g, 0) >= (3 << (L - 2)))
+        if (tq && PSL::index(t, g, 0) >= 3 * (M / 4))
             continue;
         W y[RUN];
         fwd_final<W, LOOSE, LOGE, PSL::R, fwd_last_b0<L, LOGE>(2), 0>(x, g * RUN, y, k);
@@ -1002,36 +942,75 @@ __device__ __forceinline__ void fwd_reg_body(const Win *__restrict__ in, int64_t
     }
 }
 
+// Segment of block b: segments are sorted by their first block, without gaps
+template <typename S>
+__device__ __forceinline__ const S &seg_of(const S *segs, int nseg, int64_t b)
+{
+    int lo = 0, hi = nseg - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (segs[mid].block0 <= b)
+            lo = mid;
+        else
+            hi = mid - 1;
+    }
+    return segs[lo];
+}
+
+// The operands of a launch: a table in device memory (batched products), or
+// one or two of them by value (both operands of a product in one launch: two
+// launches of 1024 transforms of 8192 points each fill the chip twice over
+// and drain it twice).
+template <typename S>
+struct SegList {
+    const S *tab;
+    int n;
+    S s[2];
+    __device__ __forceinline__ S of(int64_t b) const
+    {
+        if (tab)
+            return seg_of(as_global(tab), n, b);
+        return n > 1 && b >= s[1].block0 ? s[1] : s[0];
+    }
+};
+
 // TRUNC (3/4-truncated transforms) is a template parameter: its branches,
 // even when not taken, take the radix-32 kernels past 256 registers (one
-// wave per SIMD instead of two).
-template <typename Win, typename W, bool LOOSE, int L, int LOGE, bool TRUNC>
-__global__ void __launch_bounds__(1 << (L - LOGE)) __attribute__((amdgpu_waves_per_eu(LOGE == 5 ? kFwdWaves32 : 1)))
-ntt_fwd_reg(const Win *__restrict__ in, int64_t in_stride, int64_t in_len, W *__restrict__ out,
-            int64_t units, int logR, int logP, NttTab<W> tab, W p, int pre)
+// wave per SIMD instead of two).  Every segment of one launch has the
+// launch's TRUNC.
+template <typename Win, typename W, bool LOOSE, int L, int LOGE, int MODE, bool TRUNC>
+__global__ void __launch_bounds__((kXformThreads<L, LOGE>)) __attribute__((amdgpu_waves_per_eu(kXformWaves<LOGE>)))
+ntt_fwd_reg(SegList<FwdSeg<Win, W>> segs, int logR, int logP, NttTab<W> tab, W p)
 {
-    // pre: the column pass's rows as input
-    fwd_reg_body<Win, W, LOOSE, L, LOGE>(in, in_stride, in_len, out, units,
-                                         xcd_unit(blockIdx.x, units), logR, logP, tab, p,
-                                         pre != 0, TRUNC);
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+    const int64_t b = xcd_unit(blockIdx.x, gridDim.x);
+    const FwdSeg<Win, W> sg = segs.of(b);
+    const int sub = kXforms<L, LOGE> > 1 ? (int)threadIdx.x >> (L - LOGE) : 0;
+    const int t = threadIdx.x & ((1 << (L - LOGE)) - 1);
+    const int64_t u0 = (b - uniform(sg.block0)) * kXforms<L, LOGE>, count = uniform(sg.count);
+    const bool live = kXforms<L, LOGE> == 1 || u0 + sub < count;  // (several transforms: logR = 0)
+    fwd_reg_body<Win, W, LOOSE, L, LOGE, MODE>(as_global(sg.in), uniform(sg.in_stride), uniform(sg.in_len),
+                                               as_global(sg.out), count, u0, sub, live,
+                                               reinterpret_cast<W *>(smem_raw) + sub * kXformLds<L>, t,
+                                               logR, logP, tab, p, TRUNC);
 }
 
 template <typename W, typename Wout, bool LOOSE, int L, int LOGE>
 __device__ __forceinline__ void inv_reg_body(const W *__restrict__ in, Wout *__restrict__ out,
                                              int64_t out_stride, int64_t lo, int64_t hi,
-                                             W *__restrict__ tmp, int64_t units, int64_t u,
-                                             int logR, int logP, const NttTab<W> &tab, W p,
-                                             bool trunc = false)
+                                             W *__restrict__ tmp, int64_t count, int64_t u0, int sub,
+                                             bool live, W *lds, int t, int logR, int logP,
+                                             const NttTab<W> &tab, W p, bool trunc)
 {
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-    W *lds = reinterpret_cast<W *>(smem_raw);
+    static_assert(sizeof(Wout) == 8, "outputs are 64-bit words");
     constexpr int E = 1 << LOGE, M = 1 << L;
-    const int t = threadIdx.x;
-    const int64_t e = u >> logR;
+    if constexpr (kXforms<L, LOGE> > 1)
+        logR = 0;
     const int R = 1 << logR;
-    const int gg = (int)(u & (R - 1));
+    const int64_t e0 = u0 >> logR;  // uniform
+    const int64_t e = live ? e0 + sub : e0;
+    const int gg = (int)(u0 & (R - 1));
     const int64_t N = (int64_t)M << logR;
-    const int64_t count = units >> logR;
     constexpr int SLAST = ((L - 1) / LOGE) * LOGE;
     if (trunc && R == 4 && gg == 3)  // dropped sub-transform (see fwd_reg_body)
         return;
@@ -1046,7 +1025,7 @@ __device__ __forceinline__ void inv_reg_body(const W *__restrict__ in, Wout *__r
     W x[E];
 #pragma unroll
     for (int g = 0; g < PSF::G; ++g) {
-        if (tq && PSF::index(t, g, 0) >= (3 << (L - 2))) {
+        if (tq && PSF::index(t, g, 0) >= 3 * (M / 4)) {
             // dropped quarter of a truncated product: never read
 #pragma unroll
             for (int j = 0; j < RUN; ++j)
@@ -1069,33 +1048,51 @@ __device__ __forceinline__ void inv_reg_body(const W *__restrict__ in, Wout *__r
     // inputs below 8p (the pointwise products' lazy outputs)
     inv_passes<W, LOOSE, L, LOGE, SLAST, 8>(x, tw, lds, t, tab, k, tq);
     // pass-0 arrangement: element j is index (j << (L-LOGE)) | t
-    if (R == 1 && tq) {
-        // truncated: scaled outputs corrected by the dropped quarter
-        // (trunc_correct); register j + q E/4 holds position i + q N/4
-        Wout *o = out + e * out_stride;
-        constexpr int E4 = E >> 2;
+    if (R == 1) {
+        // offsets of positions outside [lo, hi) fall outside the buffer
+        const int64_t width = hi - lo;
+        auto put = [&](auto store) __attribute__((always_inline)) {
+            if (tq) {
+                // truncated: scaled outputs corrected by the dropped quarter
+                // (trunc_correct); register j + q E/4 holds position i + q N/4
+                constexpr int E4 = E >> 2;
 #pragma unroll
-        for (int j = 0; j < E4; ++j) {
-            W c0 = shoup<W>(x[j], tab.ninv, tab.ninvq, p);
-            W c1 = shoup<W>(x[j + E4], tab.ninv, tab.ninvq, p);
-            W c2 = shoup<W>(x[j + 2 * E4], tab.ninv, tab.ninvq, p);
-            trunc_correct<W>(c0, c1, c2, shoup<W>(x[j + 3 * E4], tab.ninv, tab.ninvq, p), tab, p);
-            const int i1 = (j << (L - LOGE)) | t;
-            const int q1 = M >> 2;
-            if (i1 >= lo && i1 < hi)
-                o[i1 - lo] = (Wout)c0;
-            if (i1 + q1 >= lo && i1 + q1 < hi)
-                o[i1 + q1 - lo] = (Wout)c1;
-            if (i1 + 2 * q1 >= lo && i1 + 2 * q1 < hi)
-                o[i1 + 2 * q1 - lo] = (Wout)c2;
-        }
-    } else if (R == 1) {
-        Wout *o = out + e * out_stride;
+                for (int j = 0; j < E4; ++j) {
+                    W c0 = shoup<W>(x[j], tab.ninv, tab.ninvq, p);
+                    W c1 = shoup<W>(x[j + E4], tab.ninv, tab.ninvq, p);
+                    W c2 = shoup<W>(x[j + 2 * E4], tab.ninv, tab.ninvq, p);
+                    trunc_correct<W>(c0, c1, c2, shoup<W>(x[j + 3 * E4], tab.ninv, tab.ninvq, p), tab, p);
+                    const int i1 = (j << (L - LOGE)) | t;
+                    store(i1, (Wout)c0);
+                    store(i1 + (M >> 2), (Wout)c1);
+                    store(i1 + 2 * (M >> 2), (Wout)c2);
+                }
+            } else {
 #pragma unroll
-        for (int j = 0; j < E; ++j) {
-            const int i1 = (j << (L - LOGE)) | t;
-            if (i1 >= lo && i1 < hi)
-                o[i1 - lo] = (Wout)shoup<W>(x[j], tab.ninv, tab.ninvq, p);
+                for (int j = 0; j < E; ++j)
+                    store((j << (L - LOGE)) | t, (Wout)shoup<W>(x[j], tab.ninv, tab.ninvq, p));
+            }
+        };
+        if (kXforms<L, LOGE> == 1) {
+            // (N <= 2^14 positions: lo, hi and the offsets fit 32 bits)
+            const __amdgpu_buffer_rsrc_t r = buffer_of(out + e0 * out_stride, width * 8);
+            put([&](int i, Wout v) __attribute__((always_inline)) {
+                buffer_store(r, (uint32_t)(i - (int)lo) * 8, v);
+            });
+        } else if (out_stride < ((int64_t)1 << 20)) {
+            const __amdgpu_buffer_rsrc_t r =
+                buffer_of(out + e0 * out_stride, (int64_t)kXforms<L, LOGE> * out_stride * 8);
+            const uint32_t base = (uint32_t)sub * (uint32_t)out_stride * 8;
+            put([&](int i, Wout v) __attribute__((always_inline)) {
+                const bool in = i >= (int)lo && i < (int)hi && live;
+                buffer_store(r, in ? base + (uint32_t)(i - (int)lo) * 8 : kOutside, v);
+            });
+        } else {
+            Wout *o = out + e * out_stride;
+            put([&](int i, Wout v) __attribute__((always_inline)) {
+                if (i >= lo && i < hi && live)
+                    o[i - lo] = v;
+            });
         }
     } else {
         // lazy values: the merge pass starts with a Shoup product (twist),
@@ -1107,177 +1104,169 @@ __device__ __forceinline__ void inv_reg_body(const W *__restrict__ in, Wout *__r
     }
 }
 
-// With 16 elements per thread the inverse is held to 128 VGPRs, so that four
-// waves share each SIMD and hide the LDS-exchange latency.
 template <typename W, typename Wout, bool LOOSE, int L, int LOGE>
-__global__ void __launch_bounds__(1 << (L - LOGE)) __attribute__((amdgpu_waves_per_eu(LOGE == 4 ? kInvWaves : 1)))
-ntt_inv_reg(const W *__restrict__ in, Wout *__restrict__ out, int64_t out_stride, int64_t lo,
-            int64_t hi, W *__restrict__ tmp, int64_t units, int logR, int logP, NttTab<W> tab, W p,
-            int trunc)
+__global__ void __launch_bounds__((kXformThreads<L, LOGE>)) __attribute__((amdgpu_waves_per_eu(kXformWaves<LOGE>)))
+ntt_inv_reg(SegList<InvSeg<W, Wout>> segs, int logR, int logP, NttTab<W> tab, W p)
 {
-    inv_reg_body<W, Wout, LOOSE, L, LOGE>(in, out, out_stride, lo, hi, tmp, units,
-                                          xcd_unit(blockIdx.x, units), logR, logP, tab, p,
-                                          trunc != 0);
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+    const int64_t b = xcd_unit(blockIdx.x, gridDim.x);
+    const InvSeg<W, Wout> sg = segs.of(b);
+    const int sub = kXforms<L, LOGE> > 1 ? (int)threadIdx.x >> (L - LOGE) : 0;
+    const int t = threadIdx.x & ((1 << (L - LOGE)) - 1);
+    const int64_t u0 = (b - uniform(sg.block0)) * kXforms<L, LOGE>, count = uniform(sg.count);
+    const bool live = kXforms<L, LOGE> == 1 || u0 + sub < count;
+    inv_reg_body<W, Wout, LOOSE, L, LOGE>(as_global(sg.in), as_global(sg.out), uniform(sg.out_stride),
+                                          uniform(sg.lo), uniform(sg.hi), as_global(sg.tmp), count, u0, sub,
+                                          live,
+                                          reinterpret_cast<W *>(smem_raw) + sub * kXformLds<L>, t, logR,
+                                          logP, tab, p, __builtin_amdgcn_readfirstlane(sg.trunc) != 0);
 }
 
-// Register-kernel launchers.  logE (elements per thread) is a tuning
-// parameter: 4 (radix-16 passes, more threads, fewer registers) or 5
-// (radix-32 passes, fewer LDS exchanges).
-template <typename Win, typename W, bool LOOSE, int L, int LOGE, bool TRUNC>
-hipError_t launch_fwd_reg4(const Win *in, int64_t in_stride, int64_t in_len, W *out,
-                           int64_t units, int logR, int logP, const NttTab<W> &tab, W p,
-                           hipStream_t s, int pre)
+// workgroups of `count` entries (of 2^logR transforms of 2^logM points each)
+inline int64_t xform_blocks(int64_t count, int logM, int logR)
 {
-    constexpr int T = 1 << (L - LOGE);
-    const size_t lds = (size_t)((1 << L) + (1 << L) / 32) * sizeof(W);
-    static bool attr = false;
-    if (!attr) {
-        hipError_t e = hipFuncSetAttribute((const void *)ntt_fwd_reg<Win, W, LOOSE, L, LOGE, TRUNC>,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess)
-            return e;
-        attr = true;
+    if (logM >= 11)
+        return count << logR;
+    const int nb = 256 >> (logM - small_log_e(logM));
+    return (count + nb - 1) / nb;
+}
+
+// Register-kernel launchers.  From 2^12 points on, logE (log2 of the elements
+// per thread) is a tuning parameter: 4 (radix-16 passes, more threads, fewer
+// registers) or 5 (radix-32 passes, fewer LDS exchanges).
+template <int L, int LOGE, typename W, typename Kern, typename... Args>
+hipError_t launch_xform(Kern *kern, int64_t blocks, hipStream_t s, Args... args)
+{
+    constexpr size_t lds = (size_t)kXforms<L, LOGE> * kXformLds<L> * sizeof(W);
+    if constexpr (lds > 64 * 1024) {
+        static bool attr = false;
+        if (!attr) {
+            hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                               (int)lds);
+            if (e != hipSuccess)
+                return e;
+            attr = true;
+        }
     }
-    hipLaunchKernelGGL((ntt_fwd_reg<Win, W, LOOSE, L, LOGE, TRUNC>), dim3((unsigned)units), dim3(T),
-                       lds, s, in, in_stride, in_len, out, units, logR, logP, tab, p, pre);
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kXformThreads<L, LOGE>), lds, s, args...);
     return hipGetLastError();
 }
 
-// pre: bit 0 the column pass's rows as input, bit 1 a 3/4-truncated transform
 template <typename Win, typename W, bool LOOSE, int L, int LOGE>
-hipError_t launch_fwd_reg3(const Win *in, int64_t in_stride, int64_t in_len, W *out,
-                           int64_t units, int logR, int logP, const NttTab<W> &tab, W p,
-                           hipStream_t s, int pre)
+hipError_t launch_fwd_e(const SegList<FwdSeg<Win, W>> &segs, int64_t blocks, int logR, int logP,
+                        const NttTab<W> &tab, W p, hipStream_t s, bool pre, bool trunc)
 {
-    if (pre & 2)
-        return launch_fwd_reg4<Win, W, LOOSE, L, LOGE, true>(in, in_stride, in_len, out, units,
-                                                             logR, logP, tab, p, s, pre & 1);
-    return launch_fwd_reg4<Win, W, LOOSE, L, LOGE, false>(in, in_stride, in_len, out, units, logR,
-                                                          logP, tab, p, s, pre & 1);
-}
-
-template <typename W, typename Wout, bool LOOSE, int L, int LOGE>
-hipError_t launch_inv_reg3(const W *in, Wout *out, int64_t out_stride, int64_t lo, int64_t hi,
-                           W *tmp, int64_t units, int logR, int logP, const NttTab<W> &tab, W p,
-                           hipStream_t s, int trunc)
-{
-    constexpr int T = 1 << (L - LOGE);
-    const size_t lds = (size_t)((1 << L) + (1 << L) / 32) * sizeof(W);
-    static bool attr = false;
-    if (!attr) {
-        hipError_t e = hipFuncSetAttribute((const void *)ntt_inv_reg<W, Wout, LOOSE, L, LOGE>,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess)
-            return e;
-        attr = true;
-    }
-    hipLaunchKernelGGL((ntt_inv_reg<W, Wout, LOOSE, L, LOGE>), dim3((unsigned)units), dim3(T), lds,
-                       s, in, out, out_stride, lo, hi, tmp, units, logR, logP, tab, p, trunc);
-    return hipGetLastError();
-}
-
-template <typename Win, typename W, bool LOOSE, int L>
-hipError_t launch_fwd_reg2(int logE, const Win *in, int64_t in_stride, int64_t in_len, W *out,
-                           int64_t units, int logR, int logP, const NttTab<W> &tab, W p,
-                           hipStream_t s, int pre)
-{
-    if (logE == 5 && L >= 12)
-        return launch_fwd_reg3<Win, W, LOOSE, L, (L >= 12 ? 5 : 4)>(in, in_stride, in_len, out,
-                                                                   units, logR, logP, tab, p, s,
-                                                                   pre);
-    return launch_fwd_reg3<Win, W, LOOSE, L, 4>(in, in_stride, in_len, out, units, logR, logP, tab,
-                                                p, s, pre);
-}
-
-template <typename W, typename Wout, bool LOOSE, int L>
-hipError_t launch_inv_reg2(int logE, const W *in, Wout *out, int64_t out_stride, int64_t lo,
-                           int64_t hi, W *tmp, int64_t units, int logR, int logP,
-                           const NttTab<W> &tab, W p, hipStream_t s, int trunc)
-{
-    if (logE == 5 && L >= 12)
-        return launch_inv_reg3<W, Wout, LOOSE, L, (L >= 12 ? 5 : 4)>(in, out, out_stride, lo, hi,
-                                                                    tmp, units, logR, logP, tab,
-                                                                    p, s, trunc);
-    return launch_inv_reg3<W, Wout, LOOSE, L, 4>(in, out, out_stride, lo, hi, tmp, units, logR,
-                                                 logP, tab, p, s, trunc);
+    constexpr int top = NttLimits<W>::max_log_m;
+    if constexpr (L == top)
+        if (pre)
+            return launch_xform<L, LOGE, W>(ntt_fwd_reg<Win, W, LOOSE, L, LOGE, kRows, false>, blocks, s, segs,
+                                            logR, logP, tab, p);
+    if constexpr (L >= top - 1)
+        if (logR > 0) {
+            if (trunc)
+                return launch_xform<L, LOGE, W>(ntt_fwd_reg<Win, W, LOOSE, L, LOGE, kSplit, true>, blocks, s,
+                                                segs, logR, logP, tab, p);
+            if constexpr (L == top)
+                return launch_xform<L, LOGE, W>(ntt_fwd_reg<Win, W, LOOSE, L, LOGE, kSplit, false>, blocks, s,
+                                                segs, logR, logP, tab, p);
+        }
+    if (pre || logR > 0)
+        return hipErrorInvalidValue;
+    if constexpr (L >= kTruncMinLog)
+        if (trunc)
+            return launch_xform<L, LOGE, W>(ntt_fwd_reg<Win, W, LOOSE, L, LOGE, kWhole, true>, blocks, s, segs,
+                                            logR, logP, tab, p);
+    return launch_xform<L, LOGE, W>(ntt_fwd_reg<Win, W, LOOSE, L, LOGE, kWhole, false>, blocks, s, segs, logR,
+                                    logP, tab, p);
 }
 
 template <typename Win, typename W, int L>
-hipError_t launch_fwd_reg(int logE, const Win *in, int64_t in_stride, int64_t in_len, W *out,
-                          int64_t units, int logR, int logP, const NttTab<W> &tab, W p,
-                          hipStream_t s, int pre)
+hipError_t launch_fwd_l(int logE, const SegList<FwdSeg<Win, W>> &segs, int64_t blocks, int logR, int logP,
+                        const NttTab<W> &tab, W p, hipStream_t s, bool pre, bool trunc)
 {
-    if constexpr (sizeof(W) == 8) {
-        if ((uint64_t)p < ((uint64_t)1 << 60))
-            return launch_fwd_reg2<Win, W, true, L>(logE, in, in_stride, in_len, out, units, logR,
-                                                    logP, tab, p, s, pre);
+    constexpr int E4 = L >= 11 ? 4 : small_log_e(L), E5 = L >= 12 ? 5 : E4;
+    if (sizeof(W) == 8 && (uint64_t)p < ((uint64_t)1 << 60)) {
+        if constexpr (sizeof(W) == 8) {
+            if (logE == 5)
+                return launch_fwd_e<Win, W, true, L, E5>(segs, blocks, logR, logP, tab, p, s, pre, trunc);
+            return launch_fwd_e<Win, W, true, L, E4>(segs, blocks, logR, logP, tab, p, s, pre, trunc);
+        }
     }
-    return launch_fwd_reg2<Win, W, false, L>(logE, in, in_stride, in_len, out, units, logR, logP,
-                                             tab, p, s, pre);
+    if (logE == 5)
+        return launch_fwd_e<Win, W, false, L, E5>(segs, blocks, logR, logP, tab, p, s, pre, trunc);
+    return launch_fwd_e<Win, W, false, L, E4>(segs, blocks, logR, logP, tab, p, s, pre, trunc);
 }
 
 template <typename W, typename Wout, int L>
-hipError_t launch_inv_reg(int logE, const W *in, Wout *out, int64_t out_stride, int64_t lo,
-                          int64_t hi, W *tmp, int64_t units, int logR, int logP,
-                          const NttTab<W> &tab, W p, hipStream_t s, int trunc)
+hipError_t launch_inv_l(int logE, const SegList<InvSeg<W, Wout>> &segs, int64_t blocks, int logR, int logP,
+                        const NttTab<W> &tab, W p, hipStream_t s)
 {
+    constexpr int E4 = L >= 11 ? 4 : small_log_e(L), E5 = L >= 12 ? 5 : E4;
     if constexpr (sizeof(W) == 8) {
-        if ((uint64_t)p < ((uint64_t)1 << 60))
-            return launch_inv_reg2<W, Wout, true, L>(logE, in, out, out_stride, lo, hi, tmp, units,
-                                                     logR, logP, tab, p, s, trunc);
+        if ((uint64_t)p < ((uint64_t)1 << 60)) {
+            if (logE == 5)
+                return launch_xform<L, E5, W>(ntt_inv_reg<W, Wout, true, L, E5>, blocks, s, segs, logR, logP,
+                                              tab, p);
+            return launch_xform<L, E4, W>(ntt_inv_reg<W, Wout, true, L, E4>, blocks, s, segs, logR, logP, tab,
+                                          p);
+        }
     }
-    return launch_inv_reg2<W, Wout, false, L>(logE, in, out, out_stride, lo, hi, tmp, units, logR,
-                                              logP, tab, p, s, trunc);
+    if (logE == 5)
+        return launch_xform<L, E5, W>(ntt_inv_reg<W, Wout, false, L, E5>, blocks, s, segs, logR, logP, tab, p);
+    return launch_xform<L, E4, W>(ntt_inv_reg<W, Wout, false, L, E4>, blocks, s, segs, logR, logP, tab, p);
+}
+
+// f with the sub-transform's size as a compile-time constant
+template <typename W, typename F>
+hipError_t with_log_m(int logM, F f)
+{
+    switch (logM) {
+#define PMLG_CASE(L_)                               \
+    case L_:                                        \
+        return f(std::integral_constant<int, L_>{});
+        PMLG_CASE(1)
+        PMLG_CASE(2)
+        PMLG_CASE(3)
+        PMLG_CASE(4)
+        PMLG_CASE(5)
+        PMLG_CASE(6)
+        PMLG_CASE(7)
+        PMLG_CASE(8)
+        PMLG_CASE(9)
+        PMLG_CASE(10)
+        PMLG_CASE(11)
+        PMLG_CASE(12)
+        PMLG_CASE(13)
+    case 14:
+        if constexpr (sizeof(W) == 4)
+            return f(std::integral_constant<int, 14>{});
+        [[fallthrough]];
+    default:
+        return hipErrorInvalidValue;
+#undef PMLG_CASE
+    }
 }
 
 template <typename Win, typename W>
-hipError_t dispatch_fwd_reg(int logM, int logE, const Win *in, int64_t in_stride, int64_t in_len,
-                            W *out, int64_t units, int logR, int logP, const NttTab<W> &tab, W p,
-                            hipStream_t s, int pre = 0)
+hipError_t dispatch_fwd(int logM, int logE, const SegList<FwdSeg<Win, W>> &segs, int64_t blocks, int logR,
+                        int logP, const NttTab<W> &tab, W p, hipStream_t s, bool pre, bool trunc)
 {
-    switch (logM) {
-    case 11:
-        return launch_fwd_reg<Win, W, 11>(logE, in, in_stride, in_len, out, units, logR, logP, tab,
-                                          p, s, pre);
-    case 12:
-        return launch_fwd_reg<Win, W, 12>(logE, in, in_stride, in_len, out, units, logR, logP, tab,
-                                          p, s, pre);
-    case 13:
-        return launch_fwd_reg<Win, W, 13>(logE, in, in_stride, in_len, out, units, logR, logP, tab,
-                                          p, s, pre);
-    case 14:
-        if constexpr (sizeof(W) == 4)
-            return launch_fwd_reg<Win, W, 14>(logE, in, in_stride, in_len, out, units, logR, logP,
-                                              tab, p, s, pre);
-        [[fallthrough]];
-    default:
+    if (blocks > INT32_MAX || (logM < kRegMinLog && logR > 0))
         return hipErrorInvalidValue;
-    }
+    return with_log_m<W>(logM, [&](auto l) {
+        return launch_fwd_l<Win, W, decltype(l)::value>(logE, segs, blocks, logR, logP, tab, p, s, pre, trunc);
+    });
 }
 
 template <typename W, typename Wout>
-hipError_t dispatch_inv_reg(int logM, int logE, const W *in, Wout *out, int64_t out_stride,
-                            int64_t lo, int64_t hi, W *tmp, int64_t units, int logR, int logP,
-                            const NttTab<W> &tab, W p, hipStream_t s, int trunc = 0)
+hipError_t dispatch_inv(int logM, int logE, const SegList<InvSeg<W, Wout>> &segs, int64_t blocks, int logR,
+                        int logP, const NttTab<W> &tab, W p, hipStream_t s)
 {
-    switch (logM) {
-    case 11:
-        return launch_inv_reg<W, Wout, 11>(logE, in, out, out_stride, lo, hi, tmp, units, logR,
-                                           logP, tab, p, s, trunc);
-    case 12:
-        return launch_inv_reg<W, Wout, 12>(logE, in, out, out_stride, lo, hi, tmp, units, logR,
-                                           logP, tab, p, s, trunc);
-    case 13:
-        return launch_inv_reg<W, Wout, 13>(logE, in, out, out_stride, lo, hi, tmp, units, logR,
-                                           logP, tab, p, s, trunc);
-    case 14:
-        if constexpr (sizeof(W) == 4)
-            return launch_inv_reg<W, Wout, 14>(logE, in, out, out_stride, lo, hi, tmp, units, logR,
-                                               logP, tab, p, s, trunc);
-        [[fallthrough]];
-    default:
+    if (blocks > INT32_MAX || (logM < kRegMinLog && logR > 0))
         return hipErrorInvalidValue;
-    }
+    return with_log_m<W>(logM, [&](auto l) {
+        return launch_inv_l<W, Wout, decltype(l)::value>(logE, segs, blocks, logR, logP, tab, p, s);
+    });
 }
 
 // ===========================================================================
@@ -1435,8 +1424,6 @@ hipError_t launch_cols_inv(const W *tmp, Wout *out, int64_t out_stride, int64_t 
     return hipGetLastError();
 }
 
-constexpr int kRegMinLog = 11;
-
 // Stage tables for sub-transforms of 2^logM points.  The tables of length
 // 2^logN are built for min(logN, max_log_m); a truncated transform split in
 // four one level below that (logN = max_log_m + 1) uses the larger table's
@@ -1456,45 +1443,60 @@ NttTab<W> tab_for_sub(const NttTab<W> &tab, int logN, int logM)
 
 }  // namespace
 
+template <typename W>
+static int sub_log_m(int logN, bool trunc)
+{
+    // a truncated transform longer than one sub-transform is split in four
+    if (trunc && logN > NttLimits<W>::max_log_m)
+        return logN - 2;
+    return logN < NttLimits<W>::max_log_m ? logN : NttLimits<W>::max_log_m;
+}
+
 template <typename Win, typename W>
-hipError_t launch_ntt_fwd(const Win *in, int64_t in_stride, int64_t in_len, W *out,
-                          int64_t count, int logN, int logP, const NttTune &tune,
-                          const NttTab<W> &tab, W p, hipStream_t s, Win *tmp,
+hipError_t launch_ntt_fwd(const FwdOp<Win, W> *ops, int nops, int logN, int logP,
+                          const NttTune &tune, const NttTab<W> &tab, W p, hipStream_t s, Win *tmp,
                           const ColTab<W> *ct, bool trunc)
 {
-    if (count <= 0)
-        return hipSuccess;
-    // a truncated transform longer than one sub-transform is split in four
-    const int logM = trunc && logN > NttLimits<W>::max_log_m
-                         ? logN - 2
-                         : (logN < NttLimits<W>::max_log_m ? logN : NttLimits<W>::max_log_m);
+    const int logM = sub_log_m<W>(logN, trunc);
     const int logR = logN - logM;
-    if (logR > NttLimits<W>::max_log_r || logP > logN)
+    if (logR > NttLimits<W>::max_log_r || logP > logN || logN < 1 || nops < 1 || nops > 2)
         return hipErrorInvalidValue;
     if (trunc && (logR > 2 || logN < kTruncMinLog || (logR > 0 && logM < kRegMinLog)))
         return hipErrorInvalidValue;
-    const int64_t units = count << logR;
+    const int64_t N = (int64_t)1 << logN;
     if (logR > 2) {
-        // long transform: column pass into tmp, then the rows
+        // long transforms: column pass into tmp, then the rows, one operand
+        // after the other
         if (!tmp || !ct)
             return hipErrorInvalidValue;
-        hipError_t e = launch_cols_fwd<Win, W>(in, in_stride, in_len, tmp, count, logM, logR, *ct,
-                                               p, s);
-        if (e != hipSuccess)
-            return e;
-        return dispatch_fwd_reg<Win, W>(logM, tune.fwd_log_e, tmp, (int64_t)1 << logN,
-                                        (int64_t)1 << logN, out, units, logR, logP, tab, p, s, 1);
+        for (int i = 0; i < nops; ++i) {
+            const FwdOp<Win, W> &o = ops[i];
+            if (o.count <= 0)
+                continue;
+            hipError_t e = launch_cols_fwd<Win, W>(o.in, o.in_stride, o.in_len, tmp, o.count, logM, logR,
+                                                   *ct, p, s);
+            if (e != hipSuccess)
+                return e;
+            SegList<FwdSeg<Win, W>> segs{nullptr, 1, {{tmp, o.out, N, N, o.count, 0, 0, 0}, {}}};
+            e = dispatch_fwd<Win, W>(logM, tune.fwd_log_e, segs, xform_blocks(o.count, logM, logR), logR,
+                                     logP, tab, p, s, true, false);
+            if (e != hipSuccess)
+                return e;
+        }
+        return hipSuccess;
     }
-    if (logM >= kRegMinLog)
-        return dispatch_fwd_reg<Win, W>(logM, tune.fwd_log_e, in, in_stride, in_len, out, units,
-                                        logR, logP, tab_for_sub(tab, logN, logM), p, s,
-                                        trunc ? 2 : 0);
-    const int lognb = pick_lognb(logM);
-    const int64_t blocks = (units + (1 << lognb) - 1) >> lognb;
-    const size_t lds = ((size_t)1 << (logM + lognb)) * sizeof(W);
-    hipLaunchKernelGGL((ntt_fwd_kernel<Win, W>), dim3((unsigned)blocks), dim3(kThreads), lds, s, in,
-                       in_stride, in_len, out, units, logN, logR, lognb, logP, tab, p, trunc ? 1 : 0);
-    return hipGetLastError();
+    SegList<FwdSeg<Win, W>> segs{nullptr, 0, {}};
+    int64_t blocks = 0;
+    for (int i = 0; i < nops; ++i)
+        if (ops[i].count > 0) {
+            segs.s[segs.n++] = FwdSeg<Win, W>{ops[i].in, ops[i].out, ops[i].in_stride, ops[i].in_len,
+                                              ops[i].count, blocks, 0, 0};
+            blocks += xform_blocks(ops[i].count, logM, logR);
+        }
+    if (blocks == 0)
+        return hipSuccess;
+    return dispatch_fwd<Win, W>(logM, tune.fwd_log_e, segs, blocks, logR, logP,
+                                tab_for_sub(tab, logN, logM), p, s, false, trunc);
 }
 
 template <typename W, typename Wout>
@@ -1508,30 +1510,16 @@ hipError_t launch_ntt_inv(const W *in, Wout *out, int64_t out_stride, int64_t lo
         hi = N;
     if (count <= 0 || hi <= lo)
         return hipSuccess;
-    const int logM = trunc && logN > NttLimits<W>::max_log_m
-                         ? logN - 2
-                         : (logN < NttLimits<W>::max_log_m ? logN : NttLimits<W>::max_log_m);
+    const int logM = sub_log_m<W>(logN, trunc);
     const int logR = logN - logM;
-    if (logR > NttLimits<W>::max_log_r || (logR > 0 && tmp == nullptr) || logP > logN ||
+    if (logR > NttLimits<W>::max_log_r || (logR > 0 && tmp == nullptr) || logP > logN || logN < 1 ||
         (logR > 2 && (!ct || logM < kRegMinLog)) ||
         (trunc && (logR > 2 || logN < kTruncMinLog || hi > 3 * (N >> 2) ||
                    (logR > 0 && logM < kRegMinLog))))
         return hipErrorInvalidValue;
-    const int64_t units = count << logR;
-    hipError_t err;
-    if (logM >= kRegMinLog) {
-        err = dispatch_inv_reg<W, Wout>(logM, tune.inv_log_e, in, out, out_stride, lo, hi, tmp,
-                                        units, logR, logP, tab_for_sub(tab, logN, logM), p, s,
-                                        trunc ? 1 : 0);
-    } else {
-        const int lognb = pick_lognb(logM);
-        const int64_t blocks = (units + (1 << lognb) - 1) >> lognb;
-        const size_t lds = ((size_t)1 << (logM + lognb)) * sizeof(W);
-        hipLaunchKernelGGL((ntt_inv_kernel<W, Wout>), dim3((unsigned)blocks), dim3(kThreads), lds,
-                           s, in, out, out_stride, lo, hi, tmp, units, logN, logR, lognb, logP,
-                           tab, p, trunc ? 1 : 0);
-        err = hipGetLastError();
-    }
+    SegList<InvSeg<W, Wout>> segs{nullptr, 1, {{in, out, tmp, out_stride, lo, hi, count, 0, 0, trunc, 0}, {}}};
+    hipError_t err = dispatch_inv<W, Wout>(logM, tune.inv_log_e, segs, xform_blocks(count, logM, logR), logR,
+                                           logP, tab_for_sub(tab, logN, logM), p, s);
     if (err != hipSuccess || logR == 0)
         return err;
     if (logR > 2)
@@ -1564,20 +1552,6 @@ hipError_t launch_ntt_inv(const W *in, Wout *out, int64_t out_stride, int64_t lo
 namespace {
 
 template <typename S>
-__device__ __forceinline__ const S &seg_of(const S *segs, int nseg, int64_t b)
-{
-    int lo = 0, hi = nseg - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (segs[mid].block0 <= b)
-            lo = mid;
-        else
-            hi = mid - 1;
-    }
-    return segs[lo];
-}
-
-template <typename S>
 __device__ __forceinline__ const S &mseg_of(const S *segs, int nseg, int64_t b)
 {
     int lo = 0, hi = nseg - 1;
@@ -1589,52 +1563,6 @@ __device__ __forceinline__ const S &mseg_of(const S *segs, int nseg, int64_t b)
             hi = mid - 1;
     }
     return segs[lo];
-}
-
-template <typename Win, typename W>
-__global__ void __launch_bounds__(kThreads)
-ntt_fwd_segs_lds(const FwdSeg<Win, W> *__restrict__ segs, int nseg, int logN, int logR, int lognb,
-                 int logP, NttTab<W> tab, W p)
-{
-    const int64_t b = xcd_unit(blockIdx.x, gridDim.x);
-    const FwdSeg<Win, W> &sg = seg_of(segs, nseg, b);
-    fwd_lds_body<Win, W>(sg.in, sg.in_stride, sg.in_len, sg.out, sg.count << logR,
-                         (b - sg.block0) << lognb, logN, logR, lognb, logP, tab, p, sg.trunc != 0);
-}
-
-template <typename W, typename Wout>
-__global__ void __launch_bounds__(kThreads)
-ntt_inv_segs_lds(const InvSeg<W, Wout> *__restrict__ segs, int nseg, int logN, int logR,
-                 int lognb, int logP, NttTab<W> tab, W p)
-{
-    const int64_t b = xcd_unit(blockIdx.x, gridDim.x);
-    const InvSeg<W, Wout> &sg = seg_of(segs, nseg, b);
-    inv_lds_body<W, Wout>(sg.in, sg.out, sg.out_stride, sg.lo, sg.hi, sg.tmp, sg.count << logR,
-                          (b - sg.block0) << lognb, logN, logR, lognb, logP, tab, p, sg.trunc != 0);
-}
-
-// every segment of one launch has the launch's TRUNC (see ntt_fwd_reg)
-template <typename Win, typename W, bool LOOSE, int L, int LOGE, bool TRUNC>
-__global__ void __launch_bounds__(1 << (L - LOGE)) __attribute__((amdgpu_waves_per_eu(LOGE == 5 ? kFwdWaves32 : 1)))
-ntt_fwd_segs_reg(const FwdSeg<Win, W> *__restrict__ segs, int nseg, int logR, int logP,
-                 NttTab<W> tab, W p)
-{
-    const int64_t b = xcd_unit(blockIdx.x, gridDim.x);
-    const FwdSeg<Win, W> &sg = seg_of(segs, nseg, b);
-    fwd_reg_body<Win, W, LOOSE, L, LOGE>(sg.in, sg.in_stride, sg.in_len, sg.out, sg.count << logR,
-                                         b - sg.block0, logR, logP, tab, p, false, TRUNC);
-}
-
-template <typename W, typename Wout, bool LOOSE, int L, int LOGE>
-__global__ void __launch_bounds__(1 << (L - LOGE)) __attribute__((amdgpu_waves_per_eu(LOGE == 4 ? kInvWaves : 1)))
-ntt_inv_segs_reg(const InvSeg<W, Wout> *__restrict__ segs, int nseg, int logR, int logP,
-                 NttTab<W> tab, W p)
-{
-    const int64_t b = xcd_unit(blockIdx.x, gridDim.x);
-    const InvSeg<W, Wout> &sg = seg_of(segs, nseg, b);
-    inv_reg_body<W, Wout, LOOSE, L, LOGE>(sg.in, sg.out, sg.out_stride, sg.lo, sg.hi, sg.tmp,
-                                          sg.count << logR, b - sg.block0, logR, logP, tab, p,
-                                          sg.trunc != 0);
 }
 
 template <typename W, typename Wout>
@@ -1655,119 +1583,13 @@ ntt_merge_segs(const InvSeg<W, Wout> *__restrict__ segs, int nseg, int logN, int
         merge_one<W, Wout>(sg.tmp, sg.out, sg.out_stride, sg.lo, width, idx, logN, logR, tab, p);
 }
 
-template <typename Kern>
-hipError_t set_lds_attr(Kern *k, size_t lds, bool &done)
-{
-    if (done || lds <= 64 * 1024)
-        return hipSuccess;
-    hipError_t e = hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       (int)lds);
-    if (e == hipSuccess)
-        done = true;
-    return e;
-}
-
-template <typename Win, typename W, bool LOOSE, int L, int LOGE, bool TRUNC>
-hipError_t fwd_segs_reg4(const FwdSeg<Win, W> *segs, int nseg, int64_t blocks, int logR, int logP,
-                         const NttTab<W> &tab, W p, hipStream_t s)
-{
-    const size_t lds = (size_t)((1 << L) + (1 << L) / 32) * sizeof(W);
-    static bool attr = false;
-    hipError_t e = set_lds_attr(ntt_fwd_segs_reg<Win, W, LOOSE, L, LOGE, TRUNC>, lds, attr);
-    if (e != hipSuccess)
-        return e;
-    hipLaunchKernelGGL((ntt_fwd_segs_reg<Win, W, LOOSE, L, LOGE, TRUNC>), dim3((unsigned)blocks),
-                       dim3(1 << (L - LOGE)), lds, s, segs, nseg, logR, logP, tab, p);
-    return hipGetLastError();
-}
-
-template <typename Win, typename W, bool LOOSE, int L, int LOGE>
-hipError_t fwd_segs_reg3(const FwdSeg<Win, W> *segs, int nseg, int64_t blocks, int logR, int logP,
-                         const NttTab<W> &tab, W p, hipStream_t s, bool trunc)
-{
-    if (trunc)
-        return fwd_segs_reg4<Win, W, LOOSE, L, LOGE, true>(segs, nseg, blocks, logR, logP, tab, p,
-                                                           s);
-    return fwd_segs_reg4<Win, W, LOOSE, L, LOGE, false>(segs, nseg, blocks, logR, logP, tab, p, s);
-}
-
-template <typename W, typename Wout, bool LOOSE, int L, int LOGE>
-hipError_t inv_segs_reg3(const InvSeg<W, Wout> *segs, int nseg, int64_t blocks, int logR, int logP,
-                         const NttTab<W> &tab, W p, hipStream_t s)
-{
-    const size_t lds = (size_t)((1 << L) + (1 << L) / 32) * sizeof(W);
-    static bool attr = false;
-    hipError_t e = set_lds_attr(ntt_inv_segs_reg<W, Wout, LOOSE, L, LOGE>, lds, attr);
-    if (e != hipSuccess)
-        return e;
-    hipLaunchKernelGGL((ntt_inv_segs_reg<W, Wout, LOOSE, L, LOGE>), dim3((unsigned)blocks),
-                       dim3(1 << (L - LOGE)), lds, s, segs, nseg, logR, logP, tab, p);
-    return hipGetLastError();
-}
-
-template <typename Win, typename W, bool LOOSE, int L>
-hipError_t fwd_segs_reg2(int logE, const FwdSeg<Win, W> *segs, int nseg, int64_t blocks, int logR,
-                         int logP, const NttTab<W> &tab, W p, hipStream_t s, bool trunc)
-{
-    if (logE == 5 && L >= 12)
-        return fwd_segs_reg3<Win, W, LOOSE, L, (L >= 12 ? 5 : 4)>(segs, nseg, blocks, logR, logP,
-                                                                 tab, p, s, trunc);
-    return fwd_segs_reg3<Win, W, LOOSE, L, 4>(segs, nseg, blocks, logR, logP, tab, p, s, trunc);
-}
-
-template <typename W, typename Wout, bool LOOSE, int L>
-hipError_t inv_segs_reg2(int logE, const InvSeg<W, Wout> *segs, int nseg, int64_t blocks,
-                         int logR, int logP, const NttTab<W> &tab, W p, hipStream_t s)
-{
-    if (logE == 5 && L >= 12)
-        return inv_segs_reg3<W, Wout, LOOSE, L, (L >= 12 ? 5 : 4)>(segs, nseg, blocks, logR, logP,
-                                                                  tab, p, s);
-    return inv_segs_reg3<W, Wout, LOOSE, L, 4>(segs, nseg, blocks, logR, logP, tab, p, s);
-}
-
-template <typename Win, typename W, int L>
-hipError_t fwd_segs_reg(int logE, const FwdSeg<Win, W> *segs, int nseg, int64_t blocks, int logR,
-                        int logP, const NttTab<W> &tab, W p, hipStream_t s, bool trunc)
-{
-    if constexpr (sizeof(W) == 8) {
-        if ((uint64_t)p < ((uint64_t)1 << 60))
-            return fwd_segs_reg2<Win, W, true, L>(logE, segs, nseg, blocks, logR, logP, tab, p, s,
-                                                  trunc);
-    }
-    return fwd_segs_reg2<Win, W, false, L>(logE, segs, nseg, blocks, logR, logP, tab, p, s, trunc);
-}
-
-template <typename W, typename Wout, int L>
-hipError_t inv_segs_reg(int logE, const InvSeg<W, Wout> *segs, int nseg, int64_t blocks, int logR,
-                        int logP, const NttTab<W> &tab, W p, hipStream_t s)
-{
-    if constexpr (sizeof(W) == 8) {
-        if ((uint64_t)p < ((uint64_t)1 << 60))
-            return inv_segs_reg2<W, Wout, true, L>(logE, segs, nseg, blocks, logR, logP, tab, p, s);
-    }
-    return inv_segs_reg2<W, Wout, false, L>(logE, segs, nseg, blocks, logR, logP, tab, p, s);
-}
-
-template <typename W>
-int seg_log_m(int logN, bool trunc)
-{
-    // a truncated product longer than one sub-transform is split in four
-    if (trunc && logN > NttLimits<W>::max_log_m)
-        return logN - 2;
-    return logN < NttLimits<W>::max_log_m ? logN : NttLimits<W>::max_log_m;
-}
-
 }  // namespace
 
 template <typename W>
 int64_t ntt_seg_blocks(int64_t count, int logN, bool trunc)
 {
-    const int logM = seg_log_m<W>(logN, trunc);
-    const int64_t units = count << (logN - logM);
-    if (logM >= kRegMinLog)
-        return units;
-    const int lognb = pick_lognb(logM);
-    return (units + (1 << lognb) - 1) >> lognb;
+    const int logM = sub_log_m<W>(logN, trunc);
+    return xform_blocks(count, logM, logN - logM);
 }
 
 template <typename W>
@@ -1787,36 +1609,12 @@ hipError_t launch_ntt_fwd_segs(const FwdSeg<Win, W> *segs, int nseg, int64_t blo
 {
     if (nseg <= 0 || blocks <= 0)
         return hipSuccess;
-    const int logM = seg_log_m<W>(logN, trunc);
+    const int logM = sub_log_m<W>(logN, trunc);
     const int logR = logN - logM;
-    if (logR > 2 || logP > logN || blocks > INT32_MAX)
+    if (logR > 2 || logP > logN || logN < 1)
         return hipErrorInvalidValue;
-    const NttTab<W> st = tab_for_sub(tab, logN, logM);
-    if (logM >= kRegMinLog) {
-        switch (logM) {
-        case 11:
-            return fwd_segs_reg<Win, W, 11>(log_e, segs, nseg, blocks, logR, logP, st, p, s,
-                                             trunc);
-        case 12:
-            return fwd_segs_reg<Win, W, 12>(log_e, segs, nseg, blocks, logR, logP, st, p, s,
-                                             trunc);
-        case 13:
-            return fwd_segs_reg<Win, W, 13>(log_e, segs, nseg, blocks, logR, logP, st, p, s,
-                                             trunc);
-        case 14:
-            if constexpr (sizeof(W) == 4)
-                return fwd_segs_reg<Win, W, 14>(log_e, segs, nseg, blocks, logR, logP, st, p, s,
-                                                 trunc);
-            [[fallthrough]];
-        default:
-            return hipErrorInvalidValue;
-        }
-    }
-    const int lognb = pick_lognb(logM);
-    const size_t lds = ((size_t)1 << (logM + lognb)) * sizeof(W);
-    hipLaunchKernelGGL((ntt_fwd_segs_lds<Win, W>), dim3((unsigned)blocks), dim3(kThreads), lds, s,
-                       segs, nseg, logN, logR, lognb, logP, tab, p);
-    return hipGetLastError();
+    return dispatch_fwd<Win, W>(logM, log_e, SegList<FwdSeg<Win, W>>{segs, nseg, {}}, blocks, logR, logP,
+                                tab_for_sub(tab, logN, logM), p, s, false, trunc);
 }
 
 template <typename W, typename Wout>
@@ -1826,39 +1624,12 @@ hipError_t launch_ntt_inv_segs(const InvSeg<W, Wout> *segs, int nseg, int64_t bl
 {
     if (nseg <= 0 || blocks <= 0)
         return hipSuccess;
-    const int logM = seg_log_m<W>(logN, trunc);
+    const int logM = sub_log_m<W>(logN, trunc);
     const int logR = logN - logM;
-    if (logR > 2 || logP > logN || blocks > INT32_MAX || mblocks > INT32_MAX)
+    if (logR > 2 || logP > logN || logN < 1 || mblocks > INT32_MAX)
         return hipErrorInvalidValue;
-    const NttTab<W> st = tab_for_sub(tab, logN, logM);
-    hipError_t err;
-    if (logM >= kRegMinLog) {
-        switch (logM) {
-        case 11:
-            err = inv_segs_reg<W, Wout, 11>(log_e, segs, nseg, blocks, logR, logP, st, p, s);
-            break;
-        case 12:
-            err = inv_segs_reg<W, Wout, 12>(log_e, segs, nseg, blocks, logR, logP, st, p, s);
-            break;
-        case 13:
-            err = inv_segs_reg<W, Wout, 13>(log_e, segs, nseg, blocks, logR, logP, st, p, s);
-            break;
-        case 14:
-            if constexpr (sizeof(W) == 4) {
-                err = inv_segs_reg<W, Wout, 14>(log_e, segs, nseg, blocks, logR, logP, st, p, s);
-                break;
-            }
-            [[fallthrough]];
-        default:
-            return hipErrorInvalidValue;
-        }
-    } else {
-        const int lognb = pick_lognb(logM);
-        const size_t lds = ((size_t)1 << (logM + lognb)) * sizeof(W);
-        hipLaunchKernelGGL((ntt_inv_segs_lds<W, Wout>), dim3((unsigned)blocks), dim3(kThreads), lds,
-                           s, segs, nseg, logN, logR, lognb, logP, tab, p);
-        err = hipGetLastError();
-    }
+    hipError_t err = dispatch_inv<W, Wout>(logM, log_e, SegList<InvSeg<W, Wout>>{segs, nseg, {}}, blocks,
+                                           logR, logP, tab_for_sub(tab, logN, logM), p, s);
     if (err != hipSuccess || logR == 0 || mblocks <= 0)
         return err;
     hipLaunchKernelGGL((ntt_merge_segs<W, Wout>), dim3((unsigned)mblocks), dim3(kThreads), 0, s,
@@ -1887,13 +1658,11 @@ template hipError_t launch_ntt_inv_segs<uint32_t, uint64_t>(const InvSeg<uint32_
                                                             const NttTab<uint32_t> &, uint32_t,
                                                             hipStream_t, bool);
 
-template hipError_t launch_ntt_fwd<uint64_t, uint64_t>(const uint64_t *, int64_t, int64_t,
-                                                       uint64_t *, int64_t, int, int,
+template hipError_t launch_ntt_fwd<uint64_t, uint64_t>(const FwdOp<uint64_t, uint64_t> *, int, int, int,
                                                        const NttTune &, const NttTab<uint64_t> &,
                                                        uint64_t, hipStream_t, uint64_t *,
                                                        const ColTab<uint64_t> *, bool);
-template hipError_t launch_ntt_fwd<uint64_t, uint32_t>(const uint64_t *, int64_t, int64_t,
-                                                       uint32_t *, int64_t, int, int,
+template hipError_t launch_ntt_fwd<uint64_t, uint32_t>(const FwdOp<uint64_t, uint32_t> *, int, int, int,
                                                        const NttTune &, const NttTab<uint32_t> &,
                                                        uint32_t, hipStream_t, uint64_t *,
                                                        const ColTab<uint32_t> *, bool);

@@ -562,9 +562,12 @@ pw_mfma_segs(const PwSeg<W> *__restrict__ segs, int nseg, int64_t blocks, ModCon
             continue;
         const PwSeg<W> &sg = pw_seg_of(segs, nseg, b);
         ModConst mcs = mc;
-        mcs.redc_small = sg.redc_small;
-        mfma_wave<W, PT>(sg.Ah, sg.Bh, sg.Ch, sg.m, sg.k, sg.n, sg.N, sg.logP, sg.logPc, mcs,
-                         (b - sg.block0) * kWaves + wave);
+        mcs.redc_small = __builtin_amdgcn_readfirstlane(sg.redc_small);
+        mfma_wave<W, PT>(as_global(sg.Ah), as_global(sg.Bh), as_global(sg.Ch),
+                         __builtin_amdgcn_readfirstlane(sg.m), __builtin_amdgcn_readfirstlane(sg.k),
+                         __builtin_amdgcn_readfirstlane(sg.n), uniform(sg.N),
+                         __builtin_amdgcn_readfirstlane(sg.logP), __builtin_amdgcn_readfirstlane(sg.logPc),
+                         mcs, (b - uniform(sg.block0)) * kWaves + wave);
     }
 }
 
@@ -580,7 +583,8 @@ pw_plain_segs(const PwSeg<W> *__restrict__ segs, int nseg, int64_t blocks, ModCo
         const int64_t by = lb / gx;
         const int64_t q = (lb - by * gx) * 64 + (threadIdx.x & 63);
         const int tile = (int)by * kWaves + (threadIdx.x >> 6);
-        plain_body<W>(sg.Ah, sg.Bh, sg.Ch, sg.m, sg.k, sg.n, sg.N, sg.logP, sg.logPc, mc, q, tile);
+        plain_body<W>(as_global(sg.Ah), as_global(sg.Bh), as_global(sg.Ch), sg.m, sg.k, sg.n, sg.N, sg.logP,
+                      sg.logPc, mc, q, tile);
     }
 }
 
