@@ -20,9 +20,12 @@
 //     shift[piv[r]] += 1 (r < rank), row piv[rank+t] += sum_r X[t][r] row piv[r],
 //     rows piv[r] multiplied by x (length grows when one of them reaches the top).
 //
-// Kernel 1 (one workgroup) does 2-4 and writes the step's description;
-// kernel 2 (a grid) applies the row operations to appbas and R, reading one
-// buffer and writing the other.  All control (nullity cases, basis length)
+// Kernel 1 (one workgroup) does 2-4 for a window of consecutive orders: it
+// holds the window's residual coefficients in LDS, updates them itself after
+// each order, and writes every order's description; kernel 2 (a grid) then
+// applies the window's row operations, one after the other, to tiles of
+// appbas and of the rest of R held in LDS, reading one buffer and writing the
+// other.  All control (nullity cases, basis length)
 // stays on the device: a leaf is a fixed sequence of launches.  The steps
 // skip the division by the pivots in 3: with D the product of the pivots,
 // they apply D X and multiply the updated rows by D, so each basis row is the
@@ -48,35 +51,63 @@ constexpr int kStepThreads = 1024;
 constexpr int kMaxM = 256;    // rows of F (basis dimension) in the device M-Basis step
 constexpr int kMaxN = 128;    // columns of F: at most two rows of the transposed residual per lane
 constexpr int kPanel = 4;     // widest Gauss-Jordan panel (LDS is sized for it)
-// dynamic LDS of the step kernel, set once for every instance: the value the
-// 128 x 128 shape needs, which every allowed shape must fit
+constexpr int kWindow = 4;    // most orders one launch of the step kernel takes
+constexpr int kTile = 16;     // coefficients of a tile of the update kernel, its w leading ones a halo
+// Shapes accepted: the transposed residual and the panel buffers within what
+// the 128 x 128 shape needs with 64-bit words
 constexpr size_t kStepLdsMax = 147968;
+constexpr size_t kLds = 159 * 1024;  // dynamic LDS of one workgroup (its static LDS is below 1 KiB)
 
-// LDS bytes of the step kernel for an m x n residual with words of wbytes:
-// shifts (m 64-bit words), At (n rows of odd stride m | 1), the pivot
-// cofactors (kMaxN), two coefficient buffers (kMaxN x (kPanel + 1) each),
-// then the int arrays (4 of m, 3 of kMaxN); as laid out in the kernel
+// LDS bytes that decide whether an m x n residual with words of wbytes is
+// accepted: shifts (m 64-bit words), At (n rows of odd stride m | 1), the
+// pivot cofactors (kMaxN), two coefficient buffers (kMaxN x (kPanel + 1) each),
+// then the int arrays (4 of m, 3 of kMaxN)
 __host__ __device__ inline size_t step_lds_bytes(int m, int n, size_t wbytes)
 {
     return (size_t)m * 8 +
            ((size_t)n * (m | 1) + kMaxN + 2 * (size_t)kMaxN * (kPanel + 1)) * wbytes +
            (4 * (size_t)m + 3 * (size_t)kMaxN) * sizeof(int);
 }
+// LDS bytes of the step kernel with a window of w orders: the above, the row
+// scales and delays, and for w > 1 the window's residual coefficients
+__host__ __device__ inline size_t window_lds_bytes(int m, int n, int w, size_t wbytes)
+{
+    return step_lds_bytes(m, n, wbytes) + (size_t)m * (wbytes + sizeof(int)) +
+           (w > 1 ? (size_t)m * n * w * wbytes : 0);
+}
+// Orders per window: what fits LDS.  A longer window spares launches (the step
+// and update kernels' start-up, loads and stores: about 10 us together) and
+// lengthens the step kernel's own update of the window's remaining
+// coefficients, which one workgroup does alone.  Windows of 3 and 4 orders, step
+// plus update per order: 20.9 and 20.5 us (64 x 32, 32-bit words), 14.8 and 14.7
+// us (32 x 17, 64-bit words).
+inline int window_orders(int m, int n, size_t wbytes)
+{
+    int w = kWindow;
+    while (w > 1 && window_lds_bytes(m, n, w, wbytes) > kLds)
+        --w;
+    return w;
+}
+// LDS bytes of the update kernel but the staged vectors: the tile, the
+// window's row lists, the delays and a word per wave
+__host__ __device__ inline size_t update_lds_bytes(int m, size_t wbytes)
+{
+    return ((size_t)m * kTile * wbytes + ((size_t)m * (kWindow + 1) + 8) * sizeof(int) + 15) & ~(size_t)15;
+}
 constexpr int kXPad = 32;     // words after X read (and discarded) by the last update group
 
 // control words of one leaf
 enum Ctl {
     C_CUR = 0,    // index (0/1) of the buffers holding the current appbas and R
-    C_MODE = 1,   // what kernel 2 does at this step: 0 nothing, 1 update, 2 shift all
-    C_RANK = 2,   // rank of the residual at this step
-    C_LEN = 3,    // current length of appbas
-    C_GROW = 4,   // set by kernel 2 when the length grows by one
-    C_DONE = 5,   // full-rank residual met: the leaf is finished
-    C_SHIFT = 6,  // mode 2: power of x
-    C_LOLD = 7,   // mode 2: length before the shift
-    C_FLIP = 8,   // kernel 2 wrote the other buffers: swap before the next step
+    C_STEPS = 1,  // orders of this window that kernel 2 applies
+    C_LEN = 2,    // length of appbas at the window's start
+    C_DONE = 4,   // full-rank residual met: the leaf is finished
+    C_SHIFT = 5,  // then: power of x that appbas is still to be multiplied by
+    C_FLIP = 6,   // kernel 2 wrote the other buffers: swap before the next window
+    C_RANK = 8,   // rank of the residual at each order of the window (0: nothing to do)
     C_WORDS = 16
 };
+static_assert(C_RANK + kWindow <= C_WORDS, "a rank per order of the window");
 
 struct LeafArgs {
     int m, n;
@@ -84,18 +115,21 @@ struct LeafArgs {
     int cap;      // coefficient capacity of appbas (ordL + 1)
     uint64_t *app[2];  // m x m x cap, entry-major
     uint64_t *R[2];    // m x n x ordL, entry-major
-    uint64_t *Rn;      // m x n: the coming step's residual coefficient
+    uint64_t *Rn;      // the coming window's residual coefficients: m x n each, one after the other
     // Row scales.  The steps use unnormalised kernel vectors (own coefficient
     // D, the product of the step's pivots, instead of 1), so basis row i is
     // scale[i] times the normalised one; the leaf divides them out at its
-    // end.  scale[m] holds the current step's D for the update (plain residue
-    // for 64-bit words, Montgomery residue D 2^32 mod p for 32-bit ones).
-    uint64_t *scale;   // m + 1 words
-    uint64_t *X;       // nullity x rank, row stride m
-    int *piv;          // m
-    int *rowinfo;      // m: t >= 0 nullity row t, -1-r rank row r
+    // end.  scale[m + s] holds D of the window's order s (in the step
+    // kernel's arithmetic, as X).
+    uint64_t *scale;   // m + kWindow words
+    uint64_t *X;       // per order of the window: nullity x rank, row stride m, words of the arithmetic
+    int *piv;          // per order of the window: m
     int64_t *shift;    // m
     int *ctl;          // C_WORDS
+    // lengths that kernel 2's workgroups have seen appbas reach, two words per
+    // column (tiles of even and odd number): one word that all of them raised
+    // by atomics took 3 us of a window's update
+    int *lens;
     ModConst mc;
 };
 
@@ -195,8 +229,8 @@ struct Mont64Arith {
         mul128(a, b, hi, lo);
         return redc(hi, lo);
     }
-    // Sums of up to five products, reduced once: t < 5 p^2 < 2^64 p, so the
-    // REDC quotient is below (5p / 2^64 + 1) p < 2.25 p.
+    // Sums of up to eight products, reduced once: t < 8 p^2 <= 2^127, and the
+    // REDC quotient is below (8p / 2^64 + 1) p < 3p < 2^64.
     struct Acc {
         uint64_t hi, lo;
     };
@@ -244,6 +278,8 @@ struct Mont64Arith {
         }
     }
     __device__ V sub(V a, V b) const { return a >= b ? a - b : a + (p - b); }
+    // a factor of a lazy sum: -a as p - a (p itself for a = 0)
+    __device__ V neg(V a) const { return p - a; }
     __device__ V add(V a, V b) const
     {
         const uint64_t t = a + b;  // < 2p < 2^63
@@ -272,8 +308,8 @@ struct Mont32Arith {
         return v < u ? v : u;
     }
     __device__ V mul(V a, V b) const { return redc((uint64_t)a * b); }
-    // Sums of up to five products, reduced once: t < 5 p^2 < 5 2^60, t + mm p
-    // < 9 2^60 < 2^64 and the quotient is below (5p / 2^32 + 1) p < 2.25 p.
+    // Sums of up to eight products, reduced once: t < 8 p^2 < 2^63, t + mm p
+    // < 2^63 + 2^62 and the quotient is below (8p / 2^32 + 1) p < 3p < 2^32.
     using Acc = uint64_t;
     __device__ Acc prod(V a, V b) const { return (uint64_t)a * b; }
     __device__ Acc fma(Acc t, V a, V b) const { return t + (uint64_t)a * b; }
@@ -311,6 +347,8 @@ struct Mont32Arith {
             out[i] = v < u ? v : u;
         }
     }
+    // a factor of a lazy sum: -a as p - a (p itself for a = 0)
+    __device__ V neg(V a) const { return p - a; }
     __device__ V sub(V a, V b) const
     {
         // a - b, plus p when it wraps: min(d, d + p) as unsigned words
@@ -369,6 +407,7 @@ struct BigArith {
             out[i] = msub(pv, x[i], fr, q[i]);
     }
     __device__ V sub(V a, V b) const { return a >= b ? a - b : a + (mc.p - b); }
+    __device__ V neg(V a) const { return sub(0, a); }
     __device__ V add(V a, V b) const { return addmod_any(a, b, mc.p); }
     __device__ V one() const { return 1; }
     __device__ V to(uint64_t x) const { return x; }
@@ -411,8 +450,8 @@ __device__ __forceinline__ uint64_t lane_value(uint64_t v, int l)
 // kernel 1: permutation, left nullspace, step description
 // ---------------------------------------------------------------------------
 // Fraction-free Gauss-Jordan on At = (permuted residual)^T (n x m): pivot rows
-// stay where they are (prow[k] is the row of the k-th pivot, pivcol[k] its
-// column); for a pivot at (pr, c) every other row r becomes
+// stay where they are (prow[k] is the row of the k-th pivot); for a pivot at
+// (pr, c) every other row r becomes
 // pv * row_r - At[r][c] * row_pr with pv = At[pr][c].  The k-th row of the
 // reduced row echelon form is row prow[k] divided by its pivot; the step
 // multiplies by the other pivots' product (the pivot's cofactor) instead, so
@@ -425,8 +464,24 @@ __device__ __forceinline__ uint64_t lane_value(uint64_t v, int l)
 // residues as the one-column-at-a-time sequence.  The waves then apply that
 // combination to their own columns while the next panel is composed: one
 // barrier per panel instead of one per column.
+//
+// One launch takes the w orders ord0 .. ord0 + w - 1.  The residual's
+// coefficients of the window sit in LDS (Rw, slot d of row i its coefficient
+// ord0 + d + delay[i]: multiplying a row by x only raises its delay), and after
+// each order the kernel rows' coefficients of the orders still to come are
+// combined here, so that a window costs one launch of each kernel.  With
+// w = 1 the residual coefficient goes straight from global memory to At.
+//
+// One workgroup and a chain of n pivots: latency bounds it, not throughput.  Of
+// the 16.5 us that an order takes (64 x 32, 32-bit words, clock stamps) the
+// elimination has 9.0, 8 panels of 0.57 (composition) + 0.42 (apply) + 0.06
+// (barrier) each, the window's update 0 to 6.7 with the orders still to come
+// (3.5 on average), the sort 0.8, the rest 2.2.  Step plus update kernel per
+// order, with one order per launch and panels composed pivot by pivot / as it
+// is: 17.7 + 9.5 / 15.9 + 4.2 us (64 x 32, 32-bit), 13.5 + 6.8 / 11.0 + 3.6 us
+// (32 x 17, 64-bit).
 template <typename Arith, int H>
-__global__ void __launch_bounds__(kStepThreads) mbasis_step_kernel(LeafArgs a, int ord)
+__global__ void __launch_bounds__(kStepThreads) mbasis_step_kernel(LeafArgs a, int ord0, int w)
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     using V = typename Arith::V;
@@ -439,755 +494,1172 @@ __global__ void __launch_bounds__(kStepThreads) mbasis_step_kernel(LeafArgs a, i
     const int m = a.m, n = a.n;
     const Arith ar(a.mc);
     const int ms = m | 1;                   // odd row stride of At
-    // 64-bit words first (sh), then the V arrays, then the int arrays
-    // (layout and sizes as step_lds_bytes, whose Ck is sized for kPanel)
-    int64_t *sh = reinterpret_cast<int64_t *>(smem);                 // m
+    const int mn = m * n;
+    // the composed panels' rows (16-byte aligned), 64-bit words (sh), then the
+    // V arrays, then the int arrays (sizes as in window_lds_bytes, whose
+    // coefficient buffers are sized for kPanel)
+    struct alignas(16) Row {
+        V v[P];
+    };
+    Row *Ck = reinterpret_cast<Row *>(smem);                         // 2 x kMaxN: slots 1 .. P
+    V *C0 = reinterpret_cast<V *>(Ck + 2 * kMaxN);                   // 2 x kMaxN: slot 0
+    int64_t *sh = reinterpret_cast<int64_t *>(C0 + 2 * kMaxN);       // m
     V *At = reinterpret_cast<V *>(sh + m);                           // n x ms
     V *cof = At + n * ms;                                            // kMaxN: pivot cofactors
-    V *Ck = cof + kMaxN;                                             // 2 x kMaxN x (P + 1)
-    int *perm = reinterpret_cast<int *>(Ck + 2 * kMaxN * (kPanel + 1));  // m
+    V *scl = cof + kMaxN;                                            // m: row scales
+    V *Rw = scl + m;                                                 // w x m x n (w > 1)
+    int *perm = reinterpret_cast<int *>(Rw + (w > 1 ? w * mn : 0));  // m
     int *plist = perm + m;                                           // m
     int *colpiv = plist + m;                                         // m (columns of At)
     int *pos = colpiv + m;                                           // m (then: pivot row by column)
-    int *pivcol = pos + m;                                           // kMaxN (by rank)
-    int *prow = pivcol + kMaxN;                                      // kMaxN (by rank)
+    int *delay = pos + m;                                            // m
+    int *prow = delay + m;                                           // kMaxN (by rank)
     int *ispiv = prow + kMaxN;                                       // kMaxN (rows of At)
-    __shared__ int s_nb[2], s_prs[2][kPanel];
+    // a composed panel: which columns took a pivot (and kFastPanel), the pivots'
+    // rows, the panel's own coefficient K0 and what its pivots' cofactors have
+    // from it (by pairs: 1 for the first two, D1 for the others)
+    constexpr int kFastPanel = 1 << P;
+    __shared__ int s_tk[2], s_prs[2][kPanel];
+    __shared__ V s_K0[2], s_pre[2][kPanel];
+    __shared__ V s_D;  // the step's D
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const uint64_t p = a.mc.p;
+    const int wave = tid >> 6;
 
-    // Shifts, control words and this step's residual coefficient.  The
-    // coefficient sits in the fixed buffer Rn (m x n, row-major), written by
-    // the previous update or the leaf's initialisation, so its loads wait for
-    // no control word and are contiguous across the workgroup; the shifts are
-    // stored to LDS before those loads are issued (a wait on a vector load
-    // also waits on those issued before it).  Thread 0 writes the control
-    // words back only after full barriers.
-    const int64_t shv = tid < m ? a.shift[tid] : 0;  // m <= kMaxM <= kStepThreads
+    // Shifts, row scales, control words and the window's residual
+    // coefficients (contiguous in the fixed buffer Rn, written by the previous
+    // update or the leaf's initialisation: their loads wait for no control
+    // word).  Thread 0 writes the control words back at the end.
     int *c = a.ctl;
     const int flip = c[C_FLIP], cur0 = c[C_CUR], done = c[C_DONE];
-    if (tid < m) {
-        sh[tid] = shv;
-        pos[tid] = 0;
-        colpiv[tid] = 0;
+    if (wave == kStepThreads / 64 - 1) {
+        int len = 1;
+        for (int i = lane; i < 2 * m; i += 64)
+            len = max(len, a.lens[i]);
+        for (int d = 32; d > 0; d >>= 1)
+            len = max(len, __shfl_xor(len, d));
+        if (lane == 0)
+            c[C_LEN] = len;
+    }
+    if (tid < m) {  // m <= kMaxM <= kStepThreads
+        sh[tid] = a.shift[tid];
+        scl[tid] = ord0 == 0 ? ar.one() : (V)a.scale[tid];
+        delay[tid] = 0;
     }
     const int cur = flip ? cur0 ^ 1 : cur0;
-    // element q = tid + k kStepThreads of the coefficient (row q / n of the
-    // unpermuted residual, column q % n), stored to At[q % n][pos[q / n]] once
-    // the permutation is known; the first kPre per thread are loaded before
-    // the sort (indices past m n clamped, their values unused)
-    const int mn = m * n;
-    constexpr int kPre = 4;
-    V pre[kPre];
-#pragma unroll
-    for (int k = 0; k < kPre; ++k) {
-        const int q = tid + k * kStepThreads;
-        pre[k] = Arith::load(a.Rn + (q < mn ? q : mn - 1));
-    }
-    for (int r = tid; r < kMaxN; r += kStepThreads)
-        ispiv[r] = 0;
     if (done) {
-        __syncthreads();
         if (tid == 0) {
-            const int len = c[C_LEN] + c[C_GROW];
             c[C_CUR] = cur;
             c[C_FLIP] = 0;
-            c[C_LEN] = len;
-            c[C_GROW] = 0;
-            c[C_MODE] = 0;
+            c[C_STEPS] = 0;
         }
         return;
     }
-    lds_barrier();
+    if (w > 1)
+        for (int q = tid; q < w * mn; q += kStepThreads)
+            Rw[q] = ar.to(Arith::load(a.Rn + q));
+    // threads per row of the shift sort
+    const int sortLog = m <= 64 ? 4 : m <= 128 ? 3 : 2;
+    bool full = false;  // full-rank residual met (uniform)
+    int steps = 0;
+    for (int s = 0; s < w && !full; ++s) {
+        if (tid < m)
+            colpiv[tid] = 0;
+        if (tid < kMaxN)
+            ispiv[tid] = 0;
+        lds_barrier();
 
-    // stable permutation sorting (shift, index): pos[i] = #{j : (sh_j, j) < (sh_i, i)}
-    for (int idx = tid; idx < m * m; idx += kStepThreads) {
-        const int j = idx / m, i = idx - j * m;  // neighbouring lanes update different counters
-        const int64_t si = sh[i], sj = sh[j];
-        if ((sj < si) || (sj == si && j < i))
-            atomicAdd(&pos[i], 1);
-    }
-    lds_barrier();
-    for (int i = tid; i < m; i += kStepThreads)
-        perm[pos[i]] = i;
-#pragma unroll
-    for (int k = 0; k < kPre; ++k) {
-        const int q = tid + k * kStepThreads;
-        if (q < mn) {
-            const int i = q / n, j = q - i * n;
-            At[j * ms + pos[i]] = ar.to(pre[k]);
-        }
-    }
-    for (int q = tid + kPre * kStepThreads; q < mn; q += kStepThreads) {
-        const int i = q / n, j = q - i * n;
-        At[j * ms + pos[i]] = ar.to(Arith::load(a.Rn + q));
-    }
-    __syncthreads();
-
-    // Gauss-Jordan by panels of P columns.  Wave w owns the columns
-    // [w cw, (w + 1) cw) of At and applies every panel's combination to them;
-    // the owner of the next panel then composes it from its own updated
-    // columns (the LDS operations of one wave take effect in program order)
-    // while the other waves are still applying: one barrier per panel, with
-    // the coefficients double-buffered.
-    int rank = 0;
-    const int wave = tid >> 6;
-    // columns per wave: P times a power of two (so that cw divides the
-    // wave's 64 lanes), 16 waves covering m
-    int cw = P;
-    while (16 * cw < m)
-        cw *= 2;
-    // compose the panel of columns c0 .. c0 + P - 1 into buffer buf (the
-    // lambdas are forced inline: called from two places, compose was left as
-    // a call in the two-row kernels, its captures and arrays on the stack)
-    auto compose = [&](const int c0, const int buf) __attribute__((always_inline)) {
-        __builtin_amdgcn_s_setprio(2);
+        // stable permutation sorting (shift, index): pos[i] = #{j : (sh_j, j) < (sh_i, i)},
+        // counted by 2^sortLog neighbouring threads per row
         {
-            // rows lane + 64 h (h < H) of the panel, their pivot flags and the
-            // coefficients C[.][0..P] of the composition
-            V pn[H][P], cc[H][P + 1];
-            bool isp[H], ok[H];
-            int prs[P] = {0};
-            int tk = 0;  // panel columns that took a pivot
-#pragma unroll
-            for (int h = 0; h < H; ++h) {
-                const int r = lane + 64 * h;
-                ok[h] = r < n;
-                isp[h] = ok[h] && ispiv[r];
-#pragma unroll
-                for (int j = 0; j < P; ++j)
-                    pn[h][j] = ok[h] && c0 + j < m ? At[r * ms + c0 + j] : (V)0;
-                cc[h][0] = ar.one();
-#pragma unroll
-                for (int s2 = 1; s2 <= P; ++s2)
-                    cc[h][s2] = 0;
+            const int i = tid >> sortLog, g = tid & ((1 << sortLog) - 1);
+            if (i < m) {
+                const int64_t si = sh[i];
+                int cnt = 0;
+                for (int j = g; j < m; j += 1 << sortLog) {
+                    const int64_t sj = sh[j];
+                    cnt += (sj < si) || (sj == si && j < i) ? 1 : 0;
+                }
+                for (int d = 1; d < 1 << sortLog; d <<= 1)
+                    cnt += __shfl_xor(cnt, d);
+                if (g == 0) {
+                    pos[i] = cnt;
+                    perm[cnt] = i;
+                }
             }
-            int nb = 0;
-            // one pivot step on panel column j (a compile-time index: the
-            // convergent ballots and lane reads keep the compiler from unrolling
-            // a loop around them, and the arrays must stay in registers)
-            auto step = [&](auto jc) __attribute__((always_inline)) {
-                constexpr int j = decltype(jc)::value;
-                // columns past m, or a full rank already reached, take no pivot
-                const bool open = c0 + j < m && rank + nb < n;
-                const unsigned long long b0 = __ballot(open && ok[0] && !isp[0] && pn[0][j] != 0);
-                const unsigned long long b1 =
-                    H == 2 ? __ballot(open && ok[H - 1] && !isp[H - 1] && pn[H - 1][j] != 0) : 0ull;
-                if (!b0 && !b1)
-                    return;  // no pivot in this column
-                const int pr = b0 ? __ffsll(b0) - 1 : 63 + __ffsll(b1);
-                const int pl = pr & 63, ph = pr >> 6;
-                // broadcast the pivot row (panel values and coefficients): the
-                // pivot lane is uniform, so its registers are read into
-                // scalar registers; its self coefficient cc[0] moves to slot
-                // j + 1
-                V qp[P], qc[P + 1];
-#pragma unroll
-                for (int jj = j; jj < P; ++jj)
-                    qp[jj] = lane_value(H == 2 && ph ? pn[H - 1][jj] : pn[0][jj], pl);
-#pragma unroll
-                for (int s2 = 1; s2 <= j; ++s2)
-                    qc[s2] = lane_value(H == 2 && ph ? cc[H - 1][s2] : cc[0][s2], pl);
-                qc[j + 1] = lane_value(H == 2 && ph ? cc[H - 1][0] : cc[0][0], pl);
-                const V pv = qp[j];
-                // Only the nonzero terms are formed: column j of every other
-                // row becomes pv * fr - fr * pv = 0, and slots past j are zero
-                // in every row until this step, so slot j + 1 is -fr * qc.
-                // Every lane computes and the pivot lane keeps its own values
-                // (selects, not branches, so the step stays one basic block);
-                // rows past n hold zeros and are never published.
+        }
+        lds_barrier();
+        // the residual coefficient of this order, transposed and permuted: one
+        // row of the residual per wave, two where they have at most 32 columns
+        for (int i = n <= 32 ? tid >> 5 : wave; i < m; i += kStepThreads / (n <= 32 ? 32 : 64)) {
+            const int pi = pos[i];
+            const size_t slot = w > 1 ? (size_t)(s - delay[i]) * mn : 0;
+            for (int j = n <= 32 ? tid & 31 : lane; j < n; j += 64)
+                At[j * ms + pi] = w > 1 ? Rw[slot + i * n + j] : ar.to(Arith::load(a.Rn + i * n + j));
+        }
+        lds_barrier();
+
+        // Gauss-Jordan by panels of P columns.  Wave w owns the columns
+        // [w cw, (w + 1) cw) of At and applies every panel's combination to them;
+        // the owner of the next panel then composes it from its own updated
+        // columns (the LDS operations of one wave take effect in program order)
+        // while the other waves are still applying: one barrier per panel, with
+        // the coefficients double-buffered.
+        int rank = 0;
+        // columns per wave: P times a power of two (so that cw divides the
+        // wave's 64 lanes), 16 waves covering m
+        int cw = P;
+        while (16 * cw < m)
+            cw *= 2;
+        // compose the panel of columns c0 .. c0 + P - 1 into buffer buf (the
+        // lambdas are forced inline: called from two places, compose was left as
+        // a call in the two-row kernels, its captures and arrays on the stack)
+        auto compose = [&](const int c0, const int buf) __attribute__((always_inline)) {
+            __builtin_amdgcn_s_setprio(2);
+            {
+                // rows lane + 64 h (h < H) of the panel, their pivot flags and the
+                // coefficients C[.][0..P] of the composition
+                V pn[H][P], cc[H][P + 1];
+                bool isp[H], ok[H];
+                int prs[P] = {0};
+                V pre[P], prod = ar.one();  // product of the panel's earlier pivots
+                int tk = 0;  // panel columns that took a pivot
 #pragma unroll
                 for (int h = 0; h < H; ++h) {
-                    const bool me = lane + 64 * h == pr;
-                    const V fr = pn[h][j];
-                    // the P products of this step: panel columns j + 1 .. P - 1,
-                    // slots 1 .. j, and slot j + 1 (from zero)
-                    V xs[P], qs[P], ts[P];
+                    const int r = lane + 64 * h;
+                    ok[h] = r < n;
+                    isp[h] = ok[h] && ispiv[r];
 #pragma unroll
-                    for (int jj = j + 1; jj < P; ++jj) {
-                        xs[jj - j - 1] = pn[h][jj];
-                        qs[jj - j - 1] = qp[jj];
-                    }
+                    for (int j = 0; j < P; ++j)
+                        pn[h][j] = ok[h] && c0 + j < m ? At[r * ms + c0 + j] : (V)0;
+                    cc[h][0] = ar.one();
 #pragma unroll
-                    for (int s2 = 1; s2 <= j; ++s2) {
-                        xs[P - j - 2 + s2] = cc[h][s2];
-                        qs[P - j - 2 + s2] = qc[s2];
-                    }
-                    xs[P - 1] = 0;
-                    qs[P - 1] = qc[j + 1];
-                    ar.msub_n(pv, xs, fr, qs, ts);
+                    for (int s2 = 1; s2 <= P; ++s2)
+                        cc[h][s2] = 0;
+                }
+                int nb = 0;
+                // one pivot step on panel column j (a compile-time index: the
+                // convergent ballots and lane reads keep the compiler from unrolling
+                // a loop around them, and the arrays must stay in registers)
+                auto step = [&](auto jc) __attribute__((always_inline)) {
+                    constexpr int j = decltype(jc)::value;
+                    // columns past m, or a full rank already reached, take no pivot
+                    const bool open = c0 + j < m && rank + nb < n;
+                    const unsigned long long b0 = __ballot(open && ok[0] && !isp[0] && pn[0][j] != 0);
+                    const unsigned long long b1 =
+                        H == 2 ? __ballot(open && ok[H - 1] && !isp[H - 1] && pn[H - 1][j] != 0) : 0ull;
+                    if (!b0 && !b1)
+                        return;  // no pivot in this column
+                    const int pr = b0 ? __ffsll(b0) - 1 : 63 + __ffsll(b1);
+                    const int pl = pr & 63, ph = pr >> 6;
+                    // broadcast the pivot row (panel values and coefficients): the
+                    // pivot lane is uniform, so its registers are read into
+                    // scalar registers; its self coefficient cc[0] moves to slot
+                    // j + 1
+                    V qp[P], qc[P + 1];
 #pragma unroll
-                    for (int jj = j + 1; jj < P; ++jj)
-                        pn[h][jj] = me ? pn[h][jj] : ts[jj - j - 1];
-                    pn[h][j] = me ? fr : (V)0;
+                    for (int jj = j; jj < P; ++jj)
+                        qp[jj] = lane_value(H == 2 && ph ? pn[H - 1][jj] : pn[0][jj], pl);
 #pragma unroll
                     for (int s2 = 1; s2 <= j; ++s2)
-                        cc[h][s2] = me ? cc[h][s2] : ts[P - j - 2 + s2];
-                    cc[h][j + 1] = me ? qc[j + 1] : ts[P - 1];
-                    const V t0 = ar.mul(pv, cc[h][0]);
-                    cc[h][0] = me ? (V)0 : t0;
-                    isp[h] = isp[h] || me;
+                        qc[s2] = lane_value(H == 2 && ph ? cc[H - 1][s2] : cc[0][s2], pl);
+                    qc[j + 1] = lane_value(H == 2 && ph ? cc[H - 1][0] : cc[0][0], pl);
+                    const V pv = qp[j];
+                    // Only the nonzero terms are formed: column j of every other
+                    // row becomes pv * fr - fr * pv = 0, and slots past j are zero
+                    // in every row until this step, so slot j + 1 is -fr * qc.
+                    // Every lane computes and the pivot lane keeps its own values
+                    // (selects, not branches, so the step stays one basic block);
+                    // rows past n hold zeros and are never published.
+#pragma unroll
+                    for (int h = 0; h < H; ++h) {
+                        const bool me = lane + 64 * h == pr;
+                        const V fr = pn[h][j];
+                        // the P products of this step: panel columns j + 1 .. P - 1,
+                        // slots 1 .. j, and slot j + 1 (from zero)
+                        V xs[P], qs[P], ts[P];
+#pragma unroll
+                        for (int jj = j + 1; jj < P; ++jj) {
+                            xs[jj - j - 1] = pn[h][jj];
+                            qs[jj - j - 1] = qp[jj];
+                        }
+#pragma unroll
+                        for (int s2 = 1; s2 <= j; ++s2) {
+                            xs[P - j - 2 + s2] = cc[h][s2];
+                            qs[P - j - 2 + s2] = qc[s2];
+                        }
+                        xs[P - 1] = 0;
+                        qs[P - 1] = qc[j + 1];
+                        ar.msub_n(pv, xs, fr, qs, ts);
+#pragma unroll
+                        for (int jj = j + 1; jj < P; ++jj)
+                            pn[h][jj] = me ? pn[h][jj] : ts[jj - j - 1];
+                        pn[h][j] = me ? fr : (V)0;
+#pragma unroll
+                        for (int s2 = 1; s2 <= j; ++s2)
+                            cc[h][s2] = me ? cc[h][s2] : ts[P - j - 2 + s2];
+                        cc[h][j + 1] = me ? qc[j + 1] : ts[P - 1];
+                        const V t0 = ar.mul(pv, cc[h][0]);
+                        cc[h][0] = me ? (V)0 : t0;
+                        isp[h] = isp[h] || me;
+                    }
+                    prs[j] = pr;
+                    pre[j] = prod;
+                    prod = ar.mul(prod, pv);
+                    tk |= 1 << j;
+                    ++nb;
+                };
+                static_assert(P >= 1 && P <= 4, "the panel steps below are written out for up to 4 columns");
+                step(std::integral_constant<int, 0>{});
+                if constexpr (P > 1)
+                    step(std::integral_constant<int, 1>{});
+                if constexpr (P > 2)
+                    step(std::integral_constant<int, 2>{});
+                if constexpr (P > 3)
+                    step(std::integral_constant<int, 3>{});
+                // publish: coefficients, pivot flags, pivot rows
+#pragma unroll
+                for (int h = 0; h < H; ++h) {
+                    const int r = lane + 64 * h;
+                    if (ok[h]) {
+                        C0[buf * kMaxN + r] = cc[h][0];
+#pragma unroll
+                        for (int s2 = 1; s2 <= P; ++s2)
+                            Ck[buf * kMaxN + r].v[s2 - 1] = cc[h][s2];
+                        ispiv[r] = isp[h] ? 1 : 0;
+                    }
                 }
-                prs[j] = pr;
-                tk |= 1 << j;
-                ++nb;
-            };
-            static_assert(P >= 1 && P <= 4, "the panel steps below are written out for up to 4 columns");
-            step(std::integral_constant<int, 0>{});
-            if constexpr (P > 1)
+                if (lane == 0) {
+                    s_tk[buf] = tk;
+                    s_K0[buf] = prod;
+#pragma unroll
+                    for (int k = 0; k < P; ++k) {
+                        s_prs[buf][k] = prs[k];
+                        if (tk >> k & 1)
+                            s_pre[buf][k] = pre[k];
+                    }
+                }
+            }
+            __builtin_amdgcn_s_setprio(0);
+        };
+        // Residuals of at most 32 columns (n <= 32 rows of At) leave the upper
+        // half of the composing wave idle in compose().  compose_half() puts the
+        // coefficient slots there: upper lane 32 + r holds slots 0, 1, 2 of row r
+        // (slots 0, 1 for P = 2) and lower lane r the row's panel values and the
+        // last slots, in registers whose lower halves pass from a panel column to
+        // a slot once that column is eliminated.  Each instruction then advances
+        // a panel value and a coefficient at once: three multiply-subtracts per
+        // pivot step instead of five (two instead of three for P = 2).
+        //   P = 4, registers Z A B C: lower lane r holds row r in panel columns
+        //   0..3, A becomes slot 3 before step 2 and B slot 4 before step 3;
+        //   upper lane 32 + r holds slots 0, 1, 2 in A, B, C.
+        //   P = 2, registers Z A B: lower lane r holds columns 0, 1 in Z, A and
+        //   slot 2 in B; upper lane 32 + r holds slots 0, 1 in A, B.
+        // Slot 0 takes pv * c0 as the multiply-subtract with q = 0 (pv c0 + fr p,
+        // the same residue); a register that starts a slot holds zero, so the
+        // slot's first value is -fr * q as in compose().
+        auto compose_half = [&](const int c0, const int buf) __attribute__((always_inline)) {
+            __builtin_amdgcn_s_setprio(2);
+            {
+                static_assert(P == 2 || P == 4, "compose_half is written out for panels of 2 and 4");
+                const bool hi = lane >= 32;
+                const int r = lane & 31;
+                const bool ok = r < n;
+                auto col = [&](const int j) -> V {
+                    return !hi && ok && c0 + j < m ? At[r * ms + c0 + j] : (V)0;
+                };
+                V Z = col(0);
+                V A = hi ? ar.one() : col(1);
+                V B = P == 4 ? col(2) : (V)0;
+                V C = P == 4 ? col(3) : (V)0;
+                bool isp = !hi && ok && ispiv[r];
+                int prs[P] = {0};
+                V pre[P], prod = ar.one();  // product of the panel's earlier pivots
+                int tk = 0, nb = 0;
+                // every lane gets the value of x in lane (lane & 31)
+                auto low = [](const V x) -> V {
+                    if constexpr (sizeof(V) == 4) {
+                        return __builtin_amdgcn_permlane32_swap(x, x, false, false)[0];
+                    } else {
+                        const uint32_t l = (uint32_t)x, h = (uint32_t)(x >> 32);
+                        const uint32_t l2 = __builtin_amdgcn_permlane32_swap(l, l, false, false)[0];
+                        const uint32_t h2 = __builtin_amdgcn_permlane32_swap(h, h, false, false)[0];
+                        return ((uint64_t)h2 << 32) | l2;
+                    }
+                };
+                auto step = [&](auto jc) __attribute__((always_inline)) {
+                    constexpr int j = decltype(jc)::value;
+                    if constexpr (P == 4 && j == 2)
+                        A = hi ? A : (V)0;  // column 1 is done: lower A is slot 3
+                    if constexpr (P == 4 && j == 3)
+                        B = hi ? B : (V)0;  // column 2 is done: lower B is slot 4
+                    const V xj = j == 0 ? Z : j == 1 ? A : j == 2 ? B : C;
+                    const bool open = c0 + j < m && rank + nb < n;
+                    const unsigned long long b = __ballot(open && !hi && ok && !isp && xj != 0);
+                    if (!b)
+                        return;  // no pivot in this column
+                    const int pr = __ffsll(b) - 1;  // a lower lane
+                    const bool me = r == pr;
+                    const V pv = lane_value(xj, pr);
+                    const V fr = low(xj);
+                    const V Q = lane_value(A, 32 + pr);  // the pivot row's slot 0
+                    constexpr int G = P == 4 ? 3 : 2;
+                    V xs[G], qs[G], ts[G], kp[G];  // operands, and what the pivot row keeps
+                    const V zero = 0;
+                    if constexpr (P == 4) {
+                        xs[0] = A;
+                        xs[1] = B;
+                        xs[2] = C;
+                        if constexpr (j == 0) {
+                            const V p1 = lane_value(A, pr), p2 = lane_value(B, pr), p3 = lane_value(C, pr);
+                            qs[0] = hi ? zero : p1;
+                            qs[1] = hi ? Q : p2;
+                            qs[2] = hi ? zero : p3;
+                            kp[0] = hi ? zero : A;
+                            kp[1] = hi ? Q : B;
+                            kp[2] = C;
+                        } else if constexpr (j == 1) {
+                            const V p2 = lane_value(B, pr), p3 = lane_value(C, pr), q1 = lane_value(B, 32 + pr);
+                            qs[0] = zero;
+                            qs[1] = hi ? q1 : p2;
+                            qs[2] = hi ? Q : p3;
+                            kp[0] = hi ? zero : A;
+                            kp[1] = B;
+                            kp[2] = hi ? Q : C;
+                        } else if constexpr (j == 2) {
+                            const V p3 = lane_value(C, pr), q1 = lane_value(B, 32 + pr), q2 = lane_value(C, 32 + pr);
+                            qs[0] = hi ? zero : Q;
+                            qs[1] = hi ? q1 : zero;
+                            qs[2] = hi ? q2 : p3;
+                            kp[0] = hi ? zero : Q;
+                            kp[1] = B;
+                            kp[2] = C;
+                        } else {
+                            const V q3 = lane_value(A, pr), q1 = lane_value(B, 32 + pr), q2 = lane_value(C, 32 + pr);
+                            qs[0] = hi ? zero : q3;
+                            qs[1] = hi ? q1 : Q;
+                            qs[2] = hi ? q2 : zero;
+                            kp[0] = hi ? zero : A;
+                            kp[1] = hi ? B : Q;
+                            kp[2] = C;
+                        }
+                    } else {
+                        xs[0] = A;
+                        xs[1] = B;
+                        if constexpr (j == 0) {
+                            const V p1 = lane_value(A, pr);
+                            qs[0] = hi ? zero : p1;
+                            qs[1] = hi ? Q : zero;
+                            kp[0] = hi ? zero : A;
+                            kp[1] = hi ? Q : B;
+                        } else {
+                            const V q1 = lane_value(B, 32 + pr);
+                            qs[0] = zero;
+                            qs[1] = hi ? q1 : Q;
+                            kp[0] = hi ? zero : A;
+                            kp[1] = hi ? B : Q;
+                        }
+                    }
+                    ar.msub_n(pv, xs, fr, qs, ts);
+                    A = me ? kp[0] : ts[0];
+                    B = me ? kp[1] : ts[1];
+                    if constexpr (P == 4)
+                        C = me ? kp[2] : ts[2];
+                    isp = isp || me;  // read in the lower half only
+                    prs[j] = pr;
+                    pre[j] = prod;
+                    prod = ar.mul(prod, pv);
+                    tk |= 1 << j;
+                    ++nb;
+                };
+                step(std::integral_constant<int, 0>{});
                 step(std::integral_constant<int, 1>{});
-            if constexpr (P > 2)
-                step(std::integral_constant<int, 2>{});
-            if constexpr (P > 3)
-                step(std::integral_constant<int, 3>{});
-            // publish: coefficients, pivot flags, pivot rows
+                if constexpr (P == 4) {
+                    step(std::integral_constant<int, 2>{});
+                    step(std::integral_constant<int, 3>{});
+                }
+                // publish: coefficients, pivot flags, pivot rows
+                if (ok) {
+                    V *ck = Ck[buf * kMaxN + r].v;
+                    if (hi) {
+                        C0[buf * kMaxN + r] = A;
+                        ck[0] = B;
+                        if constexpr (P == 4)
+                            ck[1] = C;
+                    } else {
+                        if constexpr (P == 4) {
+                            ck[2] = A;
+                            ck[3] = B;
+                        } else {
+                            ck[1] = B;
+                        }
+                        ispiv[r] = isp ? 1 : 0;
+                    }
+                }
+                if (lane == 0) {
+                    s_tk[buf] = tk;
+                    s_K0[buf] = prod;
+#pragma unroll
+                    for (int k = 0; k < P; ++k) {
+                        s_prs[buf][k] = prs[k];
+                        if (tk >> k & 1)
+                            s_pre[buf][k] = pre[k];
+                    }
+                }
+            }
+            __builtin_amdgcn_s_setprio(0);
+        };
+        // While every panel so far went this way, the pivot rows are simply the
+        // rows in order, rank, rank + 1, ..., taken two at a time: for rows s1,
+        // s2 with the block [a b; c d] in columns 1, 2 and D1 = ad - bc, every
+        // row becomes D1 row - C1 row_s1 - C2 row_s2, C1 = v1 d - v2 c, C2 = v2 a - v1 b
+        // (v1, v2 its own values there), and rows s1, s2 their adjugate combinations
+        // d row_s1 - b row_s2 and a row_s2 - c row_s1, as the same expression with
+        // C1 = D1 - d, C2 = b and C1 = c, C2 = D1 - a.  Two such steps make a panel
+        // of four.  Nothing is searched for, so no ballot, bit search and lane read
+        // stands between one pivot and the next, and a panel is 6 dependent
+        // reductions instead of 4 times 2; the two blocks' determinants must be
+        // nonzero, else (false) this panel and the step's later ones are composed
+        // pivot by pivot.  The pivots
+        // come out as another nonzero multiple than there, which their cofactors
+        // take up: a row outside the panel is multiplied by K0, the product of its
+        // determinants (or of its pivots), and with D the product of all K0, the
+        // cofactor D / pivot of a step's pivots is the product of the earlier steps'
+        // determinants (pivots).
+        // With n <= 32 (HALF) the lanes 32 + r repeat row r and form the second of
+        // every pair of values while the lanes r form the first.
+        auto compose_fast = [&](const int c0, const int buf, auto halfc) __attribute__((always_inline)) -> bool {
+            constexpr bool HALF = decltype(halfc)::value;
+            if (c0 + P > m || rank + P > n)
+                return false;
+            const bool hi = HALF && lane >= 32;
+            // (loads without branches; lanes past row n - 1 repeat it and publish nothing)
+            V pn[H][P];
+            bool ok[H];
 #pragma unroll
             for (int h = 0; h < H; ++h) {
-                const int r = lane + 64 * h;
+                const int r = HALF ? lane & 31 : lane + 64 * h;
+                ok[h] = r < n;
+                const V *x = At + (ok[h] ? r : n - 1) * ms + c0;
+#pragma unroll
+                for (int j = 0; j < P; ++j)
+                    pn[h][j] = x[j];
+            }
+            int sr[P];
+#pragma unroll
+            for (int k = 0; k < P; ++k)
+                sr[k] = rank + k;
+            // value of x in row r (uniform), and of panel column j
+            auto at = [&](const V (&x)[H], const int r) -> V {
+                return lane_value(H == 2 && r >= 64 ? x[H - 1] : x[0], r & 63);
+            };
+            auto col = [&](const int j, const int r) -> V {
+                return lane_value(H == 2 && r >= 64 ? pn[H - 1][j] : pn[0][j], r & 63);
+            };
+            auto row_of = [&](const int h) { return HALF ? lane & 31 : lane + 64 * h; };
+            // the other half's value
+            auto other = [&](const V x) -> V {
+                if constexpr (!HALF) {
+                    return x;
+                } else if constexpr (sizeof(V) == 4) {
+                    const auto v = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+                    return hi ? v[0] : v[1];
+                } else {
+                    const uint32_t l = (uint32_t)x, u = (uint32_t)(x >> 32);
+                    const auto vl = __builtin_amdgcn_permlane32_swap(l, l, false, false);
+                    const auto vu = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+                    return hi ? ((uint64_t)vu[0] << 32) | vl[0] : ((uint64_t)vu[1] << 32) | vl[1];
+                }
+            };
+            // C1, C2 (with HALF: its own one and the other half's) of a 2 x 2 step on
+            // rows r1, r2 and the values x1, x2 (with HALF: own and other) of every row
+            auto pair = [&](const V (&x1)[H], const V (&x2)[H], const V a, const V b, const V cc, const V d,
+                            const V det, const int r1, const int r2, V (&C1)[H], V (&C2)[H]) {
+                const V na = ar.sub(det, a), nd = ar.sub(det, d);
+#pragma unroll
+                for (int h = 0; h < H; ++h) {
+                    const bool me1 = row_of(h) == r1, me2 = row_of(h) == r2;
+                    const V t = ar.msub(x1[h], hi ? a : d, x2[h], hi ? b : cc);
+                    C1[h] = me1 ? (hi ? b : nd) : me2 ? (hi ? na : cc) : t;
+                    if constexpr (HALF) {
+                        C2[h] = other(C1[h]);
+                    } else {
+                        const V u = ar.msub(x2[h], a, x1[h], b);
+                        C2[h] = me1 ? b : me2 ? na : u;
+                    }
+                }
+            };
+            const V a1 = col(0, sr[0]), b1 = col(1, sr[0]);
+            const V c1 = col(0, sr[1]), d1 = col(1, sr[1]);
+            const V D1 = ar.msub(a1, d1, b1, c1);
+            V x1[H], x2[H], C1[H], C2[H];
+#pragma unroll
+            for (int h = 0; h < H; ++h) {
+                x1[h] = hi ? pn[h][1] : pn[h][0];
+                x2[h] = hi ? pn[h][0] : pn[h][1];
+            }
+            pair(x1, x2, a1, b1, c1, d1, D1, sr[0], sr[1], C1, C2);
+            V K0 = D1, k1[H], k2[H], k3[H], k4[H];  // with HALF: k1 | k2 in k1, k3 | k4 in k3
+            if constexpr (P == 2) {
+#pragma unroll
+                for (int h = 0; h < H; ++h) {
+                    k1[h] = ar.sub(0, C1[h]);
+                    k2[h] = ar.sub(0, C2[h]);
+                }
+            } else {
+                // the other two columns after the first step
+                const V q13 = ar.neg(col(2, sr[0])), q14 = ar.neg(col(3, sr[0]));
+                const V q23 = ar.neg(col(2, sr[1])), q24 = ar.neg(col(3, sr[1]));
+                V v3[H], v4[H];
+#pragma unroll
+                for (int h = 0; h < H; ++h) {
+                    v3[h] = ar.reduce(ar.fma(ar.fma(ar.prod(D1, hi ? pn[h][3] : pn[h][2]), C1[h], hi ? q24 : q13),
+                                             C2[h], hi ? q14 : q23));
+                    v4[h] = HALF ? other(v3[h])
+                                 : ar.reduce(ar.fma(ar.fma(ar.prod(D1, pn[h][3]), C1[h], q14), C2[h], q24));
+                }
+                // the second block; with HALF lane 32 + r holds the fourth column
+                const V a2 = at(v3, sr[2]), c2 = at(v3, sr[3]);
+                const V b2 = HALF ? lane_value(v3[0], 32 + sr[2]) : at(v4, sr[2]);
+                const V d2 = HALF ? lane_value(v3[0], 32 + sr[3]) : at(v4, sr[3]);
+                const V D2 = ar.msub(a2, d2, b2, c2);
+                V C3[H], C4[H];
+                pair(v3, v4, a2, b2, c2, d2, D2, sr[2], sr[3], C3, C4);
+                // D2 (D1 row - C1 q1 - C2 q2) - C3 (D1 q3 - c31 q1 - c32 q2) - C4 (D1 q4 - c41 q1 - c42 q2)
+                const V c31 = at(C1, sr[2]), c41 = at(C1, sr[3]);
+                const V c32 = HALF ? lane_value(C1[0], 32 + sr[2]) : at(C2, sr[2]);
+                const V c42 = HALF ? lane_value(C1[0], 32 + sr[3]) : at(C2, sr[3]);
+                const V nD1 = ar.sub(0, D1), nD2 = ar.sub(0, D2);
+                K0 = ar.mul(D1, D2);
+#pragma unroll
+                for (int h = 0; h < H; ++h) {
+                    k1[h] = ar.reduce(ar.fma(ar.fma(ar.prod(nD2, C1[h]), C3[h], hi ? c42 : c31), C4[h], hi ? c32 : c41));
+                    k3[h] = ar.mul(C3[h], nD1);
+                    if constexpr (!HALF) {
+                        k2[h] = ar.reduce(ar.fma(ar.fma(ar.prod(nD2, C2[h]), C3[h], c32), C4[h], c42));
+                        k4[h] = ar.mul(C4[h], nD1);
+                    }
+                }
+            }
+            if (K0 == 0)
+                return false;
+            // publish the coefficients (what the pivot by pivot composition reads
+            // beside them is brought up to date when it first runs)
+#pragma unroll
+            for (int h = 0; h < H; ++h) {
+                V *ck = Ck[buf * kMaxN + row_of(h)].v;
                 if (ok[h]) {
-#pragma unroll
-                    for (int s2 = 0; s2 <= P; ++s2)
-                        Ck[(buf * kMaxN + r) * (P + 1) + s2] = cc[h][s2];
-                    ispiv[r] = isp[h] ? 1 : 0;
+                    if constexpr (HALF) {
+                        ck[hi ? 1 : 0] = k1[h];
+                        if constexpr (P == 4)
+                            ck[hi ? 3 : 2] = k3[h];
+                    } else {
+                        ck[0] = k1[h];
+                        ck[1] = k2[h];
+                        if constexpr (P == 4) {
+                            ck[2] = k3[h];
+                            ck[3] = k4[h];
+                        }
+                    }
                 }
             }
             if (lane == 0) {
-                // pivot bookkeeping, read only after the elimination
-                int q = rank;
-#pragma unroll
-                for (int k = 0; k < P; ++k) {
-                    if (tk >> k & 1) {
-                        prow[q] = prs[k];
-                        pivcol[q] = c0 + k;
-                        colpiv[c0 + k] = 1;
-                        pos[c0 + k] = prs[k];  // the column's pivot row
-                        ++q;
-                    }
-                }
-                s_nb[buf] = nb;
-#pragma unroll
-                for (int k = 0; k < P; ++k)
-                    s_prs[buf][k] = prs[k];
+                s_tk[buf] = kFastPanel | (kFastPanel - 1);
+                s_K0[buf] = K0;
+                s_pre[buf][0] = D1;
             }
-        }
-        __builtin_amdgcn_s_setprio(0);
-    };
-    // Residuals of at most 32 columns (n <= 32 rows of At) leave the upper
-    // half of the composing wave idle in compose().  compose_half() puts the
-    // coefficient slots there: upper lane 32 + r holds slots 0, 1, 2 of row r
-    // (slots 0, 1 for P = 2) and lower lane r the row's panel values and the
-    // last slots, in registers whose lower halves pass from a panel column to
-    // a slot once that column is eliminated.  Each instruction then advances
-    // a panel value and a coefficient at once: three multiply-subtracts per
-    // pivot step instead of five (two instead of three for P = 2).
-    //   P = 4, registers Z A B C: lower lane r holds row r in panel columns
-    //   0..3, A becomes slot 3 before step 2 and B slot 4 before step 3;
-    //   upper lane 32 + r holds slots 0, 1, 2 in A, B, C.
-    //   P = 2, registers Z A B: lower lane r holds columns 0, 1 in Z, A and
-    //   slot 2 in B; upper lane 32 + r holds slots 0, 1 in A, B.
-    // Slot 0 takes pv * c0 as the multiply-subtract with q = 0 (pv c0 + fr p,
-    // the same residue); a register that starts a slot holds zero, so the
-    // slot's first value is -fr * q as in compose().
-    auto compose_half = [&](const int c0, const int buf) __attribute__((always_inline)) {
-        __builtin_amdgcn_s_setprio(2);
-        {
-            static_assert(P == 2 || P == 4, "compose_half is written out for panels of 2 and 4");
-            const bool hi = lane >= 32;
-            const int r = lane & 31;
-            const bool ok = r < n;
-            auto col = [&](const int j) -> V {
-                return !hi && ok && c0 + j < m ? At[r * ms + c0 + j] : (V)0;
-            };
-            V Z = col(0);
-            V A = hi ? ar.one() : col(1);
-            V B = P == 4 ? col(2) : (V)0;
-            V C = P == 4 ? col(3) : (V)0;
-            bool isp = !hi && ok && ispiv[r];
-            int prs[P] = {0};
-            int tk = 0, nb = 0;
-            // every lane gets the value of x in lane (lane & 31)
-            auto low = [](const V x) -> V {
-                if constexpr (sizeof(V) == 4) {
-                    return __builtin_amdgcn_permlane32_swap(x, x, false, false)[0];
-                } else {
-                    const uint32_t l = (uint32_t)x, h = (uint32_t)(x >> 32);
-                    const uint32_t l2 = __builtin_amdgcn_permlane32_swap(l, l, false, false)[0];
-                    const uint32_t h2 = __builtin_amdgcn_permlane32_swap(h, h, false, false)[0];
-                    return ((uint64_t)h2 << 32) | l2;
-                }
-            };
-            auto step = [&](auto jc) __attribute__((always_inline)) {
-                constexpr int j = decltype(jc)::value;
-                if constexpr (P == 4 && j == 2)
-                    A = hi ? A : (V)0;  // column 1 is done: lower A is slot 3
-                if constexpr (P == 4 && j == 3)
-                    B = hi ? B : (V)0;  // column 2 is done: lower B is slot 4
-                const V xj = j == 0 ? Z : j == 1 ? A : j == 2 ? B : C;
-                const bool open = c0 + j < m && rank + nb < n;
-                const unsigned long long b = __ballot(open && !hi && ok && !isp && xj != 0);
-                if (!b)
-                    return;  // no pivot in this column
-                const int pr = __ffsll(b) - 1;  // a lower lane
-                const bool me = r == pr;
-                const V pv = lane_value(xj, pr);
-                const V fr = low(xj);
-                const V Q = lane_value(A, 32 + pr);  // the pivot row's slot 0
-                constexpr int G = P == 4 ? 3 : 2;
-                V xs[G], qs[G], ts[G], kp[G];  // operands, and what the pivot row keeps
-                const V zero = 0;
-                if constexpr (P == 4) {
-                    xs[0] = A;
-                    xs[1] = B;
-                    xs[2] = C;
-                    if constexpr (j == 0) {
-                        const V p1 = lane_value(A, pr), p2 = lane_value(B, pr), p3 = lane_value(C, pr);
-                        qs[0] = hi ? zero : p1;
-                        qs[1] = hi ? Q : p2;
-                        qs[2] = hi ? zero : p3;
-                        kp[0] = hi ? zero : A;
-                        kp[1] = hi ? Q : B;
-                        kp[2] = C;
-                    } else if constexpr (j == 1) {
-                        const V p2 = lane_value(B, pr), p3 = lane_value(C, pr), q1 = lane_value(B, 32 + pr);
-                        qs[0] = zero;
-                        qs[1] = hi ? q1 : p2;
-                        qs[2] = hi ? Q : p3;
-                        kp[0] = hi ? zero : A;
-                        kp[1] = B;
-                        kp[2] = hi ? Q : C;
-                    } else if constexpr (j == 2) {
-                        const V p3 = lane_value(C, pr), q1 = lane_value(B, 32 + pr), q2 = lane_value(C, 32 + pr);
-                        qs[0] = hi ? zero : Q;
-                        qs[1] = hi ? q1 : zero;
-                        qs[2] = hi ? q2 : p3;
-                        kp[0] = hi ? zero : Q;
-                        kp[1] = B;
-                        kp[2] = C;
-                    } else {
-                        const V q3 = lane_value(A, pr), q1 = lane_value(B, 32 + pr), q2 = lane_value(C, 32 + pr);
-                        qs[0] = hi ? zero : q3;
-                        qs[1] = hi ? q1 : Q;
-                        qs[2] = hi ? q2 : zero;
-                        kp[0] = hi ? zero : A;
-                        kp[1] = hi ? B : Q;
-                        kp[2] = C;
+            return true;
+        };
+        // the split composition needs one row per lane and the Montgomery forms;
+        // the composition by pairs does not fit the registers with two rows of
+        // 64-bit words per lane
+        constexpr bool kMont = !std::is_same<Arith, BigArith>::value;
+        constexpr bool kFast = kMont && (H == 1 || sizeof(V) == 4);
+        constexpr bool kHalf = H == 1 && kMont;
+        const bool half = kHalf && n <= 32;
+        bool inorder = kFast;  // every panel so far by compose_fast (uniform)
+        auto compose_panel = [&](const int c0, const int buf) __attribute__((always_inline)) {
+            if constexpr (kFast) {
+                if (inorder) {
+                    __builtin_amdgcn_s_setprio(2);
+                    bool done = false;
+                    if constexpr (kHalf) {
+                        if (half)
+                            done = compose_fast(c0, buf, std::true_type{});
                     }
-                } else {
-                    xs[0] = A;
-                    xs[1] = B;
-                    if constexpr (j == 0) {
-                        const V p1 = lane_value(A, pr);
-                        qs[0] = hi ? zero : p1;
-                        qs[1] = hi ? Q : zero;
-                        kp[0] = hi ? zero : A;
-                        kp[1] = hi ? Q : B;
-                    } else {
-                        const V q1 = lane_value(B, 32 + pr);
-                        qs[0] = zero;
-                        qs[1] = hi ? q1 : Q;
-                        kp[0] = hi ? zero : A;
-                        kp[1] = hi ? B : Q;
-                    }
-                }
-                ar.msub_n(pv, xs, fr, qs, ts);
-                A = me ? kp[0] : ts[0];
-                B = me ? kp[1] : ts[1];
-                if constexpr (P == 4)
-                    C = me ? kp[2] : ts[2];
-                isp = isp || me;  // read in the lower half only
-                prs[j] = pr;
-                tk |= 1 << j;
-                ++nb;
-            };
-            step(std::integral_constant<int, 0>{});
-            step(std::integral_constant<int, 1>{});
-            if constexpr (P == 4) {
-                step(std::integral_constant<int, 2>{});
-                step(std::integral_constant<int, 3>{});
-            }
-            // publish: coefficients, pivot flags, pivot rows
-            if (ok) {
-                V *ck = Ck + (buf * kMaxN + r) * (P + 1);
-                if (hi) {
-                    ck[0] = A;
-                    ck[1] = B;
-                    if constexpr (P == 4)
-                        ck[2] = C;
-                } else {
-                    if constexpr (P == 4) {
-                        ck[3] = A;
-                        ck[4] = B;
-                    } else {
-                        ck[2] = B;
-                    }
-                    ispiv[r] = isp ? 1 : 0;
+                    if (!half)
+                        done = compose_fast(c0, buf, std::false_type{});
+                    __builtin_amdgcn_s_setprio(0);
+                    if (done)
+                        return;
+                    // the first panel pivot by pivot: the rows used before
+                    for (int r = lane; r < rank; r += 64)
+                        ispiv[r] = 1;
                 }
             }
-            if (lane == 0) {
-                // pivot bookkeeping, read only after the elimination
-                int q = rank;
-#pragma unroll
-                for (int k = 0; k < P; ++k) {
-                    if (tk >> k & 1) {
-                        prow[q] = prs[k];
-                        pivcol[q] = c0 + k;
-                        colpiv[c0 + k] = 1;
-                        pos[c0 + k] = prs[k];  // the column's pivot row
-                        ++q;
-                    }
+            if constexpr (kHalf) {
+                if (half) {
+                    compose_half(c0, buf);
+                    return;
                 }
-                s_nb[buf] = nb;
-#pragma unroll
-                for (int k = 0; k < P; ++k)
-                    s_prs[buf][k] = prs[k];
             }
-        }
-        __builtin_amdgcn_s_setprio(0);
-    };
-    // the split composition needs one row per lane and the Montgomery forms
-    constexpr bool kHalf = H == 1 && !std::is_same<Arith, BigArith>::value;
-    const bool half = kHalf && n <= 32;
-    auto compose_panel = [&](const int c0, const int buf) __attribute__((always_inline)) {
-        if constexpr (kHalf) {
-            if (half) {
-                compose_half(c0, buf);
+            compose(c0, buf);
+        };
+        // apply the combination in buffer buf to this wave's columns: the pivot
+        // rows' values are read before any row is written.  Every term is
+        // formed: a panel column without a pivot has row 0 in s_prs and zero
+        // coefficients in every row, so its term is zero, and issuing all loads
+        // before the products (no branch between them) keeps the LDS round
+        // trips of a panel to three instead of one per term.
+        // A pivot column of an earlier panel (below cdone) is zero but in its
+        // pivot row, and no later pivot row has a nonzero there: the combination
+        // only multiplies that row's value by the row's own coefficient.
+        const int acl = lane & (cw - 1), ag = lane / cw, aG = 64 / cw;  // cw: a power of two
+        const int acg = wave * cw + acl;
+        auto apply = [&](const int buf, const int cdone) __attribute__((always_inline)) {
+            if (acg >= m)
+                return;
+            // (in order: the pivot of column c < cdone = rank is in row c, and the
+            // panel's pivot rows follow, so nothing is looked up)
+            if (acg < cdone && (inorder || colpiv[acg])) {
+                const int r = inorder ? acg : pos[acg];
+                if (ag == (r & (aG - 1))) {
+                    V *x = At + r * ms + acg;
+                    *x = ar.mul(inorder ? s_K0[buf] : C0[buf * kMaxN + r], *x);
+                }
                 return;
             }
-        }
-        compose(c0, buf);
-    };
-    // apply the combination in buffer buf to this wave's columns: the pivot
-    // rows' values are read before any row is written.  Every term is
-    // formed: a panel column without a pivot has row 0 in s_prs and zero
-    // coefficients in every row, so its term is zero, and issuing all loads
-    // before the products (no branch between them) keeps the LDS round
-    // trips of a panel to three instead of one per term.
-    // A pivot column of an earlier panel (below cdone) is zero but in its
-    // pivot row, and no later pivot row has a nonzero there: the combination
-    // only multiplies that row's value by the row's own coefficient.
-    const int acl = lane & (cw - 1), ag = lane / cw, aG = 64 / cw;  // cw: a power of two
-    const int acg = wave * cw + acl;
-    auto apply = [&](const int buf, const int cdone) __attribute__((always_inline)) {
-        if (acg >= m)
-            return;
-        if (acg < cdone && colpiv[acg]) {
-            const int r = pos[acg];
-            if (ag == (r & (aG - 1))) {
-                V *x = At + r * ms + acg;
-                *x = ar.mul(Ck[(buf * kMaxN + r) * (P + 1)], *x);
+            V pvr[P];
+            if (inorder) {
+#pragma unroll
+                for (int q = 0; q < P; ++q)
+                    pvr[q] = At[(cdone + q) * ms + acg];
+            } else {
+                int prq[P];
+#pragma unroll
+                for (int q = 0; q < P; ++q)
+                    prq[q] = s_prs[buf][q];
+#pragma unroll
+                for (int q = 0; q < P; ++q)
+                    pvr[q] = At[prq[q] * ms + acg];
             }
-            return;
+            // rows in pairs (32-bit words: two rows of 64-bit words exceed the
+            // registers), their loads before the products
+            constexpr int RP = sizeof(V) == 4 ? 2 : 1;
+            const V K0 = s_K0[buf];  // slot 0 of every row (in order)
+            for (int r = ag; r < n; r += RP * aG) {
+                V *x[RP];
+                Row cv[RP];
+                V c0[RP];
+#pragma unroll
+                for (int e = 0; e < RP; ++e) {
+                    const int re = r + e * aG < n ? r + e * aG : r;  // (then the same value again)
+                    x[e] = At + re * ms + acg;
+                    cv[e] = Ck[buf * kMaxN + re];
+                    c0[e] = inorder ? K0 : C0[buf * kMaxN + re];
+                }
+                typename Arith::Acc acc[RP];
+#pragma unroll
+                for (int e = 0; e < RP; ++e)
+                    acc[e] = ar.prod(c0[e], *x[e]);
+#pragma unroll
+                for (int q = 0; q < P; ++q)
+#pragma unroll
+                    for (int e = 0; e < RP; ++e)
+                        acc[e] = ar.fma(acc[e], cv[e].v[q], pvr[q]);
+#pragma unroll
+                for (int e = 0; e < RP; ++e)
+                    *x[e] = ar.reduce(acc[e]);
+            }
+        };
+        if (wave == 0)
+            compose_panel(0, 0);
+        lds_barrier();
+        V dall = ar.one();  // in the last wave: product of the panels' own coefficients
+        for (int k = 0;; ++k) {
+            const int buf = k & 1;
+            const int tk = s_tk[buf] & (kFastPanel - 1), nb = __popc(tk);
+            inorder = inorder && (s_tk[buf] & kFastPanel);
+            if (nb > 0)
+                apply(buf, k * P);
+            if (wave == kStepThreads / 64 - 1 && lane < P) {
+                // pivot bookkeeping, off the composing wave's path: the pivots' rows
+                // and cofactors, read after the elimination, and their columns, read
+                // from the next panel's apply on
+                const V K0 = s_K0[buf];
+                if (tk >> lane & 1) {
+                    const int q = rank + __popc(tk & ((1 << lane) - 1));
+                    const int pr = inorder ? rank + lane : s_prs[buf][lane];
+                    const V pre = inorder ? (lane < 2 ? ar.one() : s_pre[buf][0]) : s_pre[buf][lane];
+                    prow[q] = pr;
+                    cof[q] = ar.mul(dall, pre);
+                    colpiv[k * P + lane] = 1;
+                    pos[k * P + lane] = pr;
+                }
+                dall = ar.mul(dall, K0);
+            }
+            rank += nb;
+            const int c1 = (k + 1) * P;
+            if (c1 >= m || rank >= n)
+                break;
+            if (wave == c1 / cw)
+                compose_panel(c1, buf ^ 1);
+            lds_barrier();
         }
-        int prq[P];
+        if (tid == kStepThreads - 64)
+            s_D = dall;
+        lds_barrier();
+        // With D the product of the panels' own coefficients and cof[k] the cofactor
+        // of pivot k (D over the pivot), the kernel vectors are D times the
+        // normalised ones, and no inverse is needed in the step.  Pivots are
+        // nonzero, so is D.
+        const V D = s_D;
+        // permutation list of left_nullspace_compact: pivot columns, then the
+        // others; one wave counts the pivot columns before each column by ballots
+        if (tid >= kStepThreads - 64) {
+            const int l = tid - (kStepThreads - 64);
+            int base = 0;
 #pragma unroll
-        for (int q = 0; q < P; ++q)
-            prq[q] = s_prs[buf][q];
-        V pvr[P];
-#pragma unroll
-        for (int q = 0; q < P; ++q)
-            pvr[q] = At[prq[q] * ms + acg];
-        const V *C = Ck + buf * kMaxN * (P + 1);
-        for (int r = ag; r < n; r += aG) {
-            const V *cr = C + r * (P + 1);
-            V *x = At + r * ms + acg;
-            V cv[P + 1];
-#pragma unroll
-            for (int s2 = 0; s2 <= P; ++s2)
-                cv[s2] = cr[s2];
-            typename Arith::Acc acc = ar.prod(cv[0], *x);
-#pragma unroll
-            for (int q = 0; q < P; ++q)
-                acc = ar.fma(acc, cv[q + 1], pvr[q]);
-            *x = ar.reduce(acc);
+            for (int h = 0; h < kMaxM / 64; ++h) {
+                const int i = l + 64 * h;
+                const bool pc = i < m && colpiv[i];
+                const unsigned long long b = __ballot(pc);
+                const int before = base + __popcll(b & ((1ull << l) - 1));
+                if (i < m) {
+                    if (pc)
+                        plist[before] = i;
+                    else
+                        plist[rank + i - before] = i;
+                }
+                base += __popcll(b);
+            }
         }
-    };
-    if (wave == 0)
-        compose_panel(0, 0);
-    __syncthreads();
-    for (int k = 0;; ++k) {
-        const int buf = k & 1;
-        const int nb = s_nb[buf];
-        if (nb > 0)
-            apply(buf, k * P);
-        rank += nb;
-        const int c1 = (k + 1) * P;
-        if (c1 >= m || rank >= n)
+        lds_barrier();
+        const int nullity = m - rank;
+        if (nullity == 0) {
+            full = true;  // appbas <- x^(ordL - ord) appbas ends the leaf
             break;
-        if (wave == c1 / cw)
-            compose_panel(c1, buf ^ 1);
-        __syncthreads();
-    }
-    __syncthreads();
-    // Cofactors of the pivots of the reduced echelon form: for pivot k, the
-    // product of all the others (Montgomery's simultaneous-inversion trick
-    // without the inversion): the kernel vectors are then D times the
-    // normalised ones, D the product of all pivots, and no inverse is needed
-    // in the step.  Wave 0, lane l holding pivots l and l + 64 (rank <= 128):
-    // prefix and suffix products by scans across the wave.  Pivots are
-    // nonzero, so is D.
-    __shared__ V s_D;
-    if (wave == 0) {
-        const V x0 = lane < rank ? At[prow[lane] * ms + pivcol[lane]] : ar.one();
-        const V x1 = lane + 64 < rank ? At[prow[lane + 64] * ms + pivcol[lane + 64]] : ar.one();
-        const V v = ar.mul(x0, x1);
-        V pre = v, suf = v;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const V up = __shfl_up(pre, d);
-            const V dn = __shfl_down(suf, d);
-            if (lane >= d)
-                pre = ar.mul(pre, up);
-            if (lane + d < 64)
-                suf = ar.mul(suf, dn);
         }
-        V ex = __shfl_up(pre, 1), exs = __shfl_down(suf, 1);
-        if (lane == 0)
-            ex = ar.one();
-        if (lane == 63)
-            exs = ar.one();
-        const V others = ar.mul(ex, exs);  // every other lane's pair
-        if (lane < rank)
-            cof[lane] = ar.mul(others, x1);
-        if (lane + 64 < rank)
-            cof[lane + 64] = ar.mul(others, x0);
-        if (lane == 63)
-            s_D = pre;
-    }
-    // permutation list of left_nullspace_compact: pivot columns, then the
-    // others; the last wave (the cofactors run on the first one) counts the
-    // pivot columns before each column by ballots
-    if (tid >= kStepThreads - 64) {
-        const int l = tid - (kStepThreads - 64);
-        int base = 0;
+        if (rank > 0) {
+            // kernel vectors: one per wave at a time, lane r (and r + 64) its entry r
+            V *X = reinterpret_cast<V *>(a.X) + (size_t)s * m * m;
+            constexpr int RH = kMaxN / 64;
+            V cf[RH];
+            int xrow[RH];
 #pragma unroll
-        for (int h = 0; h < kMaxM / 64; ++h) {
-            const int i = l + 64 * h;
-            const bool pc = i < m && colpiv[i];
-            const unsigned long long b = __ballot(pc);
-            const int before = base + __popcll(b & ((1ull << l) - 1));
-            if (i < m) {
-                if (pc)
-                    plist[before] = i;
-                else
-                    plist[rank + i - before] = i;
+            for (int h = 0; h < RH; ++h) {
+                const int r = lane + 64 * h;
+                cf[h] = r < rank ? cof[r] : (V)0;
+                xrow[h] = r < rank ? prow[r] * ms : 0;
             }
-            base += __popcll(b);
-        }
-    }
-    __syncthreads();
-    const int nullity = m - rank;
-    const int mode = nullity == 0 ? 2 : (nullity == m ? 0 : 1);
-    if (mode == 1) {
-        for (int idx = tid; idx < nullity * rank; idx += kStepThreads) {
-            const int t = idx / rank, r = idx - t * rank;
-            const uint64_t v = ar.from(ar.mul(At[prow[r] * ms + plist[rank + t]], cof[r]));
-            a.X[(size_t)t * m + r] = v ? p - v : 0;
-        }
-        for (int i = tid; i < m; i += kStepThreads) {
-            const int row = perm[plist[i]];
-            a.piv[i] = row;
-            a.rowinfo[row] = i < rank ? -1 - i : i - rank;
-            if (i < rank)
-                a.shift[row] = sh[row] + 1;
-            // rows updated by a kernel vector take the factor D; the scales
-            // start at 1 (Montgomery form) at the leaf's first step
-            if (ord == 0 || i >= rank) {
-                const V s0 = ord == 0 ? ar.one() : (V)a.scale[row];
-                a.scale[row] = i >= rank ? ar.mul(s0, s_D) : s0;
+            for (int t = wave; t < nullity; t += kStepThreads / 64) {
+                const int col = plist[rank + t];
+#pragma unroll
+                for (int h = 0; h < RH; ++h) {
+                    const int r = lane + 64 * h;
+                    if (r < rank) {
+                        const V v = ar.sub(0, ar.mul(At[xrow[h] + col], cf[h]));
+                        At[xrow[h] + col] = v;
+                        X[(size_t)t * m + r] = v;
+                    }
+                }
+            }
+            if (tid < m) {
+                const int row = perm[plist[tid]];
+                a.piv[s * m + tid] = row;
+                // rows updated by a kernel vector take the factor D
+                if (tid >= rank)
+                    scl[row] = ar.mul(scl[row], D);
+            }
+            if (tid == 0)
+                a.scale[m + s] = D;
+            // The window's remaining coefficients, orders s + 1 .. w - 1: two kernel
+            // rows per wave at a time, a lane per (order, column).  The vectors and
+            // the pivot rows' places sit in registers, lane r for pivot r, and are
+            // read lane by lane into scalar registers: per pivot one LDS load for
+            // two products.  With at most 32 (order, column) pairs the wave's halves,
+            // quarters or eighths take a kernel row each and read their vectors'
+            // entries from LDS.  The pivot rows' coefficients are read before they
+            // move up by their delay; a kernel row's own are read and written by its
+            // lanes alone.
+            lds_barrier();
+            if (s + 1 < w) {
+                const int ncol = (w - 1 - s) * n;
+                int rbase[RH];
+#pragma unroll
+                for (int h = 0; h < RH; ++h) {
+                    const int r = lane + 64 * h;
+                    const int pr = r < rank ? perm[plist[r]] : 0;
+                    rbase[h] = r < rank ? (s + 1 - delay[pr]) * mn + pr * n : 0;
+                }
+                constexpr int NW = kStepThreads / 64;
+                const int gl = ncol <= 8 ? 3 : ncol <= 16 ? 4 : 5;  // log2 of a group's lanes
+                for (int t0 = wave << (6 - gl); ncol <= 32 && t0 < nullity; t0 += NW << (6 - gl)) {
+                    const int tg = t0 + (lane >> gl), ql = lane & ((1 << gl) - 1);
+                    const bool live = tg < nullity && ql < ncol;
+                    const int col = plist[rank + (live ? tg : t0)], i = perm[col];
+                    int d = 0, j = live ? ql : 0;
+                    while (j >= n) {
+                        j -= n;
+                        ++d;
+                    }
+                    const int off = d * mn + j;
+                    V *own = Rw + (s + 1 - delay[i]) * mn + i * n;
+                    V sum = ar.mul(D, own[off]);
+#pragma unroll
+                    for (int h = 0; h < RH; ++h)
+                        for (int r0 = 0; r0 < 64 && r0 + 64 * h < rank; r0 += 8) {
+                            V y[8], x[8];
+#pragma unroll
+                            for (int u = 0; u < 8; ++u) {
+                                y[u] = Rw[__builtin_amdgcn_readlane(rbase[h], r0 + u) + off];
+                                x[u] = At[__builtin_amdgcn_readlane(xrow[h], r0 + u) + col];
+                                x[u] = r0 + u + 64 * h < rank ? x[u] : (V)0;
+                            }
+                            typename Arith::Acc p1 = ar.prod(x[0], y[0]);
+#pragma unroll
+                            for (int u = 1; u < 8; ++u)
+                                p1 = ar.fma(p1, x[u], y[u]);
+                            sum = ar.add(sum, ar.reduce(p1));
+                        }
+                    if (live)
+                        own[off] = sum;
+                }
+                for (int t = wave; ncol > 32 && t < nullity; t += 2 * NW) {
+                    const int t2 = t + NW < nullity ? t + NW : t;
+                    const int col1 = plist[rank + t], col2 = plist[rank + t2];
+                    const int i1 = perm[col1], i2 = perm[col2];
+                    V xa[RH], xb[RH];
+#pragma unroll
+                    for (int h = 0; h < RH; ++h) {
+                        const int r = lane + 64 * h;
+                        xa[h] = r < rank ? At[xrow[h] + col1] : (V)0;
+                        xb[h] = r < rank ? At[xrow[h] + col2] : (V)0;
+                    }
+                    V *own1 = Rw + (s + 1 - delay[i1]) * mn + i1 * n, *own2 = Rw + (s + 1 - delay[i2]) * mn + i2 * n;
+                    for (int q0 = 0; q0 < ncol; q0 += 64) {
+                        const int q = q0 + lane < ncol ? q0 + lane : 0;
+                        int d = 0, j = q;
+                        while (j >= n) {
+                            j -= n;
+                            ++d;
+                        }
+                        const int off = d * mn + j;
+                        V sum1 = ar.mul(D, own1[off]), sum2 = ar.mul(D, own2[off]);
+#pragma unroll
+                        for (int h = 0; h < RH; ++h)
+                            for (int r0 = 0; r0 < 64 && r0 + 64 * h < rank; r0 += 8) {
+                                // (pivots past the rank: zero vectors, place 0)
+                                typename Arith::Acc p1, p2;
+                                constexpr int G = sizeof(V) == 4 ? 8 : 4;  // loads together
+#pragma unroll
+                                for (int g0 = 0; g0 < 8; g0 += G) {
+                                    V y[G];
+#pragma unroll
+                                    for (int u = 0; u < G; ++u)
+                                        y[u] = Rw[__builtin_amdgcn_readlane(rbase[h], r0 + g0 + u) + off];
+#pragma unroll
+                                    for (int u = 0; u < G; ++u) {
+                                        const V x1 = lane_value(xa[h], r0 + g0 + u);
+                                        const V x2 = lane_value(xb[h], r0 + g0 + u);
+                                        p1 = g0 + u == 0 ? ar.prod(x1, y[u]) : ar.fma(p1, x1, y[u]);
+                                        p2 = g0 + u == 0 ? ar.prod(x2, y[u]) : ar.fma(p2, x2, y[u]);
+                                    }
+                                }
+                                sum1 = ar.add(sum1, ar.reduce(p1));
+                                sum2 = ar.add(sum2, ar.reduce(p2));
+                            }
+                        if (q0 + lane < ncol) {
+                            own1[off] = sum1;
+                            own2[off] = sum2;  // (t2 = t: the same value again)
+                        }
+                    }
+                }
+            }
+            lds_barrier();
+            if (tid < rank) {
+                const int row = perm[plist[tid]];
+                sh[row] += 1;
+                delay[row] += 1;
             }
         }
         if (tid == 0)
-            a.scale[m] = sizeof(V) == 8 ? ar.from(s_D) : (uint64_t)s_D;
-    } else if (mode == 2) {
-        for (int i = tid; i < m; i += kStepThreads)
-            a.shift[i] = sh[i] + (a.ordL - ord);
+            c[C_RANK + s] = rank;
+        steps = s + 1;
+        lds_barrier();
     }
-    if (mode != 1 && ord == 0)
-        for (int i = tid; i < m; i += kStepThreads)
-            a.scale[i] = ar.one();
+    if (tid < m) {
+        a.shift[tid] = sh[tid] + (full ? a.ordL - (ord0 + steps) : 0);
+        a.scale[tid] = scl[tid];
+    }
     if (tid == 0) {
-        const int len = c[C_LEN] + c[C_GROW];
         c[C_CUR] = cur;
-        c[C_GROW] = 0;
-        c[C_LEN] = len;
-        c[C_MODE] = mode;
-        c[C_RANK] = rank;
-        c[C_FLIP] = mode != 0 ? 1 : 0;
-        if (mode == 2) {
-            c[C_SHIFT] = a.ordL - ord;
-            c[C_LOLD] = len;
-            c[C_LEN] = len + (a.ordL - ord);
+        c[C_STEPS] = steps;
+        c[C_FLIP] = steps > 0 ? 1 : 0;
+        if (full) {
             c[C_DONE] = 1;
+            c[C_SHIFT] = a.ordL - (ord0 + steps);
         }
     }
 }
 
 // ---------------------------------------------------------------------------
-// kernel 2: apply the step to appbas (and to the residual series)
+// kernel 2: apply a window to appbas and to the residual series
 // ---------------------------------------------------------------------------
-// base + sum_r X[t][r] * src[row piv[r], column j, coefficient d].  All
-// loads of a group of terms (32 words below 2^30, or 16 64-bit words: one L2
-// round trip) are issued before its products, with no branch between them:
-// terms past the rank read row piv[r] of the LDS row list (padded with row 0
-// up to kMaxM; rank <= kMaxN) and X words past the row (X carries kXPad words
-// of padding),
-// and their X coefficient is zeroed by a select after the load.
-template <bool SMALL, bool BIG>
-__device__ __forceinline__ uint64_t row_combo(const uint64_t *src, const LeafArgs &a, const int *piv, int t,
-                                              int rank, int stride, int cols, int j, int d, uint64_t base)
+// One workgroup takes kTile - w coefficients d0 .. of one column (of appbas,
+// then of R) for all m rows, and the w before them, which rows multiplied by x
+// bring in: row i of the tile Y holds coefficients d0 - w .., and its
+// coefficient d is at Y[i][d - d0 + w - del[i]] after del[i] such
+// multiplications.  The window's orders are applied one after the other in
+// LDS, a thread per coefficient of the tile and kernel row, so that the tile is
+// read and written once per window instead of once per order, and the launch,
+// the control words' round trip and the tile's are paid once.  Order s leaves
+// the first s coefficients of the halo undefined.
+// STAGE: the window's kernel vectors are brought to LDS at the start, beside
+// the tile (rows padded with zeros to a multiple of kGroup), so that the orders
+// wait for no global load; without it (vectors too large for LDS) they are
+// read where they are.
+// Latency bounds it: 16.6 us per window of 4 orders (64 x 32, 32-bit words; 4 x
+// 7.4 to 9.5 with a launch per order), of which 2.3 are the loads, 1.5 each
+// order and the rest the launch's start and end.  18.5 us with the vectors read
+// from memory order by order.
+constexpr int kUpdateThreads = 512;
+constexpr int kGroup = 16;  // pivots taken together
+__host__ __device__ inline int pad16(int r)
 {
-    const uint64_t *xr = a.X + (size_t)t * a.m;
-    const uint64_t *sj = src + (size_t)j * stride + d;
-    const size_t rstride = (size_t)cols * stride;
-    constexpr int G = SMALL ? 32 : 16;
-    uint64_t acc = base;
-    for (int r = 0; r < rank; r += G) {
-        if constexpr (SMALL) {
-            // p < 2^30: words are read through their low halves; 16 products
-            // stay below 16 (p - 1)^2 < 2^64 - 2^35, so each half-group is
-            // summed with a residue before one Barrett reduction
-            uint32_t sv[G], xv[G];
-#pragma unroll
-            for (int u = 0; u < G; ++u) {
-                sv[u] = (uint32_t)sj[(size_t)piv[r + u] * rstride];
-                const uint32_t x = (uint32_t)xr[r + u];
-                xv[u] = r + u < rank ? x : 0u;
-            }
-#pragma unroll
-            for (int h = 0; h < G; h += 16) {
-                uint64_t part = 0;
-#pragma unroll
-                for (int u = h; u < h + 16; ++u)
-                    part += (uint64_t)xv[u] * sv[u];
-                acc = barrett(acc + part, a.mc.bm, a.mc.p);
-            }
-        } else if constexpr (BIG) {
-            // p >= 2^62: every product reduced at once, the sum kept below p
-            uint64_t sv[G], xv[G];
-#pragma unroll
-            for (int u = 0; u < G; ++u) {
-                sv[u] = sj[(size_t)piv[r + u] * rstride];
-                const uint64_t x = xr[r + u];
-                xv[u] = r + u < rank ? x : 0;
-            }
-#pragma unroll
-            for (int u = 0; u < G; ++u)
-                acc = addmod_any(acc, mulmod_any(xv[u], sv[u], a.mc), a.mc.p);
-        } else {
-            // 64-bit words (p < 2^62): an exact 128-bit sum of 16 products
-            // and a residue, 16 (p - 1)^2 + p < 2^128 - 2^67, folded once (the
-            // 128-bit products are the bound here, not the loads)
-            uint64_t sv[G], xv[G];
-#pragma unroll
-            for (int u = 0; u < G; ++u) {
-                sv[u] = sj[(size_t)piv[r + u] * rstride];
-                const uint64_t x = xr[r + u];
-                xv[u] = r + u < rank ? x : 0;
-            }
-            uint64_t hi = 0, lo = acc;
-#pragma unroll
-            for (int u = 0; u < G; ++u)
-                mac128(hi, lo, xv[u], sv[u]);
-            acc = reduce128(hi, lo, a.mc);
-        }
-    }
-    return acc;
+    return (r + 15) & ~15;
 }
-
-template <bool SMALL, bool BIG>
-__global__ void __launch_bounds__(256) mbasis_update_kernel(LeafArgs a, int ord)
+// most words of one order's padded kernel vectors
+inline size_t staged_words(int m, int n)
 {
-    // The control words, the step's row list and row roles and its factor D
-    // are all requested at entry, before any branch on them: one round trip
-    // to memory instead of three dependent ones (mode, then the row lists,
-    // then rank, length and D).  In modes 0 and 2 the lists and D are stale
-    // and unused.
-    static_assert(kMaxM == 256, "one row-list entry per thread of the 256-thread workgroup");
-    const int mode = a.ctl[C_MODE];
-    const int cur = a.ctl[C_CUR];
-    const int rank = a.ctl[C_RANK];
-    const int L = a.ctl[C_LEN];
-    const uint64_t D = a.scale[a.m];
-    const int tx = threadIdx.x;
-    const int piv_t = tx < a.m ? a.piv[tx] : 0;  // groups read up to kMaxM entries
-    const int rinfo_t = tx < a.m ? a.rowinfo[tx] : 0;
-    const unsigned tstride = gridDim.x * blockDim.x;
-    const unsigned t0 = blockIdx.x * blockDim.x + threadIdx.x;
-    if (mode == 0) {
-        // residual unchanged: the coming step's coefficient is ord + 1
-        // (nothing to do once the basis is complete)
-        if (ord + 1 < a.ordL && !a.ctl[C_DONE]) {
-            const uint64_t *rs = a.R[cur];
-            for (unsigned e = t0; e < (unsigned)(a.m * a.n); e += tstride)
-                a.Rn[e] = rs[(size_t)e * a.ordL + ord + 1];
-        }
-        return;
-    }
-    const int m = a.m, n = a.n, cap = a.cap;
-    const uint64_t *src = a.app[cur];
-    uint64_t *dst = a.app[cur ^ 1];
-    if (mode == 2) {
-        const int s = a.ctl[C_SHIFT], Lold = a.ctl[C_LOLD];
-        const unsigned Lnew = (unsigned)(Lold + s);
-        const unsigned items = (unsigned)(m * m) * Lnew;
-        for (unsigned idx = t0; idx < items; idx += tstride) {
-            const unsigned e = idx / Lnew;
-            const int d = (int)(idx - e * Lnew);
-            dst[(size_t)e * cap + d] = d >= s ? src[(size_t)e * cap + d - s] : 0;
-        }
-        return;
-    }
-    __shared__ int piv[kMaxM], rinfo[kMaxM];
-    piv[tx] = piv_t;
-    rinfo[tx] = rinfo_t;
-    __syncthreads();
-    // D: the kernel vectors' own coefficient (the step's pivot product)
-    auto own = [&](uint64_t x) -> uint64_t {
-        if constexpr (SMALL)  // D in Montgomery form: REDC(x D 2^32) = x D mod p
-            return Mont32Arith(a.mc).redc((uint64_t)(uint32_t)x * (uint32_t)D);
-        else
-            return mulmod_g(x, D, a.mc);
+    size_t most = 0;
+    for (int r = 1; r <= std::min(m, n); ++r)
+        most = std::max(most, (size_t)(m - r) * pad16(r));
+    return most;
+}
+template <typename Arith, bool STAGE>
+__global__ void __launch_bounds__(kUpdateThreads)
+mbasis_update_kernel(LeafArgs a, int ord0, int w, int wnext, int tilesB, int tilesR)
+{
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    using V = typename Arith::V;
+    static_assert(kMaxM <= kUpdateThreads, "one row-list entry per thread");
+    const int m = a.m, n = a.n;
+    const int tid = threadIdx.x, lane = tid & 63;
+    V *Y = reinterpret_cast<V *>(smem);              // m x kTile
+    int *pl = reinterpret_cast<int *>(Y + m * kTile);  // kWindow x m: row lists
+    int *del = pl + kWindow * m;                     // m
+    V *Xs = reinterpret_cast<V *>(smem + update_lds_bytes(m, sizeof(V)));  // STAGE: vectors by order
+    const int q = tid % kTile, tg = tid / kTile;
+    constexpr int TG = kUpdateThreads / kTile;
+    // STAGE: 2 x 2 entries per thread of 2 TG rows x 2 kTile entries of every
+    // order's vectors, all of them in flight at once; entry e of row t (in X's
+    // bounds whatever the rank, which the first ones do not wait for)
+    constexpr int XR = 2 * TG, XE = 2 * kTile;
+    V xv[STAGE ? kWindow : 1][2][2];
+    auto fetch = [&](int tb, int eb) {
+#pragma unroll
+        for (int s = 0; s < kWindow; ++s)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int t = tb + tg + (u >> 1) * TG, e = eb + q + (u & 1) * kTile;
+                const size_t x = (size_t)(s < w ? s : 0) * m * m + (t < m ? t : 0) * m + (e < m ? e : 0);
+                xv[s][u >> 1][u & 1] = reinterpret_cast<const V *>(a.X)[x];
+            }
     };
-    const unsigned L1 = (unsigned)(L + 1 <= cap ? L + 1 : cap);
-    const unsigned items = (unsigned)(m * m) * L1;
-    // residual series: coefficients ord+1 .. ordL-1
-    const uint64_t *rs = a.R[cur];
-    uint64_t *rd = a.R[cur ^ 1];
-    const int spn = a.ordL - ord - 1;
-    const unsigned span = spn > 0 ? (unsigned)spn : 0u;
-    const unsigned ritems = (unsigned)(m * n) * span;
-    // one index space, basis items then residual items: with the grid sized
-    // for both, a thread has one item
-    for (unsigned idx = t0; idx < items + ritems; idx += tstride) {
-        if (idx < items) {
-            const unsigned e = idx / L1;
-            const int d = (int)(idx - e * L1);
-            const int i = (int)(e / (unsigned)m), j = (int)(e - (unsigned)i * m);
-            const int ri = rinfo[i];
-            uint64_t v;
-            if (ri >= 0) {
-                v = d < L ? row_combo<SMALL, BIG>(src, a, piv, ri, rank, cap, m, j, d, own(src[(size_t)e * cap + d]))
-                          : 0;
-            } else {
-                v = d >= 1 ? src[(size_t)e * cap + d - 1] : 0;
-                if (d == L && v != 0)
-                    atomicOr(&a.ctl[C_GROW], 1);
-            }
-            dst[(size_t)e * cap + d] = v;
-        } else {
-            const unsigned k = idx - items;
-            const unsigned e = k / span;
-            const int d = ord + 1 + (int)(k - e * span);
-            const int i = (int)(e / (unsigned)n), j = (int)(e - (unsigned)i * n);
-            const int ri = rinfo[i];
-            const uint64_t v =
-                ri >= 0 ? row_combo<SMALL, BIG>(rs, a, piv, ri, rank, a.ordL, n, j, d, own(rs[(size_t)e * a.ordL + d]))
-                        : rs[(size_t)e * a.ordL + d - 1];
-            rd[(size_t)e * a.ordL + d] = v;
-            if (d == ord + 1)
-                a.Rn[e] = v;  // the coming step's coefficient
+    if constexpr (STAGE)
+        fetch(0, 0);
+    const int steps = a.ctl[C_STEPS], cur = a.ctl[C_CUR], len = a.ctl[C_LEN];
+    int ranks[kWindow];
+    V D[kWindow];
+#pragma unroll
+    for (int s = 0; s < kWindow; ++s) {
+        ranks[s] = a.ctl[C_RANK + s];
+        D[s] = (V)a.scale[m + s];
+    }
+    // row lists of the window (orders past `steps` are not used)
+    if (tid < m) {
+#pragma unroll
+        for (int s = 0; s < kWindow; ++s)
+            pl[s * m + tid] = a.piv[s * m + tid];
+        del[tid] = 0;
+    }
+    if (steps == 0)
+        return;
+    const bool basis = (int)blockIdx.x < m * tilesB;
+    const int b = basis ? blockIdx.x : blockIdx.x - m * tilesB;
+    const int tiles = basis ? tilesB : tilesR;
+    const int j = b / tiles, tile = b - j * tiles;
+    const int cols = basis ? m : n;
+    const int stride = basis ? a.cap : a.ordL;
+    const int out = kTile - w;  // coefficients a tile writes
+    const int d0 = (basis ? 0 : ord0 + w) + tile * out;
+    // coefficients read, and written
+    const int lin = basis ? len : a.ordL;
+    const int lout = basis ? (len + steps < a.cap ? len + steps : a.cap) : a.ordL;
+    if (d0 >= lout)
+        return;
+    const uint64_t *src = basis ? a.app[cur] : a.R[cur];
+    uint64_t *dst = basis ? a.app[cur ^ 1] : a.R[cur ^ 1];
+    const Arith ar(a.mc);
+    {
+        // (four rows' loads in flight, of an entry that exists in any case)
+        const int d = d0 - w + q;
+        const bool in = d >= 0 && d < lin;
+        const uint64_t *from = src + (size_t)j * stride + (in ? d : 0);
+        const size_t rows = (size_t)cols * stride;
+        for (int i0 = tg; i0 < m; i0 += 4 * TG) {
+            V y[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                y[u] = Arith::load(from + (i0 + u * TG < m ? i0 + u * TG : 0) * rows);
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (i0 + u * TG < m)
+                    Y[(i0 + u * TG) * kTile + q] = in ? y[u] : (V)0;
         }
+    }
+    if constexpr (STAGE) {
+        int most = 0;  // entries of the longest vectors
+#pragma unroll
+        for (int s = 0; s < kWindow; ++s) {
+            ranks[s] = s < steps ? ranks[s] : 0;
+            most = ranks[s] > most ? ranks[s] : most;
+        }
+        for (int tb = 0; tb < m; tb += XR)
+            for (int eb = 0; eb < most; eb += XE) {
+                if (tb + eb > 0)
+                    fetch(tb, eb);
+                V *xs = Xs;
+#pragma unroll
+                for (int s = 0; s < kWindow; ++s) {
+                    const int rank = ranks[s], nullity = m - rank, r16 = pad16(rank);
+                    if (rank == 0)
+                        continue;
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        const int t = tb + tg + (u >> 1) * TG, e = eb + q + (u & 1) * kTile;
+                        if (t < nullity && e < r16)
+                            xs[t * r16 + e] = e < rank ? xv[s][u >> 1][u & 1] : (V)0;
+                    }
+                    xs += nullity * r16;
+                }
+            }
+    }
+    __syncthreads();
+    const int tw = __builtin_amdgcn_readfirstlane(tg);  // the wave's first
+    struct alignas(16) Group {
+        V v[kGroup];
+    };
+    constexpr int RH = kMaxN / 64;
+    int top = 0;  // length that a row multiplied by x reaches
+    const V *xstage = Xs;
+    for (int s = 0; s < steps; ++s) {
+        int rank = 0;
+        V Ds = 0;
+#pragma unroll
+        for (int u = 0; u < kWindow; ++u) {
+            rank = u == s ? ranks[u] : rank;
+            Ds = u == s ? D[u] : Ds;
+        }
+        if (rank == 0)
+            continue;  // zero residual: nothing to do at this order
+        const int *ps = pl + s * m;
+        const int nullity = m - rank;
+        const V *X = STAGE ? xstage : reinterpret_cast<const V *>(a.X) + (size_t)s * m * m;
+        const int xstride = STAGE ? pad16(rank) : m;
+        // places of the pivot rows' coefficient q = 0, lane r for pivot r (past
+        // the rank: the first row, with zero entries in the vectors)
+        int ybase[RH];
+#pragma unroll
+        for (int h = 0; h < RH; ++h) {
+            const int i = ps[lane + 64 * h < rank ? lane + 64 * h : 0];
+            ybase[h] = i * kTile - del[i];
+        }
+        // (a wave takes every round as a whole, its lanes read each other's ybase)
+        for (int t0 = tw; t0 < nullity; t0 += TG) {
+            const int t = t0 + tg - tw < nullity ? t0 + tg - tw : t0;
+            // (q below s: coefficients already undefined, read as q = s)
+            const int qq = q < s ? s : q, i = ps[rank + t];
+            V *own = Y + i * kTile + qq - del[i];
+            const V *x = X + (size_t)t * xstride;
+            V sum = ar.mul(Ds, *own);
+#pragma unroll
+            for (int h = 0; h < RH; ++h)
+                for (int r0 = 0; r0 < 64 && r0 + 64 * h < rank; r0 += kGroup) {
+                    V v[kGroup], c[kGroup];
+                    if constexpr (STAGE)
+                        *reinterpret_cast<Group *>(c) = *reinterpret_cast<const Group *>(x + r0 + 64 * h);
+#pragma unroll
+                    for (int u = 0; u < kGroup; ++u) {
+                        const int r = r0 + u + 64 * h;
+                        v[u] = Y[__builtin_amdgcn_readlane(ybase[h], r0 + u) + qq];
+                        if constexpr (!STAGE)  // (past the row's end: within X's padding)
+                            c[u] = r < rank ? x[r] : (V)0;
+                    }
+                    // two chains of eight products, the most one reduction takes
+                    typename Arith::Acc p1 = ar.prod(c[0], v[0]), p2 = ar.prod(c[8], v[8]);
+#pragma unroll
+                    for (int u = 1; u < 8; ++u) {
+                        p1 = ar.fma(p1, c[u], v[u]);
+                        p2 = ar.fma(p2, c[8 + u], v[8 + u]);
+                    }
+                    sum = ar.add(sum, ar.add(ar.reduce(p1), ar.reduce(p2)));
+                }
+            if (q >= s)
+                *own = sum;  // (t = t0 twice: the same value again)
+        }
+        xstage += nullity * pad16(rank);
+        __syncthreads();
+        if (tid < rank)
+            del[ps[tid]] += 1;
+        __syncthreads();
+        // length: a row multiplied by x with a coefficient past the old one
+        if (basis && d0 + out > len && q > s) {
+            const int d = d0 - w + q;
+            if (d >= len)
+                for (int r = tg; r < rank; r += TG) {
+                    const int i = ps[r];
+                    if (Y[i * kTile + q - del[i]] != 0)
+                        top = d + 1;
+                }
+        }
+    }
+    __syncthreads();
+    if (basis && d0 + out > len) {
+        for (int d = 32; d > 0; d >>= 1)
+            top = max(top, __shfl_xor(top, d));
+        if (lane == 0)
+            del[m + tid / 64] = top;
+        __syncthreads();
+        if (tid == 0) {
+            for (int k = 0; k < kUpdateThreads / 64; ++k)
+                top = max(top, del[m + k]);
+            if (top > len)  // (at most two tiles of a column reach past len)
+                a.lens[2 * j + (tile & 1)] = top;
+        }
+    }
+    for (int idx = tid; idx < m * kTile; idx += kUpdateThreads) {
+        const int i = idx / kTile, qq = idx % kTile, d = d0 - w + qq;
+        if (qq < w || d >= lout)
+            continue;
+        const uint64_t v = Y[i * kTile + qq - del[i]];
+        const size_t e = (size_t)i * cols + j;
+        dst[e * stride + d] = v;
+        if (!basis && d < ord0 + w + wnext)
+            a.Rn[(size_t)(d - ord0 - w) * m * n + e] = v;  // the coming window
+    }
+}
+
+// appbas <- x^s appbas (entries of capacity cap, length len before), into dst
+__global__ void leaf_shift_kernel(uint64_t *__restrict__ dst, const uint64_t *__restrict__ src, int64_t cap,
+                                  int64_t entries, int64_t len, int64_t s)
+{
+    const int64_t items = entries * (len + s);
+    for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < items;
+         idx += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t e = idx / (len + s), d = idx - e * (len + s);
+        dst[e * cap + d] = d >= s ? src[e * cap + d - s] : 0;
     }
 }
 
@@ -1219,7 +1691,7 @@ __global__ void __launch_bounds__(256) leaf_rescale_kernel(uint64_t *__restrict_
 
 // appbas <- identity (capacity cap), R <- F truncated to ordL, control reset
 __global__ void leaf_init_kernel(LeafArgs a, const uint64_t *__restrict__ F, int64_t strideF,
-                                 int64_t lenF)
+                                 int64_t lenF, int w)
 {
     const int m = a.m, n = a.n, cap = a.cap;
     const int64_t tstride = (int64_t)gridDim.x * blockDim.x;
@@ -1237,11 +1709,11 @@ __global__ void leaf_init_kernel(LeafArgs a, const uint64_t *__restrict__ F, int
         const int d = (int)(idx - e * a.ordL);
         const uint64_t v = d < lenF ? F[e * strideF + d] : 0;
         a.R[0][idx] = v;
-        if (d == 0)
-            a.Rn[e] = v;
+        if (d < w)
+            a.Rn[(size_t)d * m * n + e] = v;
     }
-    if (t0 < C_WORDS)
-        a.ctl[t0] = (t0 == C_LEN) ? 1 : 0;
+    for (int64_t idx = t0; idx < C_WORDS + 2 * m; idx += tstride)  // ctl, lens
+        a.ctl[idx] = idx == C_LEN ? 1 : 0;
 }
 
 // copies an m x m x L block between two capacities (entry-major)
@@ -1256,6 +1728,11 @@ __global__ void copy_poly_kernel(uint64_t *__restrict__ dst, int64_t dcap,
         dst[e * dcap + d] = src[e * scap + d];
     }
 }
+
+template <typename T>
+struct Tag {
+    using type = T;
+};
 
 unsigned grid_for(int64_t items)
 {
@@ -1306,81 +1783,90 @@ pmlg_status leaf(pmlg_ctx ctx, Arena &ar, const uint64_t *F, int64_t strideF, in
     a.app[1] = ar.alloc((size_t)m * m * cap);
     a.R[0] = ar.alloc((size_t)m * n * (ordL > 0 ? ordL : 1));
     a.R[1] = ar.alloc((size_t)m * n * (ordL > 0 ? ordL : 1));
-    a.Rn = ar.alloc((size_t)m * n);
-    a.scale = ar.alloc((size_t)m + 1);
-    a.X = ar.alloc((size_t)m * m + kXPad);
-    uint64_t *ints = ar.alloc((size_t)m + C_WORDS + 8);
+    // p = 2 has no Montgomery form (p must be odd): plain residues as for p >= 2^62
+    const bool big = ctx->p >= ((uint64_t)1 << 62) || ctx->p == 2;
+    const bool small = !big && ctx->p < ((uint64_t)1 << 30);
+    const size_t wbytes = small ? 4 : 8;
+    if (step_lds_bytes(m, n, wbytes) > kStepLdsMax)
+        return fail(PMLG_ERR_UNSUPPORTED, "M-Basis: an m x n residual of this size does not fit "
+                                          "the step kernel's LDS");
+    const int W = window_orders(m, n, wbytes);
+    a.Rn = ar.alloc((size_t)m * n * W);
+    a.scale = ar.alloc((size_t)m + kWindow);
+    a.X = ar.alloc((size_t)m * m * W + kXPad);
+    uint64_t *ints = ar.alloc(((size_t)m * (kWindow + 2) + C_WORDS) / 2 + 8);
     if (!a.app[0] || !a.app[1] || !a.R[0] || !a.R[1] || !a.Rn || !a.scale || !a.X || !ints)
         return fail(PMLG_ERR_ALLOC, "pmbasis: device arena exhausted");
-    a.piv = reinterpret_cast<int *>(ints);
-    a.rowinfo = a.piv + m;
-    a.ctl = a.rowinfo + m;
+    a.ctl = reinterpret_cast<int *>(ints);
+    a.lens = a.ctl + C_WORDS;
+    a.piv = a.lens + 2 * m;
     a.shift = dShift;
     a.mc = ctx->mc;
     const int64_t lt = lenF < ordL ? lenF : ordL;
     hipLaunchKernelGGL(leaf_init_kernel, dim3(grid_for((int64_t)m * m * cap + (int64_t)m * n * ordL)),
-                       dim3(256), 0, s, a, F, strideF, lt);
+                       dim3(256), 0, s, a, F, strideF, lt, W);
     HIP_TRY(hipGetLastError(), "leaf_init_kernel");
-    // p = 2 has no Montgomery form (p must be odd): plain residues as for p >= 2^62
-    const bool big = ctx->p >= ((uint64_t)1 << 62) || ctx->p == 2;
-    const bool small = !big && ctx->p < ((uint64_t)1 << 30);
-    const size_t lds = step_lds_bytes(m, n, small ? 4 : 8);
-    if (lds > kStepLdsMax)
-        return fail(PMLG_ERR_UNSUPPORTED, "M-Basis: an m x n residual of this size does not fit "
-                                          "the step kernel's LDS");
     static bool attr = false;
     if (!attr) {
-        const int maxlds = (int)kStepLdsMax;
         const void *kernels[] = {(const void *)mbasis_step_kernel<Mont64Arith, 1>,
                                  (const void *)mbasis_step_kernel<Mont64Arith, 2>,
                                  (const void *)mbasis_step_kernel<Mont32Arith, 1>,
                                  (const void *)mbasis_step_kernel<Mont32Arith, 2>,
                                  (const void *)mbasis_step_kernel<BigArith, 1>,
-                                 (const void *)mbasis_step_kernel<BigArith, 2>};
+                                 (const void *)mbasis_step_kernel<BigArith, 2>,
+                                 (const void *)mbasis_update_kernel<Mont64Arith, true>,
+                                 (const void *)mbasis_update_kernel<Mont32Arith, true>,
+                                 (const void *)mbasis_update_kernel<BigArith, true>};
         for (const void *k : kernels)
-            HIP_TRY(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, maxlds),
-                    "hipFuncSetAttribute(mbasis_step_kernel)");
+            HIP_TRY(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLds),
+                    "hipFuncSetAttribute(mbasis kernels)");
         attr = true;
     }
-    const unsigned ugrid = grid_for((int64_t)m * m * cap + (int64_t)m * n * ordL);
     // rows of the transposed residual per lane of the composing wave
     const bool one_row = n <= 64;
-    for (int ord = 0; ord < ordL; ++ord) {
-        if (small) {
-            if (one_row)
-                hipLaunchKernelGGL((mbasis_step_kernel<Mont32Arith, 1>), dim3(1), dim3(kStepThreads), lds,
-                                   s, a, ord);
-            else
-                hipLaunchKernelGGL((mbasis_step_kernel<Mont32Arith, 2>), dim3(1), dim3(kStepThreads), lds,
-                                   s, a, ord);
-            hipLaunchKernelGGL((mbasis_update_kernel<true, false>), dim3(ugrid), dim3(256), 0, s, a,
-                               ord);
-        } else if (big) {
-            if (one_row)
-                hipLaunchKernelGGL((mbasis_step_kernel<BigArith, 1>), dim3(1), dim3(kStepThreads), lds,
-                                   s, a, ord);
-            else
-                hipLaunchKernelGGL((mbasis_step_kernel<BigArith, 2>), dim3(1), dim3(kStepThreads), lds,
-                                   s, a, ord);
-            hipLaunchKernelGGL((mbasis_update_kernel<false, true>), dim3(ugrid), dim3(256), 0, s, a,
-                               ord);
-        } else {
-            if (one_row)
-                hipLaunchKernelGGL((mbasis_step_kernel<Mont64Arith, 1>), dim3(1), dim3(kStepThreads), lds,
-                                   s, a, ord);
-            else
-                hipLaunchKernelGGL((mbasis_step_kernel<Mont64Arith, 2>), dim3(1), dim3(kStepThreads), lds,
-                                   s, a, ord);
-            hipLaunchKernelGGL((mbasis_update_kernel<false, false>), dim3(ugrid), dim3(256), 0, s, a,
-                               ord);
-        }
+    const size_t xbytes = staged_words(m, n) * W * wbytes;
+    const bool stage = update_lds_bytes(m, wbytes) + xbytes <= kLds;
+    const size_t ulds = update_lds_bytes(m, wbytes) + (stage ? xbytes : 0);
+    for (int ord = 0; ord < ordL; ord += W) {
+        const int w = std::min(W, ordL - ord), wnext = std::min(W, ordL - ord - w);
+        const size_t lds = window_lds_bytes(m, n, w, wbytes);
+        // tiles of appbas (length at most ord + w + 1 after the window) and of
+        // the residual's later coefficients
+        const int out = kTile - w;
+        const int tilesB = (std::min(cap, ord + w + 1) + out - 1) / out;
+        const int tilesR = (std::max(ordL - ord - w, 0) + out - 1) / out;
+        const dim3 ugrid((unsigned)(m * tilesB + n * tilesR));
+        auto launch = [&](auto arith) {
+            using A = decltype(arith);
+            hipLaunchKernelGGL((one_row ? mbasis_step_kernel<typename A::type, 1>
+                                        : mbasis_step_kernel<typename A::type, 2>),
+                               dim3(1), dim3(kStepThreads), lds, s, a, ord, w);
+            hipLaunchKernelGGL((stage ? mbasis_update_kernel<typename A::type, true>
+                                      : mbasis_update_kernel<typename A::type, false>),
+                               ugrid, dim3(kUpdateThreads), ulds, s, a, ord, w, wnext, tilesB, tilesR);
+        };
+        if (small)
+            launch(Tag<Mont32Arith>{});
+        else if (big)
+            launch(Tag<BigArith>{});
+        else
+            launch(Tag<Mont64Arith>{});
     }
     HIP_TRY(hipGetLastError(), "mbasis kernels");
-    int ctl[C_WORDS];
-    HIP_TRY(hipMemcpyAsync(ctl, a.ctl, sizeof(ctl), hipMemcpyDeviceToHost, s), "D2H(ctl)");
+    int ctl[C_WORDS + 2 * kMaxM];  // the lengths as well
+    HIP_TRY(hipMemcpyAsync(ctl, a.ctl, (C_WORDS + 2 * m) * sizeof(int), hipMemcpyDeviceToHost, s), "D2H(ctl)");
     HIP_TRY(hipStreamSynchronize(s), "leaf sync");
-    const int res = ctl[C_CUR] ^ ctl[C_FLIP];
-    const int L = ctl[C_LEN] + ctl[C_GROW];
+    int res = ctl[C_CUR] ^ ctl[C_FLIP];
+    int L = std::max(1, *std::max_element(ctl + C_WORDS, ctl + C_WORDS + 2 * m));
+    if (ctl[C_DONE]) {
+        // full-rank residual met: the basis times the rest of the power of x
+        const int sft = ctl[C_SHIFT];
+        hipLaunchKernelGGL(leaf_shift_kernel, dim3(grid_for((int64_t)m * m * (L + sft))), dim3(256), 0, s,
+                           a.app[res ^ 1], a.app[res], (int64_t)cap, (int64_t)m * m, (int64_t)L, (int64_t)sft);
+        HIP_TRY(hipGetLastError(), "leaf_shift_kernel");
+        res ^= 1;
+        L += sft;
+    }
     if (ordL > 0) {
         // divide the row scales out of the basis
         if (small)
@@ -1458,7 +1944,8 @@ size_t arena_bytes(int64_t m, int64_t n, int64_t order, int64_t ordleaf)
     // generous bound: a few copies of every level's operands
     const double lvl = (double)m * m * (order + 2) * 4 + (double)m * n * (order + 1) * 2;
     const double leafb =
-        (double)m * m * (ordleaf + 2) * 2 + (double)m * n * (ordleaf + 2) * 2 + m * m + 64;
+        (double)m * m * (ordleaf + 2) * 2 + (double)m * n * (ordleaf + 2) * 2 +
+        (double)kWindow * (m * m + m * n + m) + 256;
     return (size_t)((2.5 * lvl + leafb + 4096.0) * 8.0);
 }
 
