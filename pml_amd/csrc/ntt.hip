@@ -46,10 +46,56 @@ __device__ __forceinline__ int64_t xcd_unit(int64_t b, int64_t units)
     return (units & 7) ? b : (b & 7) * (units >> 3) + (b >> 3);
 }
 
+// a b + c mod 2^64 as one instruction (mad32s: b uniform)
+__device__ __forceinline__ uint64_t mad32(uint32_t a, uint32_t b, uint64_t c)
+{
+    uint64_t r, carry;
+    asm("v_mad_u64_u32 %0, %1, %2, %3, %4" : "=v"(r), "=s"(carry) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+__device__ __forceinline__ uint64_t mad32s(uint32_t a, uint32_t b, uint64_t c)
+{
+    uint64_t r, carry;
+    asm("v_mad_u64_u32 %0, %1, %2, %3, %4" : "=v"(r), "=s"(carry) : "v"(a), "s"(b), "v"(c));
+    return r;
+}
+
+// x w + q n mod 2^64 (n uniform), the second half of every Shoup product, as 7
+// instructions: the four products that only count in the upper word are one
+// chain of multiply-adds.  Left to the compiler it comes out as 11, with 8
+// products and copies between register pairs.  A vector instruction costs about
+// 4.7 cycles whatever it is, but for a plain 32-bit add or copy, and a radix-2
+// butterfly on 64-bit words went from 96 to 85 cycles (two waves per SIMD).
+__device__ __forceinline__ uint64_t muladd2(uint64_t x, uint64_t w, uint64_t q, uint64_t n)
+{
+    const uint32_t x0 = (uint32_t)x, x1 = (uint32_t)(x >> 32), w0 = (uint32_t)w, w1 = (uint32_t)(w >> 32);
+    const uint32_t q0 = (uint32_t)q, q1 = (uint32_t)(q >> 32), n0 = (uint32_t)n, n1 = (uint32_t)(n >> 32);
+    const uint64_t h = mad32s(q1, n0, mad32s(q0, n1, mad32(x1, w0, (uint64_t)x0 * w1)));
+    const uint64_t r = mad32s(q0, n0, (uint64_t)x0 * w0);
+    uint32_t rh;  // (left to the compiler: a 64-bit add of h << 32)
+    asm("v_add_u32 %0, %1, %2" : "=v"(rh) : "v"((uint32_t)(r >> 32)), "v"((uint32_t)h));
+    return ((uint64_t)rh << 32) | (uint32_t)r;
+}
+
+// x w mod p in [0, 2p) and in [0, p) for any word x (p uniform)
+__device__ __forceinline__ uint64_t shoup2(uint64_t x, uint64_t w, uint64_t wq, uint64_t p)
+{
+    return muladd2(x, w, mulhi64(x, wq), (uint64_t)0 - p);
+}
+__device__ __forceinline__ uint32_t shoup2(uint32_t x, uint32_t w, uint32_t wq, uint32_t p)
+{
+    return shoup_lazy(x, w, wq, p);
+}
+template <typename W>
+__device__ __forceinline__ W shoup1(W x, W w, W wq, W p)
+{
+    return reduce_2p<W>(shoup2(x, w, wq, p), p);
+}
+
 template <typename W>
 __device__ __forceinline__ W tw_mul(W x, const W *w, const W *wq, int64_t idx, W p)
 {
-    return shoup_lazy(x, w[idx], wq[idx], p);
+    return shoup2(x, w[idx], wq[idx], p);
 }
 
 // The last two inverse stages of a 3/4-truncated product.  The forward's
@@ -67,16 +113,16 @@ template <typename W>
 __device__ __forceinline__ void trunc_solve(W &y0, W &y1, W &y2, int64_t i, const NttTab<W> &tab,
                                             W p)
 {
-    const W a = reduce_2p<W>(shoup_lazy(y0, tab.itw[0], tab.itwq[0], p), p);
-    const W u = reduce_2p<W>(shoup_lazy(y1, tab.itw[2 * i], tab.itwq[2 * i], p), p);
-    const W v = reduce_2p<W>(shoup_lazy(y2, tab.itw[i], tab.itwq[i], p), p);
+    const W a = reduce_2p<W>(shoup2(y0, tab.itw[0], tab.itwq[0], p), p);
+    const W u = reduce_2p<W>(shoup2(y1, tab.itw[2 * i], tab.itwq[2 * i], p), p);
+    const W v = reduce_2p<W>(shoup2(y2, tab.itw[i], tab.itwq[i], p), p);
     const W d = a >= u ? a - u : a + (p - u);
     W su = a + u;
     su = su >= p ? su - p : su;
-    const W x1 = shoup<W>(d, tab.ninv2, tab.ninv2q, p);
-    const W S = shoup<W>(su, tab.ninv, tab.ninvq, p);
-    const W D = shoup<W>(v, tab.ninv2, tab.ninv2q, p);
-    const W h = shoup<W>(x1, tab.thalf, tab.thalfq, p);
+    const W x1 = shoup1(d, tab.ninv2, tab.ninv2q, p);
+    const W S = shoup1(su, tab.ninv, tab.ninvq, p);
+    const W D = shoup1(v, tab.ninv2, tab.ninv2q, p);
+    const W h = shoup1(x1, tab.thalf, tab.thalfq, p);
     W sd = S + D;
     sd = sd >= p ? sd - p : sd;
     W md = S >= D ? S - D : S + (p - D);
@@ -95,7 +141,7 @@ __device__ __forceinline__ void trunc_solve(W &y0, W &y1, W &y2, int64_t i, cons
 template <typename W>
 __device__ __forceinline__ void trunc_correct(W &c0, W &c1, W &c2, W c3, const NttTab<W> &tab, W p)
 {
-    const W sc = shoup<W>(c3, tab.tquart, tab.tquartq, p);
+    const W sc = shoup1(c3, tab.tquart, tab.tquartq, p);
     c0 = c0 >= sc ? c0 - sc : c0 + (p - sc);
     c1 = c1 + c3;
     c1 = c1 >= p ? c1 - p : c1;
@@ -125,7 +171,7 @@ __device__ __forceinline__ void merge_one(const W *__restrict__ z, Wout *__restr
         const int64_t widx = (o * g) & (N - 1);
         acc = add_2p<W>(acc, tw_mul<W>(ze[(int64_t)g * M + i1], tab.itw, tab.itwq, widx, p), p2);
     }
-    out[e * out_stride + (o - lo)] = (Wout)shoup<W>(acc, tab.ninv, tab.ninvq, p);
+    out[e * out_stride + (o - lo)] = (Wout)shoup1(acc, tab.ninv, tab.ninvq, p);
 }
 
 // Merge of a truncated product split in four (N = 4M, the sub-transform of
@@ -331,13 +377,7 @@ __device__ __forceinline__ uint64_t shoup4(uint64_t x, uint64_t w, uint64_t wq, 
     const uint32_t ql = (uint32_t)wq, qh = (uint32_t)(wq >> 32);
     uint64_t q = (uint64_t)xh * qh + __umulhi(xl, qh);
     q += __umulhi(xh, ql);
-    const uint32_t q0 = (uint32_t)q, q1 = (uint32_t)(q >> 32);
-    const uint32_t w0 = (uint32_t)w, w1 = (uint32_t)(w >> 32);
-    const uint32_t n0 = (uint32_t)np, n1 = (uint32_t)(np >> 32);
-    uint64_t r = (uint64_t)xl * w0;
-    r += (uint64_t)q0 * n0;
-    const uint32_t hi = (uint32_t)(r >> 32) + xl * w1 + xh * w0 + q0 * n1 + q1 * n0;
-    return ((uint64_t)hi << 32) | (uint32_t)r;
+    return muladd2(x, w, q, np);
 }
 
 // Lazy forward rule.  Bound (in multiples of p) of register j of a forward
@@ -415,7 +455,7 @@ __device__ __forceinline__ void bfly_dif_strict(W &a, W &c, W w, W wq, const Bfl
 {
     const W u = a, v = c;
     a = add_2p<W>(u, v, k.p2);
-    c = shoup_lazy(sub_2p<W>(u, v, k.p2), w, wq, k.p);
+    c = shoup2(sub_2p<W>(u, v, k.p2), w, wq, k.p);
 }
 
 template <typename W>
@@ -431,7 +471,7 @@ template <typename W>
 __device__ __forceinline__ void bfly_dit_strict(W &a, W &c, W w, W wq, const Bfly<W> &k)
 {
     const W u = a;
-    const W v = shoup_lazy(c, w, wq, k.p);
+    const W v = shoup2(c, w, wq, k.p);
     a = add_2p<W>(u, v, k.p2);
     const W d = u + k.p2 - v;
     c = d >= k.p2 ? d - k.p2 : d;
@@ -594,7 +634,7 @@ __device__ __forceinline__ void fwd_half_pairs(W (&x)[1 << LOGE],
         else if constexpr (LOOSE)
             c = shoup4(a, w, wq, k.np);
         else
-            c = shoup_lazy(a, w, wq, k.p);
+            c = shoup2(a, w, wq, k.p);
     }
     if constexpr (J + 1 < (1 << LB))
         fwd_half_pairs<W, LOOSE, L, LOGE, J + 1>(x, tw, k);
@@ -738,6 +778,43 @@ __device__ __forceinline__ void store_words(W *dst, const W *v)
     }
 }
 
+// value of the even (ODD false) or odd lane of each pair of lanes
+template <bool ODD>
+__device__ __forceinline__ uint32_t pair_lane(uint32_t v)
+{
+    // quad_perm [0, 0, 2, 2] or [1, 1, 3, 3]
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, ODD ? 0xF5 : 0xA0, 0xF, 0xF, true);
+}
+template <bool ODD>
+__device__ __forceinline__ uint64_t pair_lane(uint64_t v)
+{
+    return ((uint64_t)pair_lane<ODD>((uint32_t)(v >> 32)) << 32) | pair_lane<ODD>((uint32_t)v);
+}
+
+// 32 bytes of each lane of a pair, the even lane's to `even` and the odd one's
+// to `odd`: each of the two stores writes one lane's 32 bytes, a half by
+// either lane, as one request to L2.  Lanes that store their own halves one
+// after the other make four requests of 16 bytes, and it is the number of
+// requests that bounds these stores (the lanes' places are far apart): forward
+// transforms took 108 us, now 96 (2048 of length 8192, 64-bit words; 68 without
+// any memory access), 200 -> 170 (32768 of length 1024), 41 -> 35.5 (6144 of
+// length 2048, 32-bit words).
+template <typename W>
+__device__ __forceinline__ void store_pair(W *even, W *odd, const W *v)
+{
+    constexpr int PER = 16 / sizeof(W);
+    const bool o = threadIdx.x & 1;
+    W a[PER], b[PER];
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+        const W hi = pair_lane<false>(v[PER + q]), lo = pair_lane<true>(v[q]);
+        a[q] = o ? hi : v[q];
+        b[q] = o ? v[PER + q] : lo;
+    }
+    store_words<W, PER>(even + (o ? PER : 0), a);
+    store_words<W, PER>(odd + (o ? PER : 0), b);
+}
+
 template <typename W, int CNT>
 __device__ __forceinline__ void load_words(const W *src, W *v)
 {
@@ -760,6 +837,25 @@ __device__ __forceinline__ void load_words(const W *src, W *v)
 #pragma unroll
         for (int j = 0; j < CNT; ++j)
             v[j] = src[j];
+    }
+}
+
+// the converse: 32 bytes of each lane of a pair from `even` and `odd`
+// (inverse transforms, 16384 of length 1024: 109 -> 101 us; 2048 of length
+// 2048, 32-bit words: 19.2 -> 17.1)
+template <typename W>
+__device__ __forceinline__ void load_pair(const W *even, const W *odd, W *v)
+{
+    constexpr int PER = 16 / sizeof(W);
+    const bool o = threadIdx.x & 1;
+    W a[PER], b[PER];
+    load_words<W, PER>(even + (o ? PER : 0), a);
+    load_words<W, PER>(odd + (o ? PER : 0), b);
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+        const W hi = pair_lane<true>(a[q]), lo = pair_lane<false>(b[q]);
+        v[q] = o ? lo : a[q];
+        v[PER + q] = o ? b[q] : hi;
     }
 }
 
@@ -928,7 +1024,19 @@ __device__ __forceinline__ void fwd_reg_body(const Win *__restrict__ in, int64_t
             continue;
         W y[RUN];
         fwd_final<W, LOOSE, LOGE, PSL::R, fwd_last_b0<L, LOGE>(2), 0>(x, g * RUN, y, k);
-        if (logP >= 2) {
+        // (a pair's runs lie in one quarter, both kept or neither)
+        constexpr int BLOCK = 32 / sizeof(W);
+        // (the radix-16 kernels with the split step have no registers left for it)
+        constexpr bool PAIRS = RUN >= BLOCK && PSL::R < L - 2 && !(MODE == kSplit && LOGE == 4);
+        if (PAIRS && logP >= (sizeof(W) == 8 ? 2 : 3)) {
+            if constexpr (PAIRS) {
+#pragma unroll
+                for (int j0 = 0; j0 < RUN; j0 += BLOCK)
+                    store_pair<W>(out + blk_addr(e, (int64_t)gg * M + PSL::index(t & ~1, g, j0), count, logP),
+                                  out + blk_addr(e, (int64_t)gg * M + PSL::index(t | 1, g, j0), count, logP),
+                                  y + j0);
+            }
+        } else if (logP >= 2) {
 #pragma unroll
             for (int j0 = 0; j0 < RUN; j0 += VEC)
                 store_words<W, VEC>(out + blk_addr(e, (int64_t)gg * M + PSL::index(t, g, j0), count,
@@ -1032,7 +1140,17 @@ __device__ __forceinline__ void inv_reg_body(const W *__restrict__ in, Wout *__r
                 x[g * RUN + j] = 0;
             continue;
         }
-        if (logP >= 2) {
+        constexpr int BLOCK = 32 / sizeof(W);
+        constexpr bool PAIRS = RUN >= BLOCK && PSF::R < L - 2;
+        if (PAIRS && logP >= (sizeof(W) == 8 ? 2 : 3)) {
+            if constexpr (PAIRS) {
+#pragma unroll
+                for (int j0 = 0; j0 < RUN; j0 += BLOCK)
+                    load_pair<W>(in + blk_addr(e, (int64_t)gg * M + PSF::index(t & ~1, g, j0), count, logP),
+                                 in + blk_addr(e, (int64_t)gg * M + PSF::index(t | 1, g, j0), count, logP),
+                                 x + g * RUN + j0);
+            }
+        } else if (logP >= 2) {
 #pragma unroll
             for (int j0 = 0; j0 < RUN; j0 += VEC)
                 load_words<W, VEC>(in + blk_addr(e, (int64_t)gg * M + PSF::index(t, g, j0), count,
@@ -1058,10 +1176,10 @@ __device__ __forceinline__ void inv_reg_body(const W *__restrict__ in, Wout *__r
                 constexpr int E4 = E >> 2;
 #pragma unroll
                 for (int j = 0; j < E4; ++j) {
-                    W c0 = shoup<W>(x[j], tab.ninv, tab.ninvq, p);
-                    W c1 = shoup<W>(x[j + E4], tab.ninv, tab.ninvq, p);
-                    W c2 = shoup<W>(x[j + 2 * E4], tab.ninv, tab.ninvq, p);
-                    trunc_correct<W>(c0, c1, c2, shoup<W>(x[j + 3 * E4], tab.ninv, tab.ninvq, p), tab, p);
+                    W c0 = shoup1(x[j], tab.ninv, tab.ninvq, p);
+                    W c1 = shoup1(x[j + E4], tab.ninv, tab.ninvq, p);
+                    W c2 = shoup1(x[j + 2 * E4], tab.ninv, tab.ninvq, p);
+                    trunc_correct<W>(c0, c1, c2, shoup1(x[j + 3 * E4], tab.ninv, tab.ninvq, p), tab, p);
                     const int i1 = (j << (L - LOGE)) | t;
                     store(i1, (Wout)c0);
                     store(i1 + (M >> 2), (Wout)c1);
@@ -1070,7 +1188,7 @@ __device__ __forceinline__ void inv_reg_body(const W *__restrict__ in, Wout *__r
             } else {
 #pragma unroll
                 for (int j = 0; j < E; ++j)
-                    store((j << (L - LOGE)) | t, (Wout)shoup<W>(x[j], tab.ninv, tab.ninvq, p));
+                    store((j << (L - LOGE)) | t, (Wout)shoup1(x[j], tab.ninv, tab.ninvq, p));
             }
         };
         if (kXforms<L, LOGE> == 1) {
@@ -1292,7 +1410,7 @@ __device__ __forceinline__ W twist(W x, int64_t a, const W *lo, const W *loq, co
                                    const W *hiq, int slog, W p)
 {
     const int64_t al = a & (((int64_t)1 << slog) - 1), ah = a >> slog;
-    return shoup_lazy(shoup_lazy(x, lo[al], loq[al], p), hi[ah], hiq[ah], p);
+    return shoup2(shoup2(x, lo[al], loq[al], p), hi[ah], hiq[ah], p);
 }
 
 template <typename Win, typename W>
@@ -1326,7 +1444,7 @@ ntt_cols_fwd(const Win *__restrict__ in, int64_t in_stride, int64_t in_len, Win 
             const int k = jj << (logR - 1 - lh);
             const W u = s[i0], v = s[i1];
             s[i0] = add_2p<W>(u, v, p2);
-            s[i1] = shoup_lazy(sub_2p<W>(u, v, p2), ct.rt[k], ct.rtq[k], p);
+            s[i1] = shoup2(sub_2p<W>(u, v, p2), ct.rt[k], ct.rtq[k], p);
         }
         __syncthreads();
     }
@@ -1373,7 +1491,7 @@ ntt_cols_inv(const W *__restrict__ tmp, Wout *__restrict__ out, int64_t out_stri
             const int i1 = i0 + h * C;
             const int k = jj << (logR - 1 - lh);
             const W u = s[i0];
-            const W v = shoup_lazy(s[i1], ct.rti[k], ct.rtiq[k], p);
+            const W v = shoup2(s[i1], ct.rti[k], ct.rtiq[k], p);
             s[i0] = add_2p<W>(u, v, p2);
             const W d = sub_2p<W>(u, v, p2);
             s[i1] = d >= p2 ? d - p2 : d;
@@ -1384,7 +1502,7 @@ ntt_cols_inv(const W *__restrict__ tmp, Wout *__restrict__ out, int64_t out_stri
     for (int idx = threadIdx.x; idx < R * C; idx += kColThreads) {
         const int64_t pos = c0 + (idx & (C - 1)) + M * (idx >> logC);
         if (pos >= lo && pos < hi)
-            o[pos - lo] = (Wout)shoup<W>(s[idx], ninv, ninvq, p);
+            o[pos - lo] = (Wout)shoup1(s[idx], ninv, ninvq, p);
     }
 }
 
