@@ -323,8 +323,8 @@ def main():
         if key in tr:
             traffic = tr[key]["hbm_bytes_per_launch"]
     # (the C2 product is not truncated: lenC = 8191 > 3N/4)
-    kernels = {"forward": "ntt_fwd_reg<u64,u64,loose,L=13,LOGE=%d,TRUNC=0>" % fe,
-               "pointwise": ("pw_mfma_segs<u64,8,%d>" % (4 >> pbs)) if kind == "mfma"
+    kernels = {"forward": "ntt_fwd_reg<u64,u64,loose,L=13,LOGE=%d,whole,TRUNC=0>" % fe,
+               "pointwise": ("pw_mfma_segs<u64,%d>" % (2 >> pbs)) if kind == "mfma"
                else "pw_plain_segs<u64>",
                "inverse": "ntt_inv_reg<u64,u64,loose,L=13,LOGE=%d>" % ie}
     roofline = {"bound": "hbm", "kernel": kernels[names[dom]], "achieved": round(achieved, 1),

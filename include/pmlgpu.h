@@ -54,7 +54,7 @@ typedef enum {
 
 /* Pointwise-product kernel selection. */
 typedef enum {
-    PMLG_METHOD_AUTO = 0,  /* MFMA when the shape and modulus allow it, plain otherwise */
+    PMLG_METHOD_AUTO = 0,  /* the cheaper of the two below for the shape and modulus */
     PMLG_METHOD_PLAIN = 1, /* per-lane exact 128-bit (or 64-bit) dot products */
     PMLG_METHOD_MFMA = 2,  /* int8-limb MFMA contraction with int32 accumulation */
     PMLG_METHOD_THRESHOLD = 3 /* batched products: the hand-set threshold rule only */
@@ -276,7 +276,7 @@ pmlg_status pmlg_polmat_mul_batch(const pmlg_mul_desc *descs, int64_t count, voi
 pmlg_status pmlg_fill_random(pmlg_ctx ctx, uint64_t *dst, int64_t n, uint64_t seed, void *stream);
 
 /* Configurations: 0 direct convolution; 1..7 transforms with the plain or
- * MFMA pointwise kernel and different transform radices / MFMA block sizes. */
+ * MFMA pointwise kernel and different transform radices / points per MFMA task. */
 int pmlg_num_configs(void);
 int pmlg_config_valid(pmlg_ctx ctx, int64_t m, int64_t k, int64_t n, int64_t lenA, int64_t lenB,
                       int config);
