@@ -842,7 +842,8 @@ __device__ __forceinline__ void load_words(const W *src, W *v)
 
 // the converse: 32 bytes of each lane of a pair from `even` and `odd`
 // (inverse transforms, 16384 of length 1024: 109 -> 101 us; 2048 of length
-// 2048, 32-bit words: 19.2 -> 17.1)
+// 2048, 32-bit words: 19.2 -> 17.1; not in the radix-32 kernels, whose 16384
+// transforms of length 8192 took 0.95 ms with it and 0.81 without)
 template <typename W>
 __device__ __forceinline__ void load_pair(const W *even, const W *odd, W *v)
 {
@@ -1141,7 +1142,7 @@ __device__ __forceinline__ void inv_reg_body(const W *__restrict__ in, Wout *__r
             continue;
         }
         constexpr int BLOCK = 32 / sizeof(W);
-        constexpr bool PAIRS = RUN >= BLOCK && PSF::R < L - 2;
+        constexpr bool PAIRS = RUN >= BLOCK && PSF::R < L - 2 && LOGE < 5;
         if (PAIRS && logP >= (sizeof(W) == 8 ? 2 : 3)) {
             if constexpr (PAIRS) {
 #pragma unroll
