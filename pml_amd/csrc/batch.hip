@@ -290,7 +290,6 @@ struct FwdGroup {
     int nseg;
     int64_t blocks;
     bool trunc;  // 3/4-truncated products (their own launches: the split may differ)
-    int chunk;
 };
 struct InvGroup {
     pmlg_ctx ctx;
@@ -300,7 +299,6 @@ struct InvGroup {
     int nseg;
     int64_t blocks, mblocks;
     bool trunc;
-    int chunk;
 };
 struct PwGroup {
     pmlg_ctx ctx;
@@ -309,7 +307,6 @@ struct PwGroup {
     size_t seg_off;
     int nseg;
     int64_t blocks;
-    int chunk;
 };
 struct SchoolGroup {
     pmlg_ctx ctx;
@@ -322,7 +319,6 @@ struct ProdInfo {
     int config;
     int logN;
     size_t ah, bh, ch, tmp;  // word offsets in the arena (bytes / word size)
-    int chunk;
 };
 
 }  // namespace
@@ -343,7 +339,6 @@ struct pmlg_batch_plan_s {
     int nfill = 0;
     size_t fill_off = 0;
     std::vector<ProdInfo> prods;
-    int chunks = 1;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     // stage timing of graph replays (pmlg_batch_plan_time_stages): one graph
@@ -384,11 +379,11 @@ const NttTab<W> *tables_for(pmlg_ctx ctx, int logN, pmlg_status *st)
 }
 
 template <typename W>
-pmlg_status launch_groups(pmlg_batch_plan plan, hipStream_t s, int chunk)
+pmlg_status launch_groups(pmlg_batch_plan plan, hipStream_t s)
 {
     const unsigned char *tb = static_cast<const unsigned char *>(plan->tables);
     for (const FwdGroup &g : plan->fwd) {
-        if ((g.ctx->small ? 4 : 8) != sizeof(W) || (chunk >= 0 && g.chunk != chunk))
+        if ((g.ctx->small ? 4 : 8) != sizeof(W))
             continue;
         pmlg_status st;
         const NttTab<W> *tab = tables_for<W>(g.ctx, g.logN, &st);
@@ -403,11 +398,11 @@ pmlg_status launch_groups(pmlg_batch_plan plan, hipStream_t s, int chunk)
 }
 
 template <typename W>
-pmlg_status launch_pw(pmlg_batch_plan plan, hipStream_t s, int chunk)
+pmlg_status launch_pw(pmlg_batch_plan plan, hipStream_t s)
 {
     const unsigned char *tb = static_cast<const unsigned char *>(plan->tables);
     for (const PwGroup &g : plan->pw) {
-        if ((g.ctx->small ? 4 : 8) != sizeof(W) || (chunk >= 0 && g.chunk != chunk))
+        if ((g.ctx->small ? 4 : 8) != sizeof(W))
             continue;
         // persistent grid: a few workgroups per CU, never more than the tasks
         const int grid = (int)std::min<int64_t>(g.blocks, g.kind == PW_MFMA ? 512 : 2048);
@@ -420,11 +415,11 @@ pmlg_status launch_pw(pmlg_batch_plan plan, hipStream_t s, int chunk)
 }
 
 template <typename W>
-pmlg_status launch_inv(pmlg_batch_plan plan, hipStream_t s, int chunk)
+pmlg_status launch_inv(pmlg_batch_plan plan, hipStream_t s)
 {
     const unsigned char *tb = static_cast<const unsigned char *>(plan->tables);
     for (const InvGroup &g : plan->inv) {
-        if ((g.ctx->small ? 4 : 8) != sizeof(W) || (chunk >= 0 && g.chunk != chunk))
+        if ((g.ctx->small ? 4 : 8) != sizeof(W))
             continue;
         pmlg_status st;
         const NttTab<W> *tab = tables_for<W>(g.ctx, g.logN, &st);
@@ -452,66 +447,54 @@ struct StageEvents {
     bool on;
 };
 
-// one stage (0: forward, 1: direct convolutions, fills and pointwise, 2:
-// inverse) of one chunk, or of all of them (chunk -1)
-pmlg_status launch_stage(pmlg_batch_plan plan, hipStream_t s, int stage, int chunk)
-{
-    const unsigned char *tb = static_cast<const unsigned char *>(plan->tables);
-    pmlg_status st;
-    if (stage == 0)
-        return (st = launch_groups<uint64_t>(plan, s, chunk)) != PMLG_OK
-                   ? st
-                   : launch_groups<uint32_t>(plan, s, chunk);
-    if (stage == 2)
-        return (st = launch_inv<uint64_t>(plan, s, chunk)) != PMLG_OK ? st
-                                                                      : launch_inv<uint32_t>(plan, s, chunk);
-    if (chunk <= 0) {
-        for (const SchoolGroup &g : plan->school) {
-            const int grid = (int)std::min<int64_t>(g.blocks, 2048);
-            hipLaunchKernelGGL(school_segs, dim3(grid), dim3(kSchoolThreads), 0, s,
-                               reinterpret_cast<const SchoolSeg *>(tb + g.seg_off), g.nseg, g.blocks,
-                               g.ctx->mc);
-            HIP_TRY(hipGetLastError(), "batched direct convolutions");
-        }
-        if (plan->nfill > 0) {
-            hipLaunchKernelGGL(fill_zero_segs, dim3(256), dim3(256), 0, s,
-                               reinterpret_cast<const FillSeg *>(tb + plan->fill_off), plan->nfill);
-            HIP_TRY(hipGetLastError(), "zero fill");
-        }
-    }
-    return (st = launch_pw<uint64_t>(plan, s, chunk)) != PMLG_OK ? st : launch_pw<uint32_t>(plan, s, chunk);
-}
-
 // `only` in 0..2 launches that stage alone (the per-stage graphs of
-// pmlg_batch_plan_time_stages), -1 all three: with `se` stage by stage, else
-// chunk by chunk
+// pmlg_batch_plan_time_stages), -1 all three
 pmlg_status launch_all(pmlg_batch_plan plan, hipStream_t s, StageEvents *se = nullptr,
                        int only = -1)
 {
-    if (only >= 0)
-        return launch_stage(plan, s, only, -1);
+    const unsigned char *tb = static_cast<const unsigned char *>(plan->tables);
     pmlg_status st;
-    if (!se) {
-        for (int c = 0; c < plan->chunks; ++c)
-            for (int stage = 0; stage < 3; ++stage)
-                if ((st = launch_stage(plan, s, stage, c)) != PMLG_OK)
-                    return st;
-        return PMLG_OK;
-    }
-    for (int stage = 0; stage < 3; ++stage) {
-        HIP_TRY(hipEventRecord(se->ev[stage], s), "hipEventRecord");
-        if ((st = launch_stage(plan, s, stage, -1)) != PMLG_OK)
+    if (se)
+        HIP_TRY(hipEventRecord(se->ev[0], s), "hipEventRecord");
+    if (only < 0 || only == 0)
+        if ((st = launch_groups<uint64_t>(plan, s)) != PMLG_OK ||
+            (st = launch_groups<uint32_t>(plan, s)) != PMLG_OK)
             return st;
+    if (se)
+        HIP_TRY(hipEventRecord(se->ev[1], s), "hipEventRecord");
+    if (only >= 0 && only != 1)
+        goto inverse;
+    for (const SchoolGroup &g : plan->school) {
+        const int grid = (int)std::min<int64_t>(g.blocks, 2048);
+        hipLaunchKernelGGL(school_segs, dim3(grid), dim3(kSchoolThreads), 0, s,
+                           reinterpret_cast<const SchoolSeg *>(tb + g.seg_off), g.nseg, g.blocks,
+                           g.ctx->mc);
+        HIP_TRY(hipGetLastError(), "batched direct convolutions");
     }
-    HIP_TRY(hipEventRecord(se->ev[3], s), "hipEventRecord");
+    if (plan->nfill > 0) {
+        hipLaunchKernelGGL(fill_zero_segs, dim3(256), dim3(256), 0, s,
+                           reinterpret_cast<const FillSeg *>(tb + plan->fill_off), plan->nfill);
+        HIP_TRY(hipGetLastError(), "zero fill");
+    }
+    if ((st = launch_pw<uint64_t>(plan, s)) != PMLG_OK || (st = launch_pw<uint32_t>(plan, s)) != PMLG_OK)
+        return st;
+inverse:
+    if (se)
+        HIP_TRY(hipEventRecord(se->ev[2], s), "hipEventRecord");
+    if (only < 0 || only == 2)
+        if ((st = launch_inv<uint64_t>(plan, s)) != PMLG_OK ||
+            (st = launch_inv<uint32_t>(plan, s)) != PMLG_OK)
+            return st;
+    if (se)
+        HIP_TRY(hipEventRecord(se->ev[3], s), "hipEventRecord");
     return PMLG_OK;
 }
 
 template <typename W>
 void add_segments(const pmlg_mul_desc &d, const ProdInfo &pi, unsigned char *arena,
-                  std::map<std::tuple<int, pmlg_ctx, int, int, int>, std::vector<FwdSeg<uint64_t, W>>> &fwd,
-                  std::map<std::tuple<int, pmlg_ctx, int, int, int>, std::vector<InvSeg<W, uint64_t>>> &inv,
-                  std::map<std::tuple<int, pmlg_ctx, int, int>, std::vector<PwSeg<W>>> &pw)
+                  std::map<std::tuple<pmlg_ctx, int, int, int>, std::vector<FwdSeg<uint64_t, W>>> &fwd,
+                  std::map<std::tuple<pmlg_ctx, int, int, int>, std::vector<InvSeg<W, uint64_t>>> &inv,
+                  std::map<std::tuple<pmlg_ctx, int, int>, std::vector<PwSeg<W>>> &pw)
 {
     pmlg_ctx ctx = d.ctx;
     const ProdConfig &cf = kConfigs[pi.config];
@@ -525,11 +508,11 @@ void add_segments(const pmlg_mul_desc &d, const ProdInfo &pi, unsigned char *are
     const int64_t lenC = d.lenA + d.lenB - 1;
     // a product of length <= 3N/4 needs 3N/4 evaluations only
     const int trunc = trunc_ok<W>(logN, lenC) ? 1 : 0;
-    auto &fv = fwd[{pi.chunk, ctx, logN, cf.fwd_e, trunc}];
+    auto &fv = fwd[{ctx, logN, cf.fwd_e, trunc}];
     fv.push_back(FwdSeg<uint64_t, W>{d.A, Ah, d.lenA, d.lenA, d.m * d.k, 0, trunc, 0});
     fv.push_back(FwdSeg<uint64_t, W>{d.B, Bh, d.lenB, d.lenB, d.k * d.n, 0, trunc, 0});
     const bool redc = sizeof(W) == 8;
-    inv[{pi.chunk, ctx, logN, cf.inv_e, (redc ? 1 : 0) | (trunc << 1)}].push_back(
+    inv[{ctx, logN, cf.inv_e, (redc ? 1 : 0) | (trunc << 1)}].push_back(
         InvSeg<W, uint64_t>{Ch, d.C, tmp, lenC, 0, lenC, d.m * d.n, 0, 0, trunc, 0});
     const int pt = cf.kind == PW_MFMA ? pw_points(sizeof(W), logP, cf.single_pt != 0) : 0;
     PwSeg<W> ps{};
@@ -547,30 +530,30 @@ void add_segments(const pmlg_mul_desc &d, const ProdInfo &pi, unsigned char *are
         const unsigned __int128 vmax = (unsigned __int128)d.k * (ctx->p - 1) * (ctx->p - 1);
         ps.redc_small = vmax < (((unsigned __int128)(3 * ctx->p - 1)) << 64) ? 1 : 0;
     }
-    pw[std::make_tuple(pi.chunk, ctx, (int)cf.kind, pt)].push_back(ps);
+    pw[std::make_tuple(ctx, (int)cf.kind, pt)].push_back(ps);
 }
 
 template <typename W>
 void finish_groups(pmlg_batch_plan plan, Blob &blob,
-                   std::map<std::tuple<int, pmlg_ctx, int, int, int>, std::vector<FwdSeg<uint64_t, W>>> &fwd,
-                   std::map<std::tuple<int, pmlg_ctx, int, int, int>, std::vector<InvSeg<W, uint64_t>>> &inv,
-                   std::map<std::tuple<int, pmlg_ctx, int, int>, std::vector<PwSeg<W>>> &pw)
+                   std::map<std::tuple<pmlg_ctx, int, int, int>, std::vector<FwdSeg<uint64_t, W>>> &fwd,
+                   std::map<std::tuple<pmlg_ctx, int, int, int>, std::vector<InvSeg<W, uint64_t>>> &inv,
+                   std::map<std::tuple<pmlg_ctx, int, int>, std::vector<PwSeg<W>>> &pw)
 {
     for (auto &kv : fwd) {
-        const int logN = std::get<2>(kv.first);
-        const bool trunc = std::get<4>(kv.first) != 0;
+        const int logN = std::get<1>(kv.first);
+        const bool trunc = std::get<3>(kv.first) != 0;
         int64_t b = 0;
         for (auto &sg : kv.second) {
             sg.block0 = b;
             b += ntt_seg_blocks<W>(sg.count, logN, trunc);
         }
-        FwdGroup g{std::get<1>(kv.first), logN, eval_log_run_in<W>(logN),
-                   std::get<3>(kv.first), blob.add(kv.second), (int)kv.second.size(), b, trunc, std::get<0>(kv.first)};
+        FwdGroup g{std::get<0>(kv.first), logN, eval_log_run_in<W>(logN),
+                   std::get<2>(kv.first), blob.add(kv.second), (int)kv.second.size(), b, trunc};
         plan->fwd.push_back(g);
     }
     for (auto &kv : inv) {
-        const int logN = std::get<2>(kv.first);
-        const bool trunc = (std::get<4>(kv.first) & 2) != 0;
+        const int logN = std::get<1>(kv.first);
+        const bool trunc = (std::get<3>(kv.first) & 2) != 0;
         int64_t b = 0, mb = 0;
         for (auto &sg : kv.second) {
             sg.block0 = b;
@@ -578,20 +561,20 @@ void finish_groups(pmlg_batch_plan plan, Blob &blob,
             b += ntt_seg_blocks<W>(sg.count, logN, trunc);
             mb += merge_seg_blocks<W>(sg.count, sg.hi - sg.lo, logN, trunc);
         }
-        InvGroup g{std::get<1>(kv.first), logN, eval_log_run_out<W>(logN),
-                   std::get<3>(kv.first), (std::get<4>(kv.first) & 1) != 0, blob.add(kv.second),
-                   (int)kv.second.size(), b, mb, trunc, std::get<0>(kv.first)};
+        InvGroup g{std::get<0>(kv.first), logN, eval_log_run_out<W>(logN),
+                   std::get<2>(kv.first), (std::get<3>(kv.first) & 1) != 0, blob.add(kv.second),
+                   (int)kv.second.size(), b, mb, trunc};
         plan->inv.push_back(g);
     }
     for (auto &kv : pw) {
-        const PointwiseKind kind = (PointwiseKind)std::get<2>(kv.first);
-        const int pt = std::get<3>(kv.first);
+        const PointwiseKind kind = (PointwiseKind)std::get<1>(kv.first);
+        const int pt = std::get<2>(kv.first);
         int64_t b = 0;
         for (auto &sg : kv.second) {
             sg.block0 = b;
             b += pw_seg_blocks(kind, pt, sg.m, sg.n, sg.N);
         }
-        PwGroup g{std::get<1>(kv.first), kind, pt, blob.add(kv.second), (int)kv.second.size(), b, std::get<0>(kv.first)};
+        PwGroup g{std::get<0>(kv.first), kind, pt, blob.add(kv.second), (int)kv.second.size(), b};
         plan->pw.push_back(g);
     }
 }
@@ -643,68 +626,6 @@ void free_plan_memory(pmlg_batch_plan plan)
 
 namespace pmlg {
 
-// Chunks of a plan: its products are run kChunkBytes of evaluations at a time,
-// forward, pointwise and inverse, so that the pointwise kernels find the
-// evaluations, and the inverse ones the products, still in the 256 MB of
-// last-level cache instead of in HBM.  Products of one length and configuration
-// stay together, so a chunk border adds at most three launches.  16 products of
-// 32 x 32 matrices of length 4096 (60-bit, 201 MB of evaluations each): pointwise
-// 0.93 -> 0.81 ms, in all 3.40 -> 3.30; 48 uneven ones 2.12 -> 2.07.  (Reusing
-// one chunk's memory for the next gave nothing more.)
-// Running a product's inverse before another's forward transform needs outputs
-// and inputs that don't overlap; else the plan is one chunk.
-constexpr double kChunkBytes = 200e6;
-
-void assign_chunks(pmlg_batch_plan plan, const pmlg_mul_desc *descs)
-{
-    struct Range {
-        uintptr_t lo, hi;
-        bool out;
-    };
-    std::vector<Range> ranges;
-    std::vector<size_t> order;
-    for (size_t i = 0; i < plan->prods.size(); ++i) {
-        const pmlg_mul_desc &d = descs[i];
-        if (d.lenA == 0 || d.lenB == 0 || d.m == 0 || d.n == 0)
-            continue;
-        auto add = [&](const uint64_t *p, int64_t words, bool out) {
-            if (words > 0)
-                ranges.push_back(Range{(uintptr_t)p, (uintptr_t)(p + words), out});
-        };
-        add(d.C, d.m * d.n * (d.lenA + d.lenB - 1), true);
-        add(d.A, d.m * d.k * d.lenA, false);
-        add(d.B, d.k * d.n * d.lenB, false);
-        if (plan->prods[i].config >= 0 && !kConfigs[plan->prods[i].config].school)
-            order.push_back(i);
-    }
-    std::sort(ranges.begin(), ranges.end(), [](const Range &a, const Range &b) { return a.lo < b.lo; });
-    uintptr_t end[2] = {0, 0};  // of the inputs and of the outputs so far
-    for (const Range &r : ranges) {
-        if (r.lo < end[r.out ? 0 : 1])
-            return;
-        end[r.out] = std::max(end[r.out], r.hi);
-    }
-    std::stable_sort(order.begin(), order.end(), [&](size_t a, size_t b) {
-        const ProdInfo &x = plan->prods[a], &y = plan->prods[b];
-        return std::make_tuple(descs[a].ctx, x.logN, x.config) < std::make_tuple(descs[b].ctx, y.logN, y.config);
-    });
-    double bytes = 0;
-    int chunk = 0;
-    for (size_t i : order) {
-        const pmlg_mul_desc &d = descs[i];
-        const double w = d.ctx->small ? 4 : 8;
-        const double own = w * (double)(d.m * d.k + d.k * d.n + d.m * d.n) *
-                           (double)((int64_t)1 << plan->prods[i].logN);
-        if (bytes > 0 && bytes + own > kChunkBytes) {
-            ++chunk;
-            bytes = 0;
-        }
-        bytes += own;
-        plan->prods[i].chunk = chunk;
-    }
-    plan->chunks = chunk + 1;
-}
-
 // Builds a plan; with `ws` non-null the arena and tables are carved from it
 // (ws_bytes long) instead of being allocated.
 pmlg_status build_plan(pmlg_batch_plan *out, const pmlg_mul_desc *descs, int64_t count, int flags,
@@ -749,7 +670,6 @@ pmlg_status build_plan(pmlg_batch_plan *out, const pmlg_mul_desc *descs, int64_t
         ProdInfo &pi = plan->prods[i];
         pi.config = -1;
         pi.logN = 0;
-        pi.chunk = 0;
         pi.tmp = (size_t)-1;
         if (d.lenA == 0 || d.lenB == 0 || d.m == 0 || d.n == 0)
             continue;  // nothing to write
@@ -781,7 +701,6 @@ pmlg_status build_plan(pmlg_batch_plan *out, const pmlg_mul_desc *descs, int64_t
             pi.tmp = take((size_t)(d.m * d.n * N) * w) / w;
     }
     const size_t arena_bytes = std::max<size_t>(words_bytes, 256);
-    assign_chunks(plan.get(), descs);
 
     // segment tables (device addresses depend on the arena, so place it first)
     unsigned char *arena = nullptr;
@@ -798,12 +717,12 @@ pmlg_status build_plan(pmlg_batch_plan *out, const pmlg_mul_desc *descs, int64_t
     plan->arena_bytes = arena_bytes;
 
     Blob blob;
-    std::map<std::tuple<int, pmlg_ctx, int, int, int>, std::vector<FwdSeg<uint64_t, uint64_t>>> f64;
-    std::map<std::tuple<int, pmlg_ctx, int, int, int>, std::vector<FwdSeg<uint64_t, uint32_t>>> f32;
-    std::map<std::tuple<int, pmlg_ctx, int, int, int>, std::vector<InvSeg<uint64_t, uint64_t>>> i64;
-    std::map<std::tuple<int, pmlg_ctx, int, int, int>, std::vector<InvSeg<uint32_t, uint64_t>>> i32;
-    std::map<std::tuple<int, pmlg_ctx, int, int>, std::vector<PwSeg<uint64_t>>> p64;
-    std::map<std::tuple<int, pmlg_ctx, int, int>, std::vector<PwSeg<uint32_t>>> p32;
+    std::map<std::tuple<pmlg_ctx, int, int, int>, std::vector<FwdSeg<uint64_t, uint64_t>>> f64;
+    std::map<std::tuple<pmlg_ctx, int, int, int>, std::vector<FwdSeg<uint64_t, uint32_t>>> f32;
+    std::map<std::tuple<pmlg_ctx, int, int, int>, std::vector<InvSeg<uint64_t, uint64_t>>> i64;
+    std::map<std::tuple<pmlg_ctx, int, int, int>, std::vector<InvSeg<uint32_t, uint64_t>>> i32;
+    std::map<std::tuple<pmlg_ctx, int, int>, std::vector<PwSeg<uint64_t>>> p64;
+    std::map<std::tuple<pmlg_ctx, int, int>, std::vector<PwSeg<uint32_t>>> p32;
     for (int64_t i = 0; i < count; ++i) {
         const ProdInfo &pi = plan->prods[i];
         if (pi.config < 0 || kConfigs[pi.config].school)

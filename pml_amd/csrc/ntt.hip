@@ -239,7 +239,7 @@ ntt_merge_kernel(const W *__restrict__ z, Wout *__restrict__ out, int64_t out_st
 // need no workgroup barrier.  (A radix-2 stage per LDS round trip and barrier,
 // as these sizes had before, took 446 us for both operands of 128 x 128
 // matrices of length 512 at 1024 points, 60-bit prime; these kernels take
-// 170, and 28.8 -> 8.9 us for 16 x 16 matrices of length 256.)
+// 196, and 28.8 -> 8.9 us for 16 x 16 matrices of length 256.)
 // ===========================================================================
 // Buffer descriptor of `bytes` bytes at the uniform address p: loads past its
 // end give 0 and stores past it are dropped, so a row of elements cut by a
