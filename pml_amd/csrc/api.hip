@@ -315,13 +315,13 @@ pmlg_status run_product_on(pmlg_ctx ctx, const Tables *T, W *Ah, W *Bh, W *Ch, v
             "ntt_fwd");
     if (prof)
         prof_end(ctx, s, &pr);
-    // Products of 64-bit words come as V 2^-64 mod p (Montgomery REDC) in [0, 4p);
+    // Products of 64-bit words come as V 2^-64 mod p (Montgomery REDC), below 4p or
+    // 2p as the inverse's butterflies need (host_redc_small);
     // the inverse transform then scales by N^-1 2^64 instead of N^-1.
     ModConst mc = ctx->mc;
     NttTab<W> itab = tab;
     if (sizeof(W) == 8) {
-        const unsigned __int128 vmax = (unsigned __int128)k * (ctx->p - 1) * (ctx->p - 1);
-        mc.redc_small = vmax < (((unsigned __int128)(3 * ctx->p - 1)) << 64) ? 1 : 0;
+        mc.redc_small = host_redc_small(ctx->p, k);
         itab.ninv = tab.ninvr;
         itab.ninvq = tab.ninvrq;
         itab.ninv2 = tab.ninvr2;

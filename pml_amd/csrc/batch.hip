@@ -525,11 +525,7 @@ void add_segments(const pmlg_mul_desc &d, const ProdInfo &pi, unsigned char *are
     ps.logP = logP;
     ps.logPc = eval_log_run_out<W>(logN);
     ps.N = trunc ? 3 * (N >> 2) : N;
-    ps.redc_small = 0;
-    if (redc) {
-        const unsigned __int128 vmax = (unsigned __int128)d.k * (ctx->p - 1) * (ctx->p - 1);
-        ps.redc_small = vmax < (((unsigned __int128)(3 * ctx->p - 1)) << 64) ? 1 : 0;
-    }
+    ps.redc_small = redc ? host_redc_small(ctx->p, d.k) : 0;
     pw[std::make_tuple(ctx, (int)cf.kind, pt)].push_back(ps);
 }
 

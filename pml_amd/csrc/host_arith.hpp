@@ -101,6 +101,18 @@ static inline uint64_t host_pow2_mod(int e, uint64_t p)
     return host_powmod(2, (uint64_t)e, p);
 }
 
+// Whether the REDC of a sum of k products of residues is small enough for the
+// inverse transform as it is (V < bound 2^64 leaves V 2^-64 mod p below bound + p).
+// The lazy butterflies (p < 2^60) take inputs below 8p, so the bound is 3p - 1
+// (outputs below 4p); the strict ones hold their values below 2p, so it is p - 1.
+// Larger sums take a Barrett step, to below 2p.
+static inline int host_redc_small(uint64_t p, int64_t k)
+{
+    const u128_t vmax = (u128_t)k * (p - 1) * (p - 1);
+    const uint64_t bound = p < ((uint64_t)1 << 60) ? 3 * p - 1 : p - 1;
+    return vmax < ((u128_t)bound << 64) ? 1 : 0;
+}
+
 static inline ModConst host_modconst(uint64_t p)
 {
     ModConst mc{};

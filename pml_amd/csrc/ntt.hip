@@ -1164,7 +1164,8 @@ __device__ __forceinline__ void inv_reg_body(const W *__restrict__ in, Wout *__r
         }
     }
     const Bfly<W> k(p);
-    // inputs below 8p (the pointwise products' lazy outputs)
+    // inputs: the pointwise products, below 8p for the lazy butterflies and below
+    // 2p for the strict ones (host_redc_small)
     inv_passes<W, LOOSE, L, LOGE, SLAST, 8>(x, tw, lds, t, tab, k, tq);
     // pass-0 arrangement: element j is index (j << (L-LOGE)) | t
     if (R == 1) {

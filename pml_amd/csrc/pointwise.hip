@@ -12,7 +12,8 @@
 //    k, the T_w are folded into three (or two) signed 64-bit partial sums,
 //    and the exact dot product is rebuilt in 128 bits and reduced.
 // 64-bit words leave V 2^-64 mod p (Montgomery REDC; the inverse transform's
-// scaling carries the 2^64), below 4p; 32-bit words are reduced to [0, p) by
+// scaling carries the 2^64), below 4p for p < 2^60 and below 2p above, as the
+// inverse's lazy and strict butterflies need; 32-bit words are reduced to [0, p) by
 // Barrett steps.  No floating point is involved.
 #include "internal.hpp"
 
@@ -447,8 +448,8 @@ __device__ __forceinline__ void mfma_task(const W *__restrict__ Ah, const W *__r
                 res[r][pt] = (W)barrett(barrett_lazy(lo, mc.bm, mc.p) + hi * mc.c64, mc.bm, mc.p);
             }
         }
-    // small k p: the REDC outputs are below 4p already; otherwise a Barrett
-    // step (they are below 2^64)
+    // small k p: the REDC outputs are within the inverse's range already;
+    // otherwise a Barrett step to below 2p (they are below 2^64)
     if (sizeof(W) == 8 && !mc.redc_small) {
 #pragma unroll
         for (int r = 0; r < 4; ++r)
