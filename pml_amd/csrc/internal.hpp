@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
+
 #include "modarith.hpp"
 
 namespace pmlg {
@@ -22,6 +24,24 @@ template <typename T>
 __device__ __forceinline__ T *as_global(T *p)
 {
     return (T *)(__attribute__((address_space(1))) T *)(uint64_t)uniform(reinterpret_cast<int64_t>(p));
+}
+
+// Raises a kernel's limit of dynamic LDS (64 KiB by default) to `bytes` on the
+// current device, once: `raised` is the kernel's own word, a bit per device.
+// Any thread may call it; two that meet both set the same limit.
+inline hipError_t raise_lds_limit(const void *kernel, size_t bytes, std::atomic<uint64_t> &raised)
+{
+    int device = 0;
+    hipError_t e = hipGetDevice(&device);
+    if (e != hipSuccess)
+        return e;
+    const uint64_t bit = (uint64_t)1 << (device & 63);
+    if (device < 64 && (raised.load(std::memory_order_acquire) & bit))
+        return hipSuccess;
+    e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+    if (e == hipSuccess)
+        raised.fetch_or(bit, std::memory_order_release);
+    return e;
 }
 
 // Root-of-unity tables for one (p, log2 N): tw[t] = w^t, itw[t] = w^-t for

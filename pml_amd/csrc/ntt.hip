@@ -1253,22 +1253,19 @@ inline int64_t xform_blocks(int64_t count, int logM, int logR)
 
 // Register-kernel launchers.  From 2^12 points on, logE (log2 of the elements
 // per thread) is a tuning parameter: 4 (radix-16 passes, more threads, fewer
-// registers) or 5 (radix-32 passes, fewer LDS exchanges).
-template <int L, int LOGE, typename W, typename Kern, typename... Args>
-hipError_t launch_xform(Kern *kern, int64_t blocks, hipStream_t s, Args... args)
+// registers) or 5 (radix-32 passes, fewer LDS exchanges).  The kernel is a
+// template argument, so that each has a flag of its own: many share one type.
+template <auto Kern, int L, int LOGE, typename W, typename... Args>
+hipError_t launch_xform(int64_t blocks, hipStream_t s, Args... args)
 {
     constexpr size_t lds = (size_t)kXforms<L, LOGE> * kXformLds<L> * sizeof(W);
     if constexpr (lds > 64 * 1024) {
-        static bool attr = false;
-        if (!attr) {
-            hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                               (int)lds);
-            if (e != hipSuccess)
-                return e;
-            attr = true;
-        }
+        static std::atomic<uint64_t> raised{0};
+        const hipError_t e = raise_lds_limit((const void *)Kern, lds, raised);
+        if (e != hipSuccess)
+            return e;
     }
-    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kXformThreads<L, LOGE>), lds, s, args...);
+    hipLaunchKernelGGL(Kern, dim3((unsigned)blocks), dim3(kXformThreads<L, LOGE>), lds, s, args...);
     return hipGetLastError();
 }
 
@@ -1279,25 +1276,25 @@ hipError_t launch_fwd_e(const SegList<FwdSeg<Win, W>> &segs, int64_t blocks, int
     constexpr int top = NttLimits<W>::max_log_m;
     if constexpr (L == top)
         if (pre)
-            return launch_xform<L, LOGE, W>(ntt_fwd_reg<Win, W, LOOSE, L, LOGE, kRows, false>, blocks, s, segs,
-                                            logR, logP, tab, p);
+            return launch_xform<ntt_fwd_reg<Win, W, LOOSE, L, LOGE, kRows, false>, L, LOGE, W>(
+                blocks, s, segs, logR, logP, tab, p);
     if constexpr (L >= top - 1)
         if (logR > 0) {
             if (trunc)
-                return launch_xform<L, LOGE, W>(ntt_fwd_reg<Win, W, LOOSE, L, LOGE, kSplit, true>, blocks, s,
-                                                segs, logR, logP, tab, p);
+                return launch_xform<ntt_fwd_reg<Win, W, LOOSE, L, LOGE, kSplit, true>, L, LOGE, W>(
+                    blocks, s, segs, logR, logP, tab, p);
             if constexpr (L == top)
-                return launch_xform<L, LOGE, W>(ntt_fwd_reg<Win, W, LOOSE, L, LOGE, kSplit, false>, blocks, s,
-                                                segs, logR, logP, tab, p);
+                return launch_xform<ntt_fwd_reg<Win, W, LOOSE, L, LOGE, kSplit, false>, L, LOGE, W>(
+                    blocks, s, segs, logR, logP, tab, p);
         }
     if (pre || logR > 0)
         return hipErrorInvalidValue;
     if constexpr (L >= kTruncMinLog)
         if (trunc)
-            return launch_xform<L, LOGE, W>(ntt_fwd_reg<Win, W, LOOSE, L, LOGE, kWhole, true>, blocks, s, segs,
-                                            logR, logP, tab, p);
-    return launch_xform<L, LOGE, W>(ntt_fwd_reg<Win, W, LOOSE, L, LOGE, kWhole, false>, blocks, s, segs, logR,
-                                    logP, tab, p);
+            return launch_xform<ntt_fwd_reg<Win, W, LOOSE, L, LOGE, kWhole, true>, L, LOGE, W>(
+                blocks, s, segs, logR, logP, tab, p);
+    return launch_xform<ntt_fwd_reg<Win, W, LOOSE, L, LOGE, kWhole, false>, L, LOGE, W>(blocks, s, segs, logR,
+                                                                                        logP, tab, p);
 }
 
 template <typename Win, typename W, int L>
@@ -1325,15 +1322,15 @@ hipError_t launch_inv_l(int logE, const SegList<InvSeg<W, Wout>> &segs, int64_t 
     if constexpr (sizeof(W) == 8) {
         if ((uint64_t)p < ((uint64_t)1 << 60)) {
             if (logE == 5)
-                return launch_xform<L, E5, W>(ntt_inv_reg<W, Wout, true, L, E5>, blocks, s, segs, logR, logP,
-                                              tab, p);
-            return launch_xform<L, E4, W>(ntt_inv_reg<W, Wout, true, L, E4>, blocks, s, segs, logR, logP, tab,
-                                          p);
+                return launch_xform<ntt_inv_reg<W, Wout, true, L, E5>, L, E5, W>(blocks, s, segs, logR, logP,
+                                                                                 tab, p);
+            return launch_xform<ntt_inv_reg<W, Wout, true, L, E4>, L, E4, W>(blocks, s, segs, logR, logP, tab,
+                                                                             p);
         }
     }
     if (logE == 5)
-        return launch_xform<L, E5, W>(ntt_inv_reg<W, Wout, false, L, E5>, blocks, s, segs, logR, logP, tab, p);
-    return launch_xform<L, E4, W>(ntt_inv_reg<W, Wout, false, L, E4>, blocks, s, segs, logR, logP, tab, p);
+        return launch_xform<ntt_inv_reg<W, Wout, false, L, E5>, L, E5, W>(blocks, s, segs, logR, logP, tab, p);
+    return launch_xform<ntt_inv_reg<W, Wout, false, L, E4>, L, E4, W>(blocks, s, segs, logR, logP, tab, p);
 }
 
 // f with the sub-transform's size as a compile-time constant

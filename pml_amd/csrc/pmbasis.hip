@@ -1806,8 +1806,7 @@ pmlg_status leaf(pmlg_ctx ctx, Arena &ar, const uint64_t *F, int64_t strideF, in
     hipLaunchKernelGGL(leaf_init_kernel, dim3(grid_for((int64_t)m * m * cap + (int64_t)m * n * ordL)),
                        dim3(256), 0, s, a, F, strideF, lt, W);
     HIP_TRY(hipGetLastError(), "leaf_init_kernel");
-    static bool attr = false;
-    if (!attr) {
+    {
         const void *kernels[] = {(const void *)mbasis_step_kernel<Mont64Arith, 1>,
                                  (const void *)mbasis_step_kernel<Mont64Arith, 2>,
                                  (const void *)mbasis_step_kernel<Mont32Arith, 1>,
@@ -1817,10 +1816,10 @@ pmlg_status leaf(pmlg_ctx ctx, Arena &ar, const uint64_t *F, int64_t strideF, in
                                  (const void *)mbasis_update_kernel<Mont64Arith, true>,
                                  (const void *)mbasis_update_kernel<Mont32Arith, true>,
                                  (const void *)mbasis_update_kernel<BigArith, true>};
-        for (const void *k : kernels)
-            HIP_TRY(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLds),
-                    "hipFuncSetAttribute(mbasis kernels)");
-        attr = true;
+        constexpr int nk = sizeof(kernels) / sizeof(kernels[0]);
+        static std::atomic<uint64_t> raised[nk];
+        for (int i = 0; i < nk; ++i)
+            HIP_TRY(raise_lds_limit(kernels[i], kLds, raised[i]), "hipFuncSetAttribute(mbasis kernels)");
     }
     // rows of the transposed residual per lane of the composing wave
     const bool one_row = n <= 64;
