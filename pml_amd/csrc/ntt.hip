@@ -22,12 +22,15 @@ constexpr int kThreads = 256;
 // transforms split into sub-transforms (logR > 0) have sub-transforms of at
 // least this size, one per workgroup
 constexpr int kRegMinLog = 11;
-// Waves per SIMD of the register kernels, by log2 of the elements a thread
-// holds: eight 64-bit words leave room for four, sixteen for four within 128
-// registers, thirty-two for two.  Without the bound the register allocator
-// drifts past the next limit on small changes of the surrounding code.
-template <int LOGE>
-constexpr int kXformWaves = LOGE == 5 ? 2 : 4;
+// Waves per SIMD of the register kernels, by the words a thread holds: eight or
+// sixteen 64-bit ones leave four within 128 registers, as do thirty-two 32-bit
+// ones; thirty-two 64-bit ones leave two.  Without the bound the register allocator
+// drifts past the next limit on small changes of the surrounding code (with two
+// waves for all thirty-two words the 32-bit kernels of 2^14 points took 150
+// registers, and one workgroup a compute unit instead of two: 32 products of 20 x 20 x
+// 20, length 5500, 3.20 -> 2.95 ms).
+template <typename W, int LOGE>
+constexpr int kXformWaves = LOGE == 5 && sizeof(W) == 8 ? 2 : 4;
 
 // Point-blocked evaluation layout: position `pos` of entry `e` (of `count`
 // entries) lives at ((pos >> logP) * count + e) * P + (pos mod P), P = 2^logP,
@@ -1088,7 +1091,7 @@ struct SegList {
 // wave per SIMD instead of two).  Every segment of one launch has the
 // launch's TRUNC.
 template <typename Win, typename W, bool LOOSE, int L, int LOGE, int MODE, bool TRUNC>
-__global__ void __launch_bounds__((kXformThreads<L, LOGE>)) __attribute__((amdgpu_waves_per_eu(kXformWaves<LOGE>)))
+__global__ void __launch_bounds__((kXformThreads<L, LOGE>)) __attribute__((amdgpu_waves_per_eu(kXformWaves<W, LOGE>)))
 ntt_fwd_reg(SegList<FwdSeg<Win, W>> segs, int logR, int logP, NttTab<W> tab, W p)
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
@@ -1225,7 +1228,7 @@ __device__ __forceinline__ void inv_reg_body(const W *__restrict__ in, Wout *__r
 }
 
 template <typename W, typename Wout, bool LOOSE, int L, int LOGE>
-__global__ void __launch_bounds__((kXformThreads<L, LOGE>)) __attribute__((amdgpu_waves_per_eu(kXformWaves<LOGE>)))
+__global__ void __launch_bounds__((kXformThreads<L, LOGE>)) __attribute__((amdgpu_waves_per_eu(kXformWaves<W, LOGE>)))
 ntt_inv_reg(SegList<InvSeg<W, Wout>> segs, int logR, int logP, NttTab<W> tab, W p)
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
