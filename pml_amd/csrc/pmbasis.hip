@@ -25,7 +25,7 @@
 // each order, and writes every order's description; kernel 2 (a grid) then
 // applies the window's row operations, one after the other, to tiles of
 // appbas and of the rest of R held in LDS, reading one buffer and writing the
-// other.  All control (nullity cases, basis length)
+// other (a thread per coefficient where windows do not pay: mbasis_window).  All control (nullity cases, basis length)
 // stays on the device: a leaf is a fixed sequence of launches.  The steps
 // skip the division by the pivots in 3: with D the product of the pivots,
 // they apply D X and multiply the updated rows by D, so each basis row is the
@@ -42,6 +42,7 @@
 
 #include "ctx.hpp"
 #include "host_arith.hpp"
+#include "rules.hpp"
 
 namespace pmlg {
 
@@ -68,25 +69,20 @@ __host__ __device__ inline size_t step_lds_bytes(int m, int n, size_t wbytes)
            ((size_t)n * (m | 1) + kMaxN + 2 * (size_t)kMaxN * (kPanel + 1)) * wbytes +
            (4 * (size_t)m + 3 * (size_t)kMaxN) * sizeof(int);
 }
-// LDS bytes of the step kernel with a window of w orders: the above, the row
-// scales and delays, and for w > 1 the window's residual coefficients
+// Residual coefficients that the step kernel holds in LDS for a window of w
+// orders: all of them, which the windows' choice makes fit, but for a single
+// order's too large for it (read from memory when the rows' places are known)
+__host__ __device__ inline int window_slots(int m, int n, int w, size_t wbytes)
+{
+    const size_t base = step_lds_bytes(m, n, wbytes) + (size_t)m * (wbytes + sizeof(int));
+    return w > 1 || base + (size_t)m * n * wbytes <= kLds ? w : 0;
+}
+// LDS bytes of the step kernel with a window of w orders: those of
+// step_lds_bytes, the row scales and delays, and the coefficients
 __host__ __device__ inline size_t window_lds_bytes(int m, int n, int w, size_t wbytes)
 {
     return step_lds_bytes(m, n, wbytes) + (size_t)m * (wbytes + sizeof(int)) +
-           (w > 1 ? (size_t)m * n * w * wbytes : 0);
-}
-// Orders per window: what fits LDS.  A longer window spares launches (the step
-// and update kernels' start-up, loads and stores: about 10 us together) and
-// lengthens the step kernel's own update of the window's remaining
-// coefficients, which one workgroup does alone.  Windows of 3 and 4 orders, step
-// plus update per order: 20.9 and 20.5 us (64 x 32, 32-bit words), 14.8 and 14.7
-// us (32 x 17, 64-bit words).
-inline int window_orders(int m, int n, size_t wbytes)
-{
-    int w = kWindow;
-    while (w > 1 && window_lds_bytes(m, n, w, wbytes) > kLds)
-        --w;
-    return w;
+           (size_t)m * n * window_slots(m, n, w, wbytes) * wbytes;
 }
 // LDS bytes of the update kernel but the staged vectors: the tile, the
 // window's row lists, the delays and a word per wave
@@ -94,7 +90,31 @@ __host__ __device__ inline size_t update_lds_bytes(int m, size_t wbytes)
 {
     return ((size_t)m * kTile * wbytes + ((size_t)m * (kWindow + 1) + 8) * sizeof(int) + 15) & ~(size_t)15;
 }
-constexpr int kXPad = 32;     // words after X read (and discarded) by the last update group
+__host__ __device__ inline int pad16(int r)
+{
+    return (r + 15) & ~15;
+}
+// most words of one order's kernel vectors, rows padded to a multiple of 16
+inline size_t staged_words(int m, int n)
+{
+    size_t most = 0;
+    for (int r = 1; r <= std::min(m, n); ++r)
+        most = std::max(most, (size_t)(m - r) * pad16(r));
+    return most;
+}
+// Orders per window that LDS allows: the step kernel's coefficients, and the
+// update kernel's vectors in half of it, so that two workgroups share a compute
+// unit (32-bit words, 192 x 24 at order 1500: 161 us an order in windows of 4, 114 in
+// windows of 2)
+inline int window_orders(int m, int n, size_t wbytes)
+{
+    int w = kWindow;
+    while (w > 1 && (window_lds_bytes(m, n, w, wbytes) > kLds ||
+                     update_lds_bytes(m, wbytes) + staged_words(m, n) * w * wbytes > kLds / 2))
+        --w;
+    return w;
+}
+constexpr int kXPad = 32;     // words after X read (and discarded) by mbasis_update1_kernel's last group
 
 // control words of one leaf
 enum Ctl {
@@ -113,6 +133,7 @@ struct LeafArgs {
     int m, n;
     int ordL;     // order of the leaf
     int cap;      // coefficient capacity of appbas (ordL + 1)
+    int window;   // orders per launch of the step kernel
     uint64_t *app[2];  // m x m x cap, entry-major
     uint64_t *R[2];    // m x n x ordL, entry-major
     uint64_t *Rn;      // the coming window's residual coefficients: m x n each, one after the other
@@ -469,8 +490,7 @@ __device__ __forceinline__ uint64_t lane_value(uint64_t v, int l)
 // coefficients of the window sit in LDS (Rw, slot d of row i its coefficient
 // ord0 + d + delay[i]: multiplying a row by x only raises its delay), and after
 // each order the kernel rows' coefficients of the orders still to come are
-// combined here, so that a window costs one launch of each kernel.  With
-// w = 1 the residual coefficient goes straight from global memory to At.
+// combined here, so that a window costs one launch of each kernel.
 //
 // One workgroup and a chain of n pivots: latency bounds it, not throughput.  Of
 // the 16.5 us that an order takes (64 x 32, 32-bit words, clock stamps) the
@@ -491,10 +511,17 @@ __global__ void __launch_bounds__(kStepThreads) mbasis_step_kernel(LeafArgs a, i
     // columns) are bound by the apply, which wider panels make shorter
     constexpr int P = sizeof(V) == 8 && H == 1 ? 2 : kPanel;
     static_assert(P <= kPanel, "LDS is sized for kPanel");
+    // the split composition needs one row per lane and the Montgomery forms;
+    // the composition by pairs does not fit the registers with two rows of
+    // 64-bit words per lane
+    constexpr bool kMont = !std::is_same<Arith, BigArith>::value;
+    constexpr bool kFast = kMont && (H == 1 || sizeof(V) == 4);
+    constexpr bool kHalf = H == 1 && kMont;
     const int m = a.m, n = a.n;
     const Arith ar(a.mc);
     const int ms = m | 1;                   // odd row stride of At
     const int mn = m * n;
+    const int slots = window_slots(m, n, w, sizeof(V));
     // the composed panels' rows (16-byte aligned), 64-bit words (sh), then the
     // V arrays, then the int arrays (sizes as in window_lds_bytes, whose
     // coefficient buffers are sized for kPanel)
@@ -507,8 +534,8 @@ __global__ void __launch_bounds__(kStepThreads) mbasis_step_kernel(LeafArgs a, i
     V *At = reinterpret_cast<V *>(sh + m);                           // n x ms
     V *cof = At + n * ms;                                            // kMaxN: pivot cofactors
     V *scl = cof + kMaxN;                                            // m: row scales
-    V *Rw = scl + m;                                                 // w x m x n (w > 1)
-    int *perm = reinterpret_cast<int *>(Rw + (w > 1 ? w * mn : 0));  // m
+    V *Rw = scl + m;                                                 // slots x m x n
+    int *perm = reinterpret_cast<int *>(Rw + slots * mn);            // m
     int *plist = perm + m;                                           // m
     int *colpiv = plist + m;                                         // m (columns of At)
     int *pos = colpiv + m;                                           // m (then: pivot row by column)
@@ -516,8 +543,8 @@ __global__ void __launch_bounds__(kStepThreads) mbasis_step_kernel(LeafArgs a, i
     int *prow = delay + m;                                           // kMaxN (by rank)
     int *ispiv = prow + kMaxN;                                       // kMaxN (rows of At)
     // a composed panel: which columns took a pivot (and kFastPanel), the pivots'
-    // rows, the panel's own coefficient K0 and what its pivots' cofactors have
-    // from it (by pairs: 1 for the first two, D1 for the others)
+    // rows, the panel's own coefficient K0 and what its pivots' cofactors are made
+    // of (by pairs: 1 for the first two, D1 for the others; else the pivots)
     constexpr int kFastPanel = 1 << P;
     __shared__ int s_tk[2], s_prs[2][kPanel];
     __shared__ V s_K0[2], s_pre[2][kPanel];
@@ -555,13 +582,12 @@ __global__ void __launch_bounds__(kStepThreads) mbasis_step_kernel(LeafArgs a, i
         }
         return;
     }
-    if (w > 1)
-        for (int q = tid; q < w * mn; q += kStepThreads)
-            Rw[q] = ar.to(Arith::load(a.Rn + q));
+    for (int q = tid; q < slots * mn; q += kStepThreads)
+        Rw[q] = ar.to(Arith::load(a.Rn + q));
     // threads per row of the shift sort
     const int sortLog = m <= 64 ? 4 : m <= 128 ? 3 : 2;
     bool full = false;  // full-rank residual met (uniform)
-    int steps = 0;
+    int steps = 0, rank = 0;
     for (int s = 0; s < w && !full; ++s) {
         if (tid < m)
             colpiv[tid] = 0;
@@ -593,9 +619,9 @@ __global__ void __launch_bounds__(kStepThreads) mbasis_step_kernel(LeafArgs a, i
         // row of the residual per wave, two where they have at most 32 columns
         for (int i = n <= 32 ? tid >> 5 : wave; i < m; i += kStepThreads / (n <= 32 ? 32 : 64)) {
             const int pi = pos[i];
-            const size_t slot = w > 1 ? (size_t)(s - delay[i]) * mn : 0;
+            const size_t slot = slots > 0 ? (size_t)(s - delay[i]) * mn : 0;
             for (int j = n <= 32 ? tid & 31 : lane; j < n; j += 64)
-                At[j * ms + pi] = w > 1 ? Rw[slot + i * n + j] : ar.to(Arith::load(a.Rn + i * n + j));
+                At[j * ms + pi] = slots > 0 ? Rw[slot + i * n + j] : ar.to(Arith::load(a.Rn + i * n + j));
         }
         lds_barrier();
 
@@ -605,7 +631,7 @@ __global__ void __launch_bounds__(kStepThreads) mbasis_step_kernel(LeafArgs a, i
         // columns (the LDS operations of one wave take effect in program order)
         // while the other waves are still applying: one barrier per panel, with
         // the coefficients double-buffered.
-        int rank = 0;
+        rank = 0;
         // columns per wave: P times a power of two (so that cw divides the
         // wave's 64 lanes), 16 waves covering m
         int cw = P;
@@ -622,7 +648,7 @@ __global__ void __launch_bounds__(kStepThreads) mbasis_step_kernel(LeafArgs a, i
                 V pn[H][P], cc[H][P + 1];
                 bool isp[H], ok[H];
                 int prs[P] = {0};
-                V pre[P], prod = ar.one();  // product of the panel's earlier pivots
+                V pvs[P];
                 int tk = 0;  // panel columns that took a pivot
 #pragma unroll
                 for (int h = 0; h < H; ++h) {
@@ -704,8 +730,7 @@ __global__ void __launch_bounds__(kStepThreads) mbasis_step_kernel(LeafArgs a, i
                         isp[h] = isp[h] || me;
                     }
                     prs[j] = pr;
-                    pre[j] = prod;
-                    prod = ar.mul(prod, pv);
+                    pvs[j] = pv;
                     tk |= 1 << j;
                     ++nb;
                 };
@@ -731,12 +756,11 @@ __global__ void __launch_bounds__(kStepThreads) mbasis_step_kernel(LeafArgs a, i
                 }
                 if (lane == 0) {
                     s_tk[buf] = tk;
-                    s_K0[buf] = prod;
 #pragma unroll
                     for (int k = 0; k < P; ++k) {
                         s_prs[buf][k] = prs[k];
                         if (tk >> k & 1)
-                            s_pre[buf][k] = pre[k];
+                            s_pre[buf][k] = pvs[k];
                     }
                 }
             }
@@ -774,7 +798,7 @@ __global__ void __launch_bounds__(kStepThreads) mbasis_step_kernel(LeafArgs a, i
                 V C = P == 4 ? col(3) : (V)0;
                 bool isp = !hi && ok && ispiv[r];
                 int prs[P] = {0};
-                V pre[P], prod = ar.one();  // product of the panel's earlier pivots
+                V pvs[P];
                 int tk = 0, nb = 0;
                 // every lane gets the value of x in lane (lane & 31)
                 auto low = [](const V x) -> V {
@@ -867,8 +891,7 @@ __global__ void __launch_bounds__(kStepThreads) mbasis_step_kernel(LeafArgs a, i
                         C = me ? kp[2] : ts[2];
                     isp = isp || me;  // read in the lower half only
                     prs[j] = pr;
-                    pre[j] = prod;
-                    prod = ar.mul(prod, pv);
+                    pvs[j] = pv;
                     tk |= 1 << j;
                     ++nb;
                 };
@@ -898,12 +921,11 @@ __global__ void __launch_bounds__(kStepThreads) mbasis_step_kernel(LeafArgs a, i
                 }
                 if (lane == 0) {
                     s_tk[buf] = tk;
-                    s_K0[buf] = prod;
 #pragma unroll
                     for (int k = 0; k < P; ++k) {
                         s_prs[buf][k] = prs[k];
                         if (tk >> k & 1)
-                            s_pre[buf][k] = pre[k];
+                            s_pre[buf][k] = pvs[k];
                     }
                 }
             }
@@ -1070,12 +1092,6 @@ __global__ void __launch_bounds__(kStepThreads) mbasis_step_kernel(LeafArgs a, i
             }
             return true;
         };
-        // the split composition needs one row per lane and the Montgomery forms;
-        // the composition by pairs does not fit the registers with two rows of
-        // 64-bit words per lane
-        constexpr bool kMont = !std::is_same<Arith, BigArith>::value;
-        constexpr bool kFast = kMont && (H == 1 || sizeof(V) == 4);
-        constexpr bool kHalf = H == 1 && kMont;
         const bool half = kHalf && n <= 32;
         bool inorder = kFast;  // every panel so far by compose_fast (uniform)
         auto compose_panel = [&](const int c0, const int buf) __attribute__((always_inline)) {
@@ -1146,7 +1162,7 @@ __global__ void __launch_bounds__(kStepThreads) mbasis_step_kernel(LeafArgs a, i
             // rows in pairs (32-bit words: two rows of 64-bit words exceed the
             // registers), their loads before the products
             constexpr int RP = sizeof(V) == 4 ? 2 : 1;
-            const V K0 = s_K0[buf];  // slot 0 of every row (in order)
+            const V K0 = kFast ? s_K0[buf] : (V)0;  // slot 0 of every row (in order)
             for (int r = ag; r < n; r += RP * aG) {
                 V *x[RP];
                 Row cv[RP];
@@ -1186,17 +1202,30 @@ __global__ void __launch_bounds__(kStepThreads) mbasis_step_kernel(LeafArgs a, i
                 // pivot bookkeeping, off the composing wave's path: the pivots' rows
                 // and cofactors, read after the elimination, and their columns, read
                 // from the next panel's apply on
-                const V K0 = s_K0[buf];
+                // (q: the cofactor of this lane's pivot, dall the product past the panel;
+                // by pivots: the products of the earlier ones, one after the other
+                // here, where no pivot step waits for them)
+                V q = dall;
+                if (inorder) {
+                    if (lane >= 2)
+                        q = ar.mul(dall, s_pre[buf][0]);
+                    dall = ar.mul(dall, s_K0[buf]);
+                } else {
+#pragma unroll
+                    for (int c = 0; c < P; ++c)
+                        if (tk >> c & 1) {
+                            q = lane == c ? dall : q;
+                            dall = ar.mul(dall, s_pre[buf][c]);
+                        }
+                }
                 if (tk >> lane & 1) {
-                    const int q = rank + __popc(tk & ((1 << lane) - 1));
+                    const int at = rank + __popc(tk & ((1 << lane) - 1));
                     const int pr = inorder ? rank + lane : s_prs[buf][lane];
-                    const V pre = inorder ? (lane < 2 ? ar.one() : s_pre[buf][0]) : s_pre[buf][lane];
-                    prow[q] = pr;
-                    cof[q] = ar.mul(dall, pre);
+                    prow[at] = pr;
+                    cof[at] = q;
                     colpiv[k * P + lane] = 1;
                     pos[k * P + lane] = pr;
                 }
-                dall = ar.mul(dall, K0);
             }
             rank += nb;
             const int c1 = (k + 1) * P;
@@ -1206,13 +1235,13 @@ __global__ void __launch_bounds__(kStepThreads) mbasis_step_kernel(LeafArgs a, i
                 compose_panel(c1, buf ^ 1);
             lds_barrier();
         }
-        if (tid == kStepThreads - 64)
-            s_D = dall;
-        lds_barrier();
         // With D the product of the panels' own coefficients and cof[k] the cofactor
         // of pivot k (D over the pivot), the kernel vectors are D times the
         // normalised ones, and no inverse is needed in the step.  Pivots are
         // nonzero, so is D.
+        if (tid == kStepThreads - 64)
+            s_D = dall;
+        lds_barrier();
         const V D = s_D;
         // permutation list of left_nullspace_compact: pivot columns, then the
         // others; one wave counts the pivot columns before each column by ballots
@@ -1252,7 +1281,20 @@ __global__ void __launch_bounds__(kStepThreads) mbasis_step_kernel(LeafArgs a, i
                 cf[h] = r < rank ? cof[r] : (V)0;
                 xrow[h] = r < rank ? prow[r] * ms : 0;
             }
-            for (int t = wave; t < nullity; t += kStepThreads / 64) {
+            // (up to 32 pivots: a vector per 2^lg lanes)
+            const int lg = rank <= 32 ? 32 - __builtin_clz(2 * rank - 1) - 1 : 6;
+            if (lg < 6) {
+                const int r = tid & ((1 << lg) - 1);
+                const V cr = r < rank ? cof[r] : (V)0;
+                const int xr = r < rank ? prow[r] * ms : 0;
+                for (int t = tid >> lg; t < nullity && r < rank; t += kStepThreads >> lg) {
+                    const int col = plist[rank + t];
+                    const V v = ar.sub(0, ar.mul(At[xr + col], cr));
+                    At[xr + col] = v;
+                    X[(size_t)t * m + r] = v;
+                }
+            }
+            for (int t = wave; lg == 6 && t < nullity; t += kStepThreads / 64) {
                 const int col = plist[rank + t];
 #pragma unroll
                 for (int h = 0; h < RH; ++h) {
@@ -1395,7 +1437,8 @@ __global__ void __launch_bounds__(kStepThreads) mbasis_step_kernel(LeafArgs a, i
     if (tid == 0) {
         c[C_CUR] = cur;
         c[C_STEPS] = steps;
-        c[C_FLIP] = steps > 0 ? 1 : 0;
+        // (single orders: nothing to apply to a zero residual)
+        c[C_FLIP] = steps > 0 && (a.window > 1 || rank > 0) ? 1 : 0;
         if (full) {
             c[C_DONE] = 1;
             c[C_SHIFT] = a.ordL - (ord0 + steps);
@@ -1415,29 +1458,15 @@ __global__ void __launch_bounds__(kStepThreads) mbasis_step_kernel(LeafArgs a, i
 // read and written once per window instead of once per order, and the launch,
 // the control words' round trip and the tile's are paid once.  Order s leaves
 // the first s coefficients of the halo undefined.
-// STAGE: the window's kernel vectors are brought to LDS at the start, beside
-// the tile (rows padded with zeros to a multiple of kGroup), so that the orders
-// wait for no global load; without it (vectors too large for LDS) they are
-// read where they are.
+// The window's kernel vectors are brought to LDS at the start, beside the tile
+// (rows padded with zeros to a multiple of kGroup), so that the orders wait for
+// no global load.
 // Latency bounds it: 16.6 us per window of 4 orders (64 x 32, 32-bit words; 4 x
 // 7.4 to 9.5 with a launch per order), of which 2.3 are the loads, 1.5 each
-// order and the rest the launch's start and end.  18.5 us with the vectors read
-// from memory order by order.
+// order and the rest the launch's start and end.
 constexpr int kUpdateThreads = 512;
 constexpr int kGroup = 16;  // pivots taken together
-__host__ __device__ inline int pad16(int r)
-{
-    return (r + 15) & ~15;
-}
-// most words of one order's padded kernel vectors
-inline size_t staged_words(int m, int n)
-{
-    size_t most = 0;
-    for (int r = 1; r <= std::min(m, n); ++r)
-        most = std::max(most, (size_t)(m - r) * pad16(r));
-    return most;
-}
-template <typename Arith, bool STAGE>
+template <typename Arith>
 __global__ void __launch_bounds__(kUpdateThreads)
 mbasis_update_kernel(LeafArgs a, int ord0, int w, int wnext, int tilesB, int tilesR)
 {
@@ -1449,14 +1478,14 @@ mbasis_update_kernel(LeafArgs a, int ord0, int w, int wnext, int tilesB, int til
     V *Y = reinterpret_cast<V *>(smem);              // m x kTile
     int *pl = reinterpret_cast<int *>(Y + m * kTile);  // kWindow x m: row lists
     int *del = pl + kWindow * m;                     // m
-    V *Xs = reinterpret_cast<V *>(smem + update_lds_bytes(m, sizeof(V)));  // STAGE: vectors by order
+    V *Xs = reinterpret_cast<V *>(smem + update_lds_bytes(m, sizeof(V)));  // vectors by order
     const int q = tid % kTile, tg = tid / kTile;
     constexpr int TG = kUpdateThreads / kTile;
-    // STAGE: 2 x 2 entries per thread of 2 TG rows x 2 kTile entries of every
+    // 2 x 2 entries per thread of 2 TG rows x 2 kTile entries of every
     // order's vectors, all of them in flight at once; entry e of row t (in X's
     // bounds whatever the rank, which the first ones do not wait for)
     constexpr int XR = 2 * TG, XE = 2 * kTile;
-    V xv[STAGE ? kWindow : 1][2][2];
+    V xv[kWindow][2][2];
     auto fetch = [&](int tb, int eb) {
 #pragma unroll
         for (int s = 0; s < kWindow; ++s)
@@ -1467,8 +1496,7 @@ mbasis_update_kernel(LeafArgs a, int ord0, int w, int wnext, int tilesB, int til
                 xv[s][u >> 1][u & 1] = reinterpret_cast<const V *>(a.X)[x];
             }
     };
-    if constexpr (STAGE)
-        fetch(0, 0);
+    fetch(0, 0);
     const int steps = a.ctl[C_STEPS], cur = a.ctl[C_CUR], len = a.ctl[C_LEN];
     int ranks[kWindow];
     V D[kWindow];
@@ -1519,7 +1547,7 @@ mbasis_update_kernel(LeafArgs a, int ord0, int w, int wnext, int tilesB, int til
                     Y[(i0 + u * TG) * kTile + q] = in ? y[u] : (V)0;
         }
     }
-    if constexpr (STAGE) {
+    {
         int most = 0;  // entries of the longest vectors
 #pragma unroll
         for (int s = 0; s < kWindow; ++s) {
@@ -1566,8 +1594,7 @@ mbasis_update_kernel(LeafArgs a, int ord0, int w, int wnext, int tilesB, int til
             continue;  // zero residual: nothing to do at this order
         const int *ps = pl + s * m;
         const int nullity = m - rank;
-        const V *X = STAGE ? xstage : reinterpret_cast<const V *>(a.X) + (size_t)s * m * m;
-        const int xstride = STAGE ? pad16(rank) : m;
+        const int xstride = pad16(rank);
         // places of the pivot rows' coefficient q = 0, lane r for pivot r (past
         // the rank: the first row, with zero entries in the vectors)
         int ybase[RH];
@@ -1582,21 +1609,16 @@ mbasis_update_kernel(LeafArgs a, int ord0, int w, int wnext, int tilesB, int til
             // (q below s: coefficients already undefined, read as q = s)
             const int qq = q < s ? s : q, i = ps[rank + t];
             V *own = Y + i * kTile + qq - del[i];
-            const V *x = X + (size_t)t * xstride;
+            const V *x = xstage + (size_t)t * xstride;
             V sum = ar.mul(Ds, *own);
 #pragma unroll
             for (int h = 0; h < RH; ++h)
                 for (int r0 = 0; r0 < 64 && r0 + 64 * h < rank; r0 += kGroup) {
                     V v[kGroup], c[kGroup];
-                    if constexpr (STAGE)
-                        *reinterpret_cast<Group *>(c) = *reinterpret_cast<const Group *>(x + r0 + 64 * h);
+                    *reinterpret_cast<Group *>(c) = *reinterpret_cast<const Group *>(x + r0 + 64 * h);
 #pragma unroll
-                    for (int u = 0; u < kGroup; ++u) {
-                        const int r = r0 + u + 64 * h;
+                    for (int u = 0; u < kGroup; ++u)
                         v[u] = Y[__builtin_amdgcn_readlane(ybase[h], r0 + u) + qq];
-                        if constexpr (!STAGE)  // (past the row's end: within X's padding)
-                            c[u] = r < rank ? x[r] : (V)0;
-                    }
                     // two chains of eight products, the most one reduction takes
                     typename Arith::Acc p1 = ar.prod(c[0], v[0]), p2 = ar.prod(c[8], v[8]);
 #pragma unroll
@@ -1609,7 +1631,7 @@ mbasis_update_kernel(LeafArgs a, int ord0, int w, int wnext, int tilesB, int til
             if (q >= s)
                 *own = sum;  // (t = t0 twice: the same value again)
         }
-        xstage += nullity * pad16(rank);
+        xstage += nullity * xstride;
         __syncthreads();
         if (tid < rank)
             del[ps[tid]] += 1;
@@ -1648,6 +1670,124 @@ mbasis_update_kernel(LeafArgs a, int ord0, int w, int wnext, int tilesB, int til
         dst[e * stride + d] = v;
         if (!basis && d < ord0 + w + wnext)
             a.Rn[(size_t)(d - ord0 - w) * m * n + e] = v;  // the coming window
+    }
+}
+
+// base + sum_r X[t][r] * src[row piv[r], column j, coefficient d].  All loads
+// of a group of terms (32 words below 2^30, or 16 64-bit words: one L2 round
+// trip) are issued before its products, with no branch between them: terms
+// past the rank read row piv[r] of the LDS row list (padded with row 0 up to
+// kMaxM; rank <= kMaxN) and X words past the row (X carries kXPad words of
+// padding), and their X coefficient is zeroed by a select after the load.
+template <typename Arith>
+__device__ __forceinline__ typename Arith::V row_combo(const Arith &ar, const uint64_t *src,
+                                                       const typename Arith::V *xr, const int *piv,
+                                                       int rank, int stride, int cols, int j, int d,
+                                                       typename Arith::V base)
+{
+    using V = typename Arith::V;
+    const uint64_t *sj = src + (size_t)j * stride + d;
+    const size_t rstride = (size_t)cols * stride;
+    constexpr int G = sizeof(V) == 4 ? 32 : 16;
+    V acc = base;
+    for (int r = 0; r < rank; r += G) {
+        V sv[G], xv[G];
+#pragma unroll
+        for (int u = 0; u < G; ++u) {
+            sv[u] = Arith::load(sj + (size_t)piv[r + u] * rstride);
+            const V x = xr[r + u];
+            xv[u] = r + u < rank ? x : (V)0;
+        }
+#pragma unroll
+        for (int h = 0; h < G; h += 8) {  // eight products, the most one reduction takes
+            typename Arith::Acc part = ar.prod(xv[h], sv[h]);
+#pragma unroll
+            for (int u = 1; u < 8; ++u)
+                part = ar.fma(part, xv[h + u], sv[h + u]);
+            acc = ar.add(acc, ar.reduce(part));
+        }
+    }
+    return acc;
+}
+
+// The same for single orders: a thread per coefficient of appbas and of the
+// residual's later coefficients, read from and written to memory.  There is
+// nothing to keep in LDS between orders, no halo and no place of a tile past the
+// basis's length, and the kernel rows spread over the chip, where a tile takes
+// all of a column's.  Step plus update per order, single orders / windows of 2 as
+// the tiles take them: 78 / 127 us (192 x 24, 64-bit words), 30 / 81 (256 x 1, the
+// same), 90 / 125 (100 x 25, p > 2^62).
+template <typename Arith>
+__global__ void __launch_bounds__(256) mbasis_update1_kernel(LeafArgs a, int ord)
+{
+    // The control words, the order's row list and its factor D are all
+    // requested at entry, before any branch on them.
+    using V = typename Arith::V;
+    static_assert(kMaxM == 256, "one row-list entry per thread of the 256-thread workgroup");
+    const int m = a.m, n = a.n, cap = a.cap, tx = threadIdx.x;
+    const int steps = a.ctl[C_STEPS], cur = a.ctl[C_CUR], L = a.ctl[C_LEN], rank = a.ctl[C_RANK];
+    const V D = (V)a.scale[m];
+    const int piv_t = tx < m ? a.piv[tx] : 0;  // groups read up to kMaxM entries
+    if (steps == 0)
+        return;
+    const unsigned tstride = gridDim.x * blockDim.x;
+    const unsigned t0 = blockIdx.x * blockDim.x + tx;
+    const uint64_t *rs = a.R[cur];
+    if (rank == 0) {
+        // residual unchanged: the coming order's coefficient is ord + 1
+        if (ord + 1 < a.ordL)
+            for (unsigned e = t0; e < (unsigned)(m * n); e += tstride)
+                a.Rn[e] = rs[(size_t)e * a.ordL + ord + 1];
+        return;
+    }
+    __shared__ int piv[kMaxM], role[kMaxM];  // role: t of a kernel row, -1 of a pivot row
+    piv[tx] = piv_t;
+    if (tx < m)
+        role[piv_t] = tx < rank ? -1 : tx - rank;
+    __syncthreads();
+    const Arith ar(a.mc);
+    const V *X = reinterpret_cast<const V *>(a.X);
+    const uint64_t *src = a.app[cur];
+    uint64_t *dst = a.app[cur ^ 1], *rd = a.R[cur ^ 1];
+    const unsigned L1 = (unsigned)(L + 1 <= cap ? L + 1 : cap);
+    const unsigned items = (unsigned)(m * m) * L1;
+    const int spn = a.ordL - ord - 1;
+    const unsigned span = spn > 0 ? (unsigned)spn : 0u;
+    const unsigned ritems = (unsigned)(m * n) * span;
+    // one index space, basis items then residual items: with the grid sized
+    // for both, a thread has one item
+    for (unsigned idx = t0; idx < items + ritems; idx += tstride) {
+        if (idx < items) {
+            const unsigned e = idx / L1;
+            const int d = (int)(idx - e * L1);
+            const int i = (int)(e / (unsigned)m), j = (int)(e - (unsigned)i * m);
+            const int t = role[i];
+            const uint64_t *x = src + (size_t)e * cap + d;
+            uint64_t v;
+            if (t >= 0) {
+                v = d < L ? row_combo<Arith>(ar, src, X + (size_t)t * m, piv, rank, cap, m, j, d,
+                                             ar.mul(D, Arith::load(x)))
+                          : 0;
+            } else {
+                v = d >= 1 ? x[-1] : 0;
+                if (d == L && v != 0)
+                    a.lens[0] = L + 1;
+            }
+            dst[(size_t)e * cap + d] = v;
+        } else {
+            const unsigned k = idx - items;
+            const unsigned e = k / span;
+            const int d = ord + 1 + (int)(k - e * span);
+            const int i = (int)(e / (unsigned)n), j = (int)(e - (unsigned)i * n);
+            const int t = role[i];
+            const uint64_t *x = rs + (size_t)e * a.ordL + d;
+            const uint64_t v = t >= 0 ? row_combo<Arith>(ar, rs, X + (size_t)t * m, piv, rank, a.ordL, n, j, d,
+                                                         ar.mul(D, Arith::load(x)))
+                                      : x[-1];
+            rd[(size_t)e * a.ordL + d] = v;
+            if (d == ord + 1)
+                a.Rn[e] = v;  // the coming order's coefficient
+        }
     }
 }
 
@@ -1790,7 +1930,9 @@ pmlg_status leaf(pmlg_ctx ctx, Arena &ar, const uint64_t *F, int64_t strideF, in
     if (step_lds_bytes(m, n, wbytes) > kStepLdsMax)
         return fail(PMLG_ERR_UNSUPPORTED, "M-Basis: an m x n residual of this size does not fit "
                                           "the step kernel's LDS");
-    const int W = window_orders(m, n, wbytes);
+    const int W = mbasis_window(small ? BASIS_W32 : big ? BASIS_ANY : BASIS_W64, m, n, ordL,
+                                window_orders(m, n, wbytes));
+    a.window = W;
     a.Rn = ar.alloc((size_t)m * n * W);
     a.scale = ar.alloc((size_t)m + kWindow);
     a.X = ar.alloc((size_t)m * m * W + kXPad);
@@ -1813,9 +1955,9 @@ pmlg_status leaf(pmlg_ctx ctx, Arena &ar, const uint64_t *F, int64_t strideF, in
                                  (const void *)mbasis_step_kernel<Mont32Arith, 2>,
                                  (const void *)mbasis_step_kernel<BigArith, 1>,
                                  (const void *)mbasis_step_kernel<BigArith, 2>,
-                                 (const void *)mbasis_update_kernel<Mont64Arith, true>,
-                                 (const void *)mbasis_update_kernel<Mont32Arith, true>,
-                                 (const void *)mbasis_update_kernel<BigArith, true>};
+                                 (const void *)mbasis_update_kernel<Mont64Arith>,
+                                 (const void *)mbasis_update_kernel<Mont32Arith>,
+                                 (const void *)mbasis_update_kernel<BigArith>};
         constexpr int nk = sizeof(kernels) / sizeof(kernels[0]);
         static std::atomic<uint64_t> raised[nk];
         for (int i = 0; i < nk; ++i)
@@ -1823,9 +1965,8 @@ pmlg_status leaf(pmlg_ctx ctx, Arena &ar, const uint64_t *F, int64_t strideF, in
     }
     // rows of the transposed residual per lane of the composing wave
     const bool one_row = n <= 64;
-    const size_t xbytes = staged_words(m, n) * W * wbytes;
-    const bool stage = update_lds_bytes(m, wbytes) + xbytes <= kLds;
-    const size_t ulds = update_lds_bytes(m, wbytes) + (stage ? xbytes : 0);
+    const size_t ulds = update_lds_bytes(m, wbytes) + staged_words(m, n) * W * wbytes;
+    const unsigned grid1 = grid_for((int64_t)m * m * cap + (int64_t)m * n * ordL);
     for (int ord = 0; ord < ordL; ord += W) {
         const int w = std::min(W, ordL - ord), wnext = std::min(W, ordL - ord - w);
         const size_t lds = window_lds_bytes(m, n, w, wbytes);
@@ -1840,9 +1981,11 @@ pmlg_status leaf(pmlg_ctx ctx, Arena &ar, const uint64_t *F, int64_t strideF, in
             hipLaunchKernelGGL((one_row ? mbasis_step_kernel<typename A::type, 1>
                                         : mbasis_step_kernel<typename A::type, 2>),
                                dim3(1), dim3(kStepThreads), lds, s, a, ord, w);
-            hipLaunchKernelGGL((stage ? mbasis_update_kernel<typename A::type, true>
-                                      : mbasis_update_kernel<typename A::type, false>),
-                               ugrid, dim3(kUpdateThreads), ulds, s, a, ord, w, wnext, tilesB, tilesR);
+            if (W == 1)
+                hipLaunchKernelGGL(mbasis_update1_kernel<typename A::type>, dim3(grid1), dim3(256), 0, s, a, ord);
+            else
+                hipLaunchKernelGGL(mbasis_update_kernel<typename A::type>, ugrid, dim3(kUpdateThreads), ulds, s,
+                                   a, ord, w, wnext, tilesB, tilesR);
         };
         if (small)
             launch(Tag<Mont32Arith>{});
