@@ -9,6 +9,7 @@
 
 #include "ctx.hpp"
 #include "host_arith.hpp"
+#include "rules.hpp"
 
 using namespace pmlg;
 
@@ -375,7 +376,8 @@ pmlg_status check_ctx(pmlg_ctx ctx)
     return PMLG_OK;
 }
 
-pmlg_status pick_kind(pmlg_ctx ctx, int method, int64_t m, int64_t k, int64_t n,
+// Pointwise kernel for an m x k by k x n product at `points` points.
+pmlg_status pick_kind(pmlg_ctx ctx, int method, int64_t m, int64_t k, int64_t n, int64_t points,
                       PointwiseKind *kind)
 {
     if (method == PMLG_METHOD_PLAIN) {
@@ -387,7 +389,7 @@ pmlg_status pick_kind(pmlg_ctx ctx, int method, int64_t m, int64_t k, int64_t n,
         *kind = PW_MFMA;
     } else if (method == PMLG_METHOD_AUTO) {
         *kind = mfma_exact((int)m, (int)k, (int)n, ctx->mc.limbs, ctx->p) &&
-                        mfma_pays((int)m, (int)k, (int)n, ctx->mc.limbs)
+                        mfma_pays((int)m, (int)k, (int)n, points, ctx->mc.limbs)
                     ? PW_MFMA
                     : PW_PLAIN;
     } else {
@@ -437,7 +439,7 @@ pmlg_status mulmid_dev_strided(pmlg_ctx ctx, uint64_t *dOut, int64_t out_stride,
                            hi_eff, method, s);
     }
     PointwiseKind kind;
-    pmlg_status st = pick_kind(ctx, method, m, k, n, &kind);
+    pmlg_status st = pick_kind(ctx, method, m, k, n, (int64_t)1 << logN, &kind);
     if (st != PMLG_OK)
         return st;
     if (hi_eff < nhi)  // coefficients beyond the product length are zero
@@ -717,7 +719,7 @@ pmlg_status pmlg_polmat_mul_dev_noalloc(pmlg_ctx ctx, uint64_t *dC, const uint64
                         " are not built on this context; any earlier product of that transform "
                         "length on it (e.g. one pmlg_polmat_mul_dev call) builds them");
     PointwiseKind kind;
-    st = pick_kind(ctx, method, m, k, n, &kind);
+    st = pick_kind(ctx, method, m, k, n, (int64_t)1 << logN, &kind);
     if (st != PMLG_OK)
         return st;
     if (ctx->small)

@@ -4,7 +4,7 @@
 // A plan groups the products by what a launch can share:
 //   * forward transforms by (modulus, transform length, radix): one
 //     segment-table launch per group covers every entry of every operand;
-//   * pointwise products by (modulus, kernel, points per task): one
+//   * pointwise products by (modulus, kernel, points per task or rows): one
 //     persistent launch per group walks the task list of all its products;
 //   * inverse transforms by (modulus, length, radix, output scaling);
 //   * short products by direct (schoolbook) convolution, one persistent
@@ -303,7 +303,7 @@ struct InvGroup {
 struct PwGroup {
     pmlg_ctx ctx;
     PointwiseKind kind;
-    int pt;  // points per MFMA task
+    int pt;  // points per MFMA task, rows of a plain tile
     size_t seg_off;
     int nseg;
     int64_t blocks;
@@ -514,7 +514,8 @@ void add_segments(const pmlg_mul_desc &d, const ProdInfo &pi, unsigned char *are
     const bool redc = sizeof(W) == 8;
     inv[{ctx, logN, cf.inv_e, (redc ? 1 : 0) | (trunc << 1)}].push_back(
         InvSeg<W, uint64_t>{Ch, d.C, tmp, lenC, 0, lenC, d.m * d.n, 0, 0, trunc, 0});
-    const int pt = cf.kind == PW_MFMA ? pw_points(sizeof(W), logP, cf.single_pt != 0) : 0;
+    const int pt = cf.kind == PW_MFMA ? pw_points(sizeof(W), logP, cf.single_pt != 0)
+                                            : pw_plain_rows((int)d.m, N);
     PwSeg<W> ps{};
     ps.Ah = Ah;
     ps.Bh = Bh;

@@ -223,11 +223,10 @@ hipError_t launch_pointwise(PointwiseKind kind, const W *Ah, const W *Bh, W *Ch,
                             int n, int64_t N, int logP, int logPc, const ModConst &mc,
                             hipStream_t s);
 
-// Whether the int8-digit MFMA kernel is exact for this shape and modulus,
-// whether it is the faster of the two where it is, and whether an explicit
+// Whether the int8-digit MFMA kernel is exact for this shape and modulus (then
+// mfma_pays tells whether it is the faster of the two), and whether an explicit
 // request for it (method or configuration) is accepted.
 bool mfma_exact(int m, int k, int n, int limbs, uint64_t p);
-bool mfma_pays(int m, int k, int n, int limbs);
 bool mfma_supported(int m, int k, int n, int limbs, uint64_t p);
 
 // One product of a batched pointwise launch (evaluations in blocked layout,
@@ -242,10 +241,13 @@ struct PwSeg {
 };
 // points per task of the MFMA kernel: 16 bytes of a run, or one
 int pw_points(int elem_bytes, int logP, bool single);
+// rows of the plain kernel's tiles, 2 or 4, and blocks of either kernel with pt
+// points per task or rows
+int pw_plain_rows(int m, int64_t N);
 int64_t pw_seg_blocks(PointwiseKind kind, int pt, int m, int n, int64_t N);
 // Persistent launch over all blocks of nseg products sharing one prime:
 // `grid` workgroups (0: one per block) walk the block list; MFMA tasks take
-// pt points each.
+// pt points each, plain tiles have pt rows.
 template <typename W>
 hipError_t launch_pointwise_segs(PointwiseKind kind, int pt, const PwSeg<W> *segs, int nseg,
                                  int64_t blocks, int grid, const ModConst &mc, hipStream_t s);

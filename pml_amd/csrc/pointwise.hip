@@ -16,6 +16,7 @@
 // inverse's lazy and strict butterflies need; 32-bit words are reduced to [0, p) by
 // Barrett steps.  No floating point is involved.
 #include "internal.hpp"
+#include "rules.hpp"
 
 namespace pmlg {
 
@@ -38,10 +39,12 @@ constexpr int kMfmaWaves = PT == 1 ? 4 : 2;
 // ---------------------------------------------------------------------------
 // plain kernel
 // ---------------------------------------------------------------------------
-// Outputs per lane.  A lane works on one point, so the wave's 64 lanes read
-// 16 (8) neighbouring runs of each entry and the lines' other entries come
-// with the next kk or column from L1.
-constexpr int TM = 4, TN = 4;
+// Outputs per lane: TM x TN, TM = 2 or 4 (plain_rows).  A lane works on one
+// point, so the wave's 64 lanes read 16 (8) neighbouring runs of each entry and
+// the lines' other entries come with the next kk or column from L1.  Four rows
+// read less per product; two leave registers for twice the waves, which hide the
+// loads' latency, and waste less on a few rows.
+constexpr int TN = 4;
 
 // V 2^-64 mod p of a 128-bit sum of at most 15 products and a residue
 // (Montgomery REDC; the inverse transform's scaling undoes the 2^-64): below
@@ -56,8 +59,9 @@ __device__ __forceinline__ uint64_t plain_redc(uint64_t hi, uint64_t lo, const M
 }
 
 // Lane (point q, output tile `tile` of TM x TN entries) of the plain product.
-// Rows and columns past the matrix read its last one and are not stored.
-template <typename W>
+// Rows and columns past the matrix are not stored; tiles of four rows read the
+// last ones instead, tiles of two none.
+template <typename W, int TM>
 __device__ __forceinline__ void plain_body(const W *__restrict__ Ah, const W *__restrict__ Bh,
                                            W *__restrict__ Ch, int m, int k, int n, int64_t N,
                                            int logP, int logPc, const ModConst &mc, int64_t q,
@@ -73,10 +77,10 @@ __device__ __forceinline__ void plain_body(const W *__restrict__ Ah, const W *__
     const W *pa[TM], *pb[TN];
 #pragma unroll
     for (int r = 0; r < TM; ++r)
-        pa[r] = Ah + (((run * m + min(i0 + r, m - 1)) * k) << logP) + off;
+        pa[r] = Ah + (((run * m + (TM == 4 ? min(i0 + r, m - 1) : i0 + r)) * k) << logP) + off;
 #pragma unroll
     for (int c = 0; c < TN; ++c)
-        pb[c] = Bh + ((run * k * n + min(j0 + c, n - 1)) << logP) + off;
+        pb[c] = Bh + ((run * k * n + (TM == 4 ? min(j0 + c, n - 1) : j0 + c)) << logP) + off;
     const int64_t bstep = (int64_t)n << logP;
     uint64_t hi[TM][TN], lo[TM][TN];  // 32-bit words: lo only
 #pragma unroll
@@ -106,10 +110,10 @@ __device__ __forceinline__ void plain_body(const W *__restrict__ Ah, const W *__
             W a[TM], b[TN];
 #pragma unroll
             for (int r = 0; r < TM; ++r)
-                a[r] = pa[r][(int64_t)kk << logP];
+                a[r] = TM == 4 || i0 + r < m ? pa[r][(int64_t)kk << logP] : (W)0;
 #pragma unroll
             for (int c = 0; c < TN; ++c)
-                b[c] = pb[c][kk * bstep];
+                b[c] = TM == 4 || j0 + c < n ? pb[c][kk * bstep] : (W)0;
 #pragma unroll
             for (int r = 0; r < TM; ++r)
 #pragma unroll
@@ -137,14 +141,14 @@ __device__ __forceinline__ void plain_body(const W *__restrict__ Ah, const W *__
 }
 
 // grid: x = 64-point chunks, y = groups of 4 output tiles (one per wave)
-template <typename W>
+template <typename W, int TM>
 __global__ void __launch_bounds__(kThreads)
 pw_plain(const W *__restrict__ Ah, const W *__restrict__ Bh, W *__restrict__ Ch, int m, int k,
          int n, int64_t N, int logP, int logPc, ModConst mc)
 {
     const int64_t q = (int64_t)blockIdx.x * 64 + (threadIdx.x & 63);
     const int tile = blockIdx.y * (kThreads / 64) + (threadIdx.x >> 6);
-    plain_body<W>(Ah, Bh, Ch, m, k, n, N, logP, logPc, mc, q, tile);
+    plain_body<W, TM>(Ah, Bh, Ch, m, k, n, N, logP, logPc, mc, q, tile);
 }
 
 // ---------------------------------------------------------------------------
@@ -573,7 +577,7 @@ pw_mfma_segs(const PwSeg<W> *__restrict__ segs, int nseg, int64_t blocks, ModCon
 }
 
 // task = (64-point chunk, group of 4 output tiles) of one product
-template <typename W>
+template <typename W, int TM>
 __global__ void __launch_bounds__(kThreads)
 pw_plain_segs(const PwSeg<W> *__restrict__ segs, int nseg, int64_t blocks, ModConst mc)
 {
@@ -584,7 +588,7 @@ pw_plain_segs(const PwSeg<W> *__restrict__ segs, int nseg, int64_t blocks, ModCo
         const int64_t by = lb / gx;
         const int64_t q = (lb - by * gx) * 64 + (threadIdx.x & 63);
         const int tile = (int)by * kWaves + (threadIdx.x >> 6);
-        plain_body<W>(as_global(sg.Ah), as_global(sg.Bh), as_global(sg.Ch), sg.m, sg.k, sg.n, sg.N, sg.logP,
+        plain_body<W, TM>(as_global(sg.Ah), as_global(sg.Bh), as_global(sg.Ch), sg.m, sg.k, sg.n, sg.N, sg.logP,
                       sg.logPc, mc, q, tile);
     }
 }
@@ -599,6 +603,22 @@ hipError_t launch_mfma_pt(const W *Ah, const W *Bh, W *Ch, int m, int k, int n, 
         return hipErrorInvalidValue;
     hipLaunchKernelGGL((pw_mfma_kernel<W, PT>), dim3((unsigned)grid), dim3(kThreads), 0, s, Ah, Bh,
                        Ch, m, k, n, N, blocks, logP, logPc, mc);
+    return hipGetLastError();
+}
+
+// groups of kWaves output tiles of `rows` rows
+inline int64_t plain_groups(int m, int n, int rows)
+{
+    return ((int64_t)((m + rows - 1) / rows) * ((n + TN - 1) / TN) + kWaves - 1) / kWaves;
+}
+
+template <typename W, int TM>
+hipError_t launch_plain(const W *Ah, const W *Bh, W *Ch, int m, int k, int n, int64_t N, int logP,
+                        int logPc, const ModConst &mc, hipStream_t s)
+{
+    const dim3 grid((unsigned)((N + 63) / 64), (unsigned)plain_groups(m, n, TM));
+    hipLaunchKernelGGL((pw_plain<W, TM>), grid, dim3(kThreads), 0, s, Ah, Bh, Ch, m, k, n, N, logP, logPc,
+                       mc);
     return hipGetLastError();
 }
 
@@ -618,11 +638,9 @@ hipError_t launch_pointwise_w(PointwiseKind kind, const W *Ah, const W *Bh, W *C
             return launch_mfma_pt<W, kPoints<W>>(Ah, Bh, Ch, m, k, n, N, logP, logPc, mc, s);
         return launch_mfma_pt<W, 1>(Ah, Bh, Ch, m, k, n, N, logP, logPc, mc, s);
     }
-    const int tiles = ((m + TM - 1) / TM) * ((n + TN - 1) / TN);
-    dim3 grid((unsigned)((N + 63) / 64), (unsigned)((tiles + kWaves - 1) / kWaves));
-    hipLaunchKernelGGL(pw_plain<W>, grid, dim3(kThreads), 0, s, Ah, Bh, Ch, m, k, n, N, logP, logPc,
-                       mc);
-    return hipGetLastError();
+    if (plain_rows(m, N, plain_waves(m, n, N)) == 4)
+        return launch_plain<W, 4>(Ah, Bh, Ch, m, k, n, N, logP, logPc, mc, s);
+    return launch_plain<W, 2>(Ah, Bh, Ch, m, k, n, N, logP, logPc, mc, s);
 }
 
 }  // namespace
@@ -644,26 +662,6 @@ bool mfma_exact(int m, int k, int n, int limbs, uint64_t p)
         limbs == 8 ? (~(unsigned __int128)0) - ((unsigned __int128)(p + 1) << 64)
                    : ((unsigned __int128)1 << 72);
     return sq == 0 || (unsigned __int128)k <= lim / sq;
-}
-
-// Cost of both kernels per 64 points, in units of about 10 ps on one MI355X:
-// the plain kernel's 4 x 4 tiles take a fixed part and one per kk, the MFMA
-// kernel's 16 x 16 tiles a fixed part (folding and reducing the outputs) and
-// one per chunk of 16 kk, whatever part of a tile the matrix fills.  Fitted
-// to 42 shapes from 2 x 2 x 2 to 64 x 64 x 64; on those the rule takes the
-// slower kernel only where both are within 10% of each other.  Measured
-// (us, plain / MFMA, 64-bit words): 4 x 4 x 4 at 2^19 points 51 / 390, 8 x 8 x 8
-// at 2^17 58 / 117, 12 x 12 x 12 at 2^16 95 / 76, 32 x 32 x 32 at 2^13 175 / 48;
-// 32-bit words: 8 x 8 x 8 26 / 68, 20 x 20 x 20 at 2^15 66 / 87, 32 x 32 x 32
-// 49 / 30.
-bool mfma_pays(int m, int k, int n, int limbs)
-{
-    const double tp = (double)((m + TM - 1) / TM) * ((n + TN - 1) / TN);
-    const double tm = (double)((m + 15) / 16) * ((n + 15) / 16);
-    const int kc = (k + 15) / 16;
-    if (limbs == 8)
-        return tm * (2080 + 2680 * kc) < tp * (150 + 72.0 * k);
-    return tm * (2000 + 950 * kc) < tp * (80 + 17.0 * k);
 }
 
 bool mfma_supported(int m, int k, int n, int limbs, uint64_t p)
@@ -691,6 +689,12 @@ hipError_t launch_pointwise<uint32_t>(PointwiseKind kind, const uint32_t *Ah, co
 // ---------------------------------------------------------------------------
 // batched launches
 // ---------------------------------------------------------------------------
+int pw_plain_rows(int m, int64_t N)
+{
+    // (the other products of the launch fill the chip)
+    return plain_rows(m, N, INT64_MAX);
+}
+
 int pw_points(int elem_bytes, int logP, bool single)
 {
     const int pt = 16 / elem_bytes;
@@ -701,8 +705,7 @@ int64_t pw_seg_blocks(PointwiseKind kind, int pt, int m, int n, int64_t N)
 {
     if (kind == PW_MFMA)
         return (MfmaTasks(m, n, N, pt).total + kWaves - 1) / kWaves;
-    const int tiles = ((m + TM - 1) / TM) * ((n + TN - 1) / TN);
-    return ((N + 63) / 64) * ((tiles + kWaves - 1) / kWaves);
+    return ((N + 63) / 64) * plain_groups(m, n, pt);
 }
 
 template <typename W>
@@ -714,8 +717,14 @@ hipError_t launch_pointwise_segs(PointwiseKind kind, int pt, const PwSeg<W> *seg
     if (kind == PW_PLAIN) {
         if (grid <= 0 || grid > blocks)
             grid = (int)(blocks < (1 << 30) ? blocks : (1 << 30));
-        hipLaunchKernelGGL(pw_plain_segs<W>, dim3((unsigned)grid), dim3(kThreads), 0, s, segs, nseg,
-                           blocks, mc);
+        if (pt == 4)
+            hipLaunchKernelGGL((pw_plain_segs<W, 4>), dim3((unsigned)grid), dim3(kThreads), 0, s, segs,
+                               nseg, blocks, mc);
+        else if (pt == 2)
+            hipLaunchKernelGGL((pw_plain_segs<W, 2>), dim3((unsigned)grid), dim3(kThreads), 0, s, segs,
+                               nseg, blocks, mc);
+        else
+            return hipErrorInvalidValue;
         return hipGetLastError();
     }
     if (mc.limbs != (int)sizeof(W))

@@ -8,6 +8,47 @@
 
 namespace pmlg {
 
+// Waves of the plain pointwise kernel for m x n outputs at N points in tiles of 4 x 4.
+inline int64_t plain_waves(int m, int n, int64_t N)
+{
+    return (N + 63) / 64 * ((m + 3) / 4) * ((n + 3) / 4);
+}
+
+// Rows of a lane's tile in the plain kernel at N points.  Two below 2048 waves of
+// four rows (two per SIMD) or with idle lanes, where the loads' latency bounds it,
+// and for up to 6 rows.
+// Microseconds, four / two rows, 64-bit words: 1 x 64 x 1 at 2^16 points 80 / 34,
+// 4 x 32 x 4 at 2^16 53 / 37, 64 x 64 x 64 at 2^8 71 / 61; 12 x 8 x 12 at 2^16 63 /
+// 66, 64 x 32 x 64 at 2^12 334 / 364; 200 x 200 x 200 at one point (transforms
+// included) 515 / 415; 32-bit words: 64 x 64 x 64 at 2^10 43 / 61.
+// (Two rows were the old kernel's; four everywhere had cost the small products
+// up to half their speed.)
+inline int plain_rows(int m, int64_t N, int64_t waves)
+{
+    return N >= 64 && waves >= 2048 && m > 6 ? 4 : 2;
+}
+
+// Whether the MFMA kernel is the faster one where both are exact: its time and the
+// plain kernel's in nanoseconds, a start and a chain (the loads of a step of 16, or
+// of one, of the inner dimension, one after another) plus what each task (a tile of
+// 16 x 16 outputs at 16 bytes of points) or wave adds.  Fitted (least squares) to
+// 1280 shapes from 1 x 2 x 1 to 64 x 64 x 64 at 2 to 2^16 points, on which the rule
+// takes the slower kernel by more than 15% and 2 us nine times.  Without the starts
+// and chains products too small to fill the chip took the plain kernel where MFMA is
+// up to five times as fast (us, plain / MFMA, 64-bit words: 4 x 200 x 4 at 2 points
+// 147 / 13, 8 x 8 x 8 at 2 points 13 / 4; 8 x 8 x 8 at 2^16 points 28 / 59, 32 x 32 x
+// 32 at 2^13 175 / 48; 32-bit words: 4 x 64 x 5 at 2^12 21 / 7, 8 x 8 x 8 at 2^16
+// 13 / 38).
+inline bool mfma_pays(int m, int k, int n, int64_t N, int limbs)
+{
+    const double steps = (k + 15) / 16;
+    const double tasks = (double)((m + 15) / 16) * ((n + 15) / 16) * std::max<int64_t>(1, limbs == 8 ? N / 2 : N / 4);
+    const double waves = (double)plain_waves(m, n, N);
+    if (limbs == 8)
+        return 2740 + 790 * steps + tasks * (1.07 + 0.50 * steps) < 2630 + 540.0 * k + waves * (1.49 + 0.26 * k);
+    return 2900 + 510 * steps + tasks * (1.65 + 0.41 * steps) < 2310 + 259.0 * k + waves * (1.02 + 0.079 * k);
+}
+
 // Orders per launch of the M-Basis step kernel (1: single orders, applied by a
 // thread per coefficient instead of in LDS tiles) for m x n residuals, in a leaf
 // of order ordL, when at most `most` fit LDS.
