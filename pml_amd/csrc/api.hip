@@ -430,7 +430,7 @@ pmlg_status mulmid_dev_strided(pmlg_ctx ctx, uint64_t *dOut, int64_t out_stride,
     const int64_t lc = la + lb - 1;
     // cyclic length: no wrapped term may land in [nlo, hi_eff)
     int64_t need = hi_eff > lc - nlo ? hi_eff : lc - nlo;
-    const int logN = transform_log(need);
+    const int logN = ceil_log2(need);
     if (logN > ctx->max_log) {
         // no 2^logN-th root of unity mod p (or p composite): multi-prime path
         if (hi_eff < nhi)
@@ -707,7 +707,7 @@ pmlg_status pmlg_polmat_mul_dev_noalloc(pmlg_ctx ctx, uint64_t *dC, const uint64
         HIP_TRY(fill_zero(dC, m * n * lenC, s), "fill_zero");
         return PMLG_OK;
     }
-    const int logN = transform_log(lenC);
+    const int logN = ceil_log2(lenC);
     if (logN > ctx->max_log)
         return fail(PMLG_ERR_UNSUPPORTED,
                     "pmlg_polmat_mul_dev_noalloc: transform length 2^" + std::to_string(logN) +

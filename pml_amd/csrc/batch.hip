@@ -687,7 +687,7 @@ pmlg_status build_plan(pmlg_batch_plan *out, const pmlg_mul_desc *descs, int64_t
             school[d.ctx].push_back(SchoolSeg{d.A, d.B, d.C, d.m, d.k, d.n, d.lenA, d.lenB, 0});
             continue;
         }
-        pi.logN = transform_log(lenC);
+        pi.logN = ceil_log2(lenC);
         const size_t w = d.ctx->small ? 4 : 8;
         const int64_t N = (int64_t)1 << pi.logN;
         pi.ah = take((size_t)(d.m * d.k * N) * w) / w;
@@ -865,7 +865,7 @@ pmlg_status time_configs(pmlg_ctx ctx, int64_t m, int64_t k, int64_t n, int64_t 
     DeviceGuard g(ctx->device);
     hipStream_t s = ctx->stream;
     const int64_t lenC = lenA + lenB - 1;
-    const int64_t N = (int64_t)1 << transform_log(lenC);
+    const int64_t N = (int64_t)1 << ceil_log2(lenC);
     // A plan runs each configuration's products inside launches shared with
     // many others, so a product is timed among `copies` identical ones (same
     // inputs, own outputs and evaluations) in one plan: enough copies that the

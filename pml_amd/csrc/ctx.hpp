@@ -140,12 +140,6 @@ struct pmlg_ctx_s {
 namespace pmlg {
 
 int ceil_log2(int64_t x);
-// log2 of the transform length for `len` coefficients (at least 1: the
-// transforms have two points or more)
-inline int transform_log(int64_t len)
-{
-    return len <= 2 ? 1 : ceil_log2(len);
-}
 pmlg_status check_ctx(pmlg_ctx ctx);
 hipError_t fill_zero(uint64_t *p, int64_t n, hipStream_t s);
 // Coefficients [nlo, nhi) of A*B into dOut (padded length nhi - nlo), device

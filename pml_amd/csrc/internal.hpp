@@ -139,7 +139,7 @@ inline bool trunc_ok(int logN, int64_t lenC)
 
 // Forward transforms of one or two operands in one launch: `count` entries
 // each, entry e reads in[e*in_stride + i] for i < in_len (zero beyond), writes
-// its N evaluations in blocked layout (the first 3N/4 when trunc).  logN >= 1.
+// its N evaluations in blocked layout (the first 3N/4 when trunc).
 // Transforms longer than 4 times the LDS limit run a column pass first into
 // tmp (the larger count times N words of Win) with the tables ct.
 template <typename Win, typename W>

@@ -1245,12 +1245,34 @@ ntt_inv_reg(SegList<InvSeg<W, Wout>> segs, int logR, int logP, NttTab<W> tab, W 
                                           logP, tab, p, __builtin_amdgcn_readfirstlane(sg.trunc) != 0);
 }
 
+// Transforms of one point (products of constant matrices): the word itself, and
+// the scaled product.  A thread per entry.  At two points these products took
+// twice the evaluations, 64-bit words 123 -> 169 us (60 x 60 x 60, plain kernel).
+template <typename Win, typename W>
+__global__ void __launch_bounds__(kThreads) ntt_fwd_point(SegList<FwdSeg<Win, W>> segs)
+{
+    const FwdSeg<Win, W> sg = segs.of(blockIdx.x);
+    const int64_t e = ((int64_t)blockIdx.x - sg.block0) * kThreads + threadIdx.x;
+    if (e < sg.count)
+        as_global(sg.out)[e] = (W)as_global(sg.in)[e * sg.in_stride];
+}
+
+template <typename W, typename Wout>
+__global__ void __launch_bounds__(kThreads)
+ntt_inv_point(SegList<InvSeg<W, Wout>> segs, NttTab<W> tab, W p)
+{
+    const InvSeg<W, Wout> sg = segs.of(blockIdx.x);
+    const int64_t e = ((int64_t)blockIdx.x - sg.block0) * kThreads + threadIdx.x;
+    if (e < sg.count)
+        as_global(sg.out)[e * sg.out_stride] = (Wout)shoup1(as_global(sg.in)[e], tab.ninv, tab.ninvq, p);
+}
+
 // workgroups of `count` entries (of 2^logR transforms of 2^logM points each)
 inline int64_t xform_blocks(int64_t count, int logM, int logR)
 {
     if (logM >= 11)
         return count << logR;
-    const int nb = 256 >> (logM - small_log_e(logM));
+    const int nb = kThreads >> (logM - small_log_e(logM));
     return (count + nb - 1) / nb;
 }
 
@@ -1373,6 +1395,10 @@ hipError_t dispatch_fwd(int logM, int logE, const SegList<FwdSeg<Win, W>> &segs,
 {
     if (blocks > INT32_MAX || (logM < kRegMinLog && logR > 0))
         return hipErrorInvalidValue;
+    if (logM == 0) {
+        hipLaunchKernelGGL((ntt_fwd_point<Win, W>), dim3((unsigned)blocks), dim3(kThreads), 0, s, segs);
+        return hipGetLastError();
+    }
     return with_log_m<W>(logM, [&](auto l) {
         return launch_fwd_l<Win, W, decltype(l)::value>(logE, segs, blocks, logR, logP, tab, p, s, pre, trunc);
     });
@@ -1384,6 +1410,10 @@ hipError_t dispatch_inv(int logM, int logE, const SegList<InvSeg<W, Wout>> &segs
 {
     if (blocks > INT32_MAX || (logM < kRegMinLog && logR > 0))
         return hipErrorInvalidValue;
+    if (logM == 0) {
+        hipLaunchKernelGGL((ntt_inv_point<W, Wout>), dim3((unsigned)blocks), dim3(kThreads), 0, s, segs, tab, p);
+        return hipGetLastError();
+    }
     return with_log_m<W>(logM, [&](auto l) {
         return launch_inv_l<W, Wout, decltype(l)::value>(logE, segs, blocks, logR, logP, tab, p, s);
     });
@@ -1579,7 +1609,7 @@ hipError_t launch_ntt_fwd(const FwdOp<Win, W> *ops, int nops, int logN, int logP
 {
     const int logM = sub_log_m<W>(logN, trunc);
     const int logR = logN - logM;
-    if (logR > NttLimits<W>::max_log_r || logP > logN || logN < 1 || nops < 1 || nops > 2)
+    if (logR > NttLimits<W>::max_log_r || logP > logN || logN < 0 || nops < 1 || nops > 2)
         return hipErrorInvalidValue;
     if (trunc && (logR > 2 || logN < kTruncMinLog || (logR > 0 && logM < kRegMinLog)))
         return hipErrorInvalidValue;
@@ -1632,7 +1662,7 @@ hipError_t launch_ntt_inv(const W *in, Wout *out, int64_t out_stride, int64_t lo
         return hipSuccess;
     const int logM = sub_log_m<W>(logN, trunc);
     const int logR = logN - logM;
-    if (logR > NttLimits<W>::max_log_r || (logR > 0 && tmp == nullptr) || logP > logN || logN < 1 ||
+    if (logR > NttLimits<W>::max_log_r || (logR > 0 && tmp == nullptr) || logP > logN || logN < 0 ||
         (logR > 2 && (!ct || logM < kRegMinLog)) ||
         (trunc && (logR > 2 || logN < kTruncMinLog || hi > 3 * (N >> 2) ||
                    (logR > 0 && logM < kRegMinLog))))
@@ -1731,7 +1761,7 @@ hipError_t launch_ntt_fwd_segs(const FwdSeg<Win, W> *segs, int nseg, int64_t blo
         return hipSuccess;
     const int logM = sub_log_m<W>(logN, trunc);
     const int logR = logN - logM;
-    if (logR > 2 || logP > logN || logN < 1)
+    if (logR > 2 || logP > logN || logN < 0)
         return hipErrorInvalidValue;
     return dispatch_fwd<Win, W>(logM, log_e, SegList<FwdSeg<Win, W>>{segs, nseg, {}}, blocks, logR, logP,
                                 tab_for_sub(tab, logN, logM), p, s, false, trunc);
@@ -1746,7 +1776,7 @@ hipError_t launch_ntt_inv_segs(const InvSeg<W, Wout> *segs, int nseg, int64_t bl
         return hipSuccess;
     const int logM = sub_log_m<W>(logN, trunc);
     const int logR = logN - logM;
-    if (logR > 2 || logP > logN || logN < 1 || mblocks > INT32_MAX)
+    if (logR > 2 || logP > logN || logN < 0 || mblocks > INT32_MAX)
         return hipErrorInvalidValue;
     hipError_t err = dispatch_inv<W, Wout>(logM, log_e, SegList<InvSeg<W, Wout>>{segs, nseg, {}}, blocks,
                                            logR, logP, tab_for_sub(tab, logN, logM), p, s);
