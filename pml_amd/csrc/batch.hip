@@ -29,6 +29,7 @@
 #include "ctx.hpp"
 #include "dispatch.hpp"
 #include "host_arith.hpp"
+#include "rules.hpp"
 
 namespace pmlg {
 
@@ -137,14 +138,14 @@ unsigned grid_for(int64_t items, int64_t cap = 4096)
 // configurations
 // ---------------------------------------------------------------------------
 const ProdConfig kConfigs[kNumConfigs] = {
-    // school, kind,     fwd_e, inv_e, single_pt
+    // school, kind,     fwd_e, inv_e, half_pt
     {1, PW_PLAIN, 5, 4, 0},  // 0: direct convolution
     {0, PW_PLAIN, 5, 4, 0},  // 1: transforms + plain pointwise
     {0, PW_MFMA, 5, 4, 0},   // 2: transforms + int8-limb MFMA pointwise
     {0, PW_PLAIN, 4, 4, 0},  // 3: plain, radix-16 forward passes
     {0, PW_MFMA, 4, 4, 0},   // 4: MFMA, radix-16 forward passes
     {0, PW_MFMA, 5, 5, 0},   // 5: MFMA, radix-32 inverse passes
-    {0, PW_MFMA, 5, 4, 1},   // 6: MFMA, one point per task
+    {0, PW_MFMA, 5, 4, 1},   // 6: MFMA, half the points per task
     {0, PW_PLAIN, 5, 5, 0},  // 7: plain, radix-32 inverse passes
 };
 
@@ -514,7 +515,7 @@ void add_segments(const pmlg_mul_desc &d, const ProdInfo &pi, unsigned char *are
     const bool redc = sizeof(W) == 8;
     inv[{ctx, logN, cf.inv_e, (redc ? 1 : 0) | (trunc << 1)}].push_back(
         InvSeg<W, uint64_t>{Ch, d.C, tmp, lenC, 0, lenC, d.m * d.n, 0, 0, trunc, 0});
-    const int pt = cf.kind == PW_MFMA ? pw_points(sizeof(W), logP, cf.single_pt != 0)
+    const int pt = cf.kind == PW_MFMA ? pw_points(sizeof(W), logP, cf.half_pt != 0)
                                             : pw_plain_rows((int)d.m, N);
     PwSeg<W> ps{};
     ps.Ah = Ah;

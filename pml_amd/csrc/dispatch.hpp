@@ -10,7 +10,7 @@ struct ProdConfig {
     int school;          // 1: direct convolution, 0: transforms + pointwise products
     PointwiseKind kind;  // pointwise kernel
     int fwd_e, inv_e;    // log2 elements per thread of the register transforms
-    int single_pt;       // MFMA tasks of one point instead of 16 bytes of a run
+    int half_pt;         // MFMA tasks of 8 bytes of a run instead of 16
 };
 
 constexpr int kNumConfigs = 8;

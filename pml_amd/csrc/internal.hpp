@@ -239,8 +239,6 @@ struct PwSeg {
     int64_t N, block0;
     int32_t redc_small, logPc;  // logPc: runs of C_hat
 };
-// points per task of the MFMA kernel: 16 bytes of a run, or one
-int pw_points(int elem_bytes, int logP, bool single);
 // rows of the plain kernel's tiles, 2 or 4, and blocks of either kernel with pt
 // points per task or rows
 int pw_plain_rows(int m, int64_t N);

@@ -32,9 +32,9 @@ constexpr int64_t kMfmaPlanes = 128 * 1024;
 typedef int v4i __attribute__((ext_vector_type(4)));
 
 // waves per SIMD of the MFMA kernel: two with its usual points per task
-// (about 200 registers), four with one point
+// (about 200 registers), four with fewer
 template <int PT, typename W>
-constexpr int kMfmaWaves = PT == 1 ? 4 : 2;
+constexpr int kMfmaWaves = PT * sizeof(W) < 16 ? 4 : 2;
 
 // ---------------------------------------------------------------------------
 // plain kernel
@@ -185,7 +185,7 @@ __device__ __forceinline__ uint32_t conv_word(uint32_t r)
     return w <= 3 ? r >> (8 * (3 - w)) : r << (8 * (w - 3));
 }
 
-// PT consecutive words at src (16-byte aligned when PT words fill 16 bytes)
+// PT consecutive words at src (aligned to the PT words, 16 bytes at most)
 template <typename W, int PT>
 __device__ __forceinline__ void load_points(const W *__restrict__ src, W (&v)[PT])
 {
@@ -200,6 +200,10 @@ __device__ __forceinline__ void load_points(const W *__restrict__ src, W (&v)[PT
             v[2] = x.z;
             v[3] = x.w;
         }
+    } else if constexpr (PT == 2) {
+        const uint2 x = *reinterpret_cast<const uint2 *>(src);
+        v[0] = x.x;
+        v[1] = x.y;
     } else {
 #pragma unroll
         for (int t = 0; t < PT; ++t)
@@ -224,6 +228,8 @@ __device__ __forceinline__ void store_points(W *dst, const W (&v)[PT])
             u.w = v[3];
         }
         *reinterpret_cast<uint4 *>(dst) = u;
+    } else if constexpr (PT == 2) {
+        *reinterpret_cast<uint2 *>(dst) = make_uint2(v[0], v[1]);
     } else {
 #pragma unroll
         for (int t = 0; t < PT; ++t)
@@ -695,12 +701,6 @@ int pw_plain_rows(int m, int64_t N)
     return plain_rows(m, N, INT64_MAX);
 }
 
-int pw_points(int elem_bytes, int logP, bool single)
-{
-    const int pt = 16 / elem_bytes;
-    return single || (1 << logP) < pt ? 1 : pt;
-}
-
 int64_t pw_seg_blocks(PointwiseKind kind, int pt, int m, int n, int64_t N)
 {
     if (kind == PW_MFMA)
@@ -735,6 +735,9 @@ hipError_t launch_pointwise_segs(PointwiseKind kind, int pt, const PwSeg<W> *seg
     grid = (int)xcd_grid(grid);
     if (pt == kPoints<W>)
         hipLaunchKernelGGL((pw_mfma_segs<W, kPoints<W>>), dim3((unsigned)grid), dim3(kThreads), 0, s,
+                           segs, nseg, blocks, mc);
+    else if (pt == kPoints<W> / 2)
+        hipLaunchKernelGGL((pw_mfma_segs<W, kPoints<W> / 2>), dim3((unsigned)grid), dim3(kThreads), 0, s,
                            segs, nseg, blocks, mc);
     else if (pt == 1)
         hipLaunchKernelGGL((pw_mfma_segs<W, 1>), dim3((unsigned)grid), dim3(kThreads), 0, s, segs,

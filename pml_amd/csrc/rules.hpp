@@ -28,6 +28,18 @@ inline int plain_rows(int m, int64_t N, int64_t waves)
     return N >= 64 && waves >= 2048 && m > 6 ? 4 : 2;
 }
 
+// Points per task of the MFMA kernel, for words of elem_bytes in runs of 2^logP
+// points: 16 bytes of a run, or 8 (half), or one point where the run is shorter.
+// Half of it takes twice the waves per SIMD and reads as many bytes in half the
+// requests that single points take; with one point for 32-bit words configuration 6
+// took 2960 us for 16 products 32 x 32 x 32 of length 4096 (30-bit prime), with two
+// 2160.
+inline int pw_points(int elem_bytes, int logP, bool half)
+{
+    const int pt = (half ? 8 : 16) / elem_bytes;
+    return (1 << logP) < pt ? 1 : pt;
+}
+
 // Whether the MFMA kernel is the faster one where both are exact: its time and the
 // plain kernel's in nanoseconds, a start and a chain (the loads of a step of 16, or
 // of one, of the inner dimension, one after another) plus what each task (a tile of
