@@ -175,10 +175,11 @@ bool config_valid(pmlg_ctx ctx, int64_t m, int64_t k, int64_t n, int64_t lenA, i
 // dimension (<= 8, 16, 32, 64) and the product length (< 2^11, 2^13, 2^15,
 // longer) select a cell, whose configuration was fitted on the recorded
 // timings (bands.inc, generated by `python -m pml_amd.learn bands`; the same
-// cell function is pml_amd.learn.band_index).  A cell without a fit, or whose
-// configuration cannot run the shape, falls back to the fixed rule: direct
-// convolution when both operands are short, else transforms with the MFMA
-// pointwise kernel whenever the shape and modulus allow it, else plain.
+// cell function is pml_amd.learn.band_index); they were recorded with earlier
+// kernels.  A cell without a fit, or whose configuration cannot run the shape,
+// falls back to the fixed rule: direct convolution when both operands are short,
+// else transforms with the MFMA pointwise kernel whenever the shape and modulus
+// allow it, else plain.
 #include "bands.inc"
 
 int band_index(bool small, int64_t m, int64_t k, int64_t n, int64_t lenA, int64_t lenB)

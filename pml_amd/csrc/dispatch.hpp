@@ -37,7 +37,7 @@ int learned_config(pmlg_ctx ctx, int64_t m, int64_t k, int64_t n, int64_t lenA, 
 // of its best are timed once per shape class (measured refinement).  The
 // network's error is about 24% RMS in log time and not uniform across
 // configurations (smooth features cannot show the MFMA tiles' padding steps
-// at multiples of 32), so the margin is wide: on 2,000 held-out shapes, with
+// at multiples of 16), so the margin is wide: on 2,000 held-out shapes, with
 // the recorded times standing in for the live ones, 15% brings the total
 // within 0.05% of the per-shape best with 4 candidates a shape (5%: 0.3%
 // above it with 2.6).

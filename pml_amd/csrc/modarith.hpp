@@ -1,7 +1,8 @@
 // Modular arithmetic for word-size primes, shared by host and device code.
 //
 // Two word types are used on the device:
-//   uint64_t for primes p < 2^62 (values kept lazily in [0, 2p) inside the NTT),
+//   uint64_t for primes p < 2^62 (inside the NTT values stay below 16p for
+//   p < 2^60 and in [0, 2p) above),
 //   uint32_t for primes p < 2^30 (values kept lazily in [0, 2p)).
 // Multiplications by a fixed operand (twiddles, recombination constants) use
 // Shoup's precomputed quotient: for w < p and w' = floor(w * 2^B / p),
@@ -113,7 +114,7 @@ struct ModConst {
     int redc_small;     // set per call: REDC output already in the inverse's range (host_redc_small)
     uint32_t p32, p32x2, p32q_unused;
     int bits;           // bit length of p
-    int limbs;          // 8 for p < 2^62, 4 for p < 2^30
+    int limbs;          // 8 for p < 2^61, 4 for p < 2^30, 0: no MFMA kernel
     // any p < 2^64: division of 128-bit values by the normalised modulus
     int norm;           // leading zero bits of p
     uint64_t dnorm;     // p << norm

@@ -299,8 +299,8 @@ struct MfmaTile {
                 fb[h][u] = (int)conv_word<w>(rb[h][u]);
         // half-word products of weight 2^(8 w), 2^(8 w + 32), 2^(8 w + 64); the
         // first product into an accumulator of the first chunk starts from
-        // zero: low x low for weights 0..6, the cross products for 7..10,
-        // high x high for 11..14
+        // zero: low x low for weights 0..3 (all seven with one half-word), the
+        // cross products for 4..7, high x high for 8..14
         constexpr bool Z = FIRST && (w < 4 || H == 1);
         t[w] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[0], fb[0], Z ? zero : t[w], 0, 0, 0);
         if constexpr (H == 2) {
