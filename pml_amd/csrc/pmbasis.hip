@@ -498,7 +498,7 @@ __device__ __forceinline__ uint64_t lane_value(uint64_t v, int l)
 // (barrier) each, the window's update 0 to 6.7 with the orders still to come
 // (3.5 on average), the sort 0.8, the rest 2.2.  Step plus update kernel per
 // order, with one order per launch and panels composed pivot by pivot / as it
-// is: 17.7 + 9.5 / 15.9 + 4.2 us (64 x 32, 32-bit), 13.5 + 6.8 / 11.0 + 3.6 us
+// is: 17.7 + 9.5 / 16.1 + 3.5 us (64 x 32, 32-bit), 13.5 + 6.8 / 11.0 + 3.6 us
 // (32 x 17, 64-bit).
 template <typename Arith, int H>
 __global__ void __launch_bounds__(kStepThreads) mbasis_step_kernel(LeafArgs a, int ord0, int w)
@@ -1461,7 +1461,7 @@ __global__ void __launch_bounds__(kStepThreads) mbasis_step_kernel(LeafArgs a, i
 // The window's kernel vectors are brought to LDS at the start, beside the tile
 // (rows padded with zeros to a multiple of kGroup), so that the orders wait for
 // no global load.
-// Latency bounds it: 16.6 us per window of 4 orders (64 x 32, 32-bit words; 4 x
+// Latency bounds it: 14.0 us per window of 4 orders (64 x 32, 32-bit words; 4 x
 // 7.4 to 9.5 with a launch per order), of which 2.3 are the loads, 1.5 each
 // order and the rest the launch's start and end.
 constexpr int kUpdateThreads = 512;
