@@ -25,8 +25,9 @@
 // each order, and writes every order's description; kernel 2 (a grid) then
 // applies the window's row operations, one after the other, to tiles of
 // appbas and of the rest of R held in LDS, reading one buffer and writing the
-// other (a thread per coefficient where windows do not pay: mbasis_window).  All control (nullity cases, basis length)
-// stays on the device: a leaf is a fixed sequence of launches.  The steps
+// other (a thread per coefficient where windows do not pay: mbasis_window).
+// All control (nullity cases, basis length) stays on the device: a leaf is a
+// fixed sequence of launches.  The steps
 // skip the division by the pivots in 3: with D the product of the pivots,
 // they apply D X and multiply the updated rows by D, so each basis row is the
 // reference's row times a known nonzero scale, and the leaf divides the
